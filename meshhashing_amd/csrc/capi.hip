@@ -2049,18 +2049,20 @@ int mh_batch_synchronize(mh_batch* b) {
 // ------------------------------------------------------------ raycast adjoint
 namespace {
 
-// FP64 partial-sum rows (up to 30 slots each) for `rows` workgroups, and the
-// 30-slot result.
+// FP64 partial-sum rows for `rows` workgroups, and the result row, each wide
+// enough for either caller's sums (the adjoint's 31, the localiser's 29).
+constexpr int kPartialSlots = kGradSlots;
+static_assert(kP2SSlots <= kPartialSlots, "partial-sum rows");
 hipError_t ensure_partials(mh_volume* v, uint32_t rows) {
   if (rows > v->rgrad_cap) {
     if (v->rgrad_partials) (void)hipFree(v->rgrad_partials);
     v->rgrad_partials = nullptr;
     v->rgrad_cap = 0;
-    const hipError_t e = dalloc(&v->rgrad_partials, (size_t)rows * 30);
+    const hipError_t e = dalloc(&v->rgrad_partials, (size_t)rows * kPartialSlots);
     if (e != hipSuccess) return e;
     v->rgrad_cap = rows;
   }
-  if (!v->rgrad_out) return dalloc(&v->rgrad_out, 30);
+  if (!v->rgrad_out) return dalloc(&v->rgrad_out, kPartialSlots);
   return hipSuccess;
 }
 
