@@ -244,6 +244,7 @@ struct Counters {
   uint32_t mc_next;        // marching cubes: worklist items handed out on demand (after the static ones)
   uint32_t vfree_count;    // entries of vfree
   uint32_t vfree_done;     // workgroups done pushing vfree on the vertex heap
+  uint32_t reduce_done;    // workgroups done in slot_reduce_kernel (0 between calls)
   WorkStripe work[kWorkStripes];
 };
 

@@ -704,15 +704,50 @@ __global__ __launch_bounds__(64) void raycast_backward_kernel(View V, RayConst R
   }
 }
 
-// Sums the per-workgroup partials in workgroup order (deterministic).
-// Sums n rows of `slots` FP64 partials column by column, in row order.
-__global__ void slot_reduce_kernel(const double* __restrict__ partials, uint32_t n, uint32_t slots,
-                                   double* __restrict__ out) {
-  const uint32_t k = threadIdx.x;
-  if (k >= slots) return;
+// Sums n rows of `slots` (<= 32) FP64 partials column by column into out, in
+// an order fixed by n alone (deterministic).  A workgroup sums kReduceRows
+// rows, eight of them at a time (32 lanes a row), and leaves the sum in the
+// first of its rows; the workgroup that finishes last adds those up the same
+// way.  A lane's chain is then kReduceRows / 8 loads rather than n: a lane
+// per column walking every row took 1135 us for a 640 x 480 image's 4800 rows
+// (71 us for 300 rows) against 9 us (5 us) here.
+constexpr uint32_t kReduceRows = 64;
+__device__ __forceinline__ double reduce_rows(const double* rows, uint32_t n, size_t stride,
+                                              uint32_t slots, double (*red)[32]) {
+  const uint32_t k = threadIdx.x & 31u, g = threadIdx.x >> 5;
   double s = 0.0;
-  for (uint32_t i = 0; i < n; ++i) s += partials[(size_t)i * slots + k];
-  out[k] = s;
+  if (k < slots)
+#pragma unroll 8
+    for (uint32_t i = g; i < n; i += 8) s += rows[i * stride + k];
+  red[g][k] = s;
+  __syncthreads();
+  double all = 0.0;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) all += red[j][k];
+  __syncthreads();
+  return all;
+}
+__global__ __launch_bounds__(256) void slot_reduce_kernel(double* partials, uint32_t n, uint32_t slots,
+                                                          uint32_t* done, double* __restrict__ out) {
+  __shared__ double red[8][32];
+  __shared__ bool last;
+  const uint32_t r0 = blockIdx.x * kReduceRows;
+  double* const mine = partials + (size_t)r0 * slots;
+  const double s = reduce_rows(mine, min(kReduceRows, n - r0), slots, slots, red);
+  if (threadIdx.x < slots) (gridDim.x == 1 ? out : mine)[threadIdx.x] = s;
+  if (gridDim.x == 1) return;
+  __threadfence();  // the row before the count that announces it
+  __syncthreads();
+  if (threadIdx.x == 0) last = atomicAdd(done, 1u) == gridDim.x - 1;
+  __syncthreads();
+  if (!last) return;
+  __threadfence();  // the other workgroups' rows after their counts
+  const double a = reduce_rows(partials, gridDim.x, (size_t)kReduceRows * slots, slots, red);
+  if (threadIdx.x < slots) out[threadIdx.x] = a;
+  if (threadIdx.x == 0) *done = 0u;  // for the next call
+}
+void launch_slot_reduce(double* partials, uint32_t n, uint32_t slots, uint32_t* done, double* out, hipStream_t s) {
+  slot_reduce_kernel<<<(n + kReduceRows - 1) / kReduceRows, 256, 0, s>>>(partials, n, slots, done, out);
 }
 
 // ------------------------------------------------------------ localisation
@@ -801,7 +836,7 @@ void launch_point_to_psdf(const View& V, const M4& wTc, int corrected, double* p
                           hipStream_t s) {
   const dim3 grid((V.cam.width / 2 + 7) / 8, (V.cam.height / 2 + 7) / 8);
   point_to_psdf_kernel<<<grid, 64, 0, s>>>(V, wTc, 1.0f / V.geo.voxel_size, corrected, partials);
-  slot_reduce_kernel<<<1, 64, 0, s>>>(partials, grid.x * grid.y, kP2SSlots, out);
+  launch_slot_reduce(partials, grid.x * grid.y, kP2SSlots, &V.ctr->reduce_done, out, s);
 }
 
 __device__ __forceinline__ const RayConst& ray_of(const One&, uint32_t, const RayConst& r) { return r; }
@@ -1011,7 +1046,7 @@ void launch_raycast_backward(const View& V, const RayConst& p, const float* obs,
   if (p.range) launch_ray_range(One{V}, nullptr, p, p.tiles, 1, s);
   raycast_backward_kernel<<<grid, 64, 0, s>>>(V, p, obs, grad_sdf, partials, max_residual,
                                               max_slope);
-  slot_reduce_kernel<<<1, 64, 0, s>>>(partials, grid.x * grid.y, kGradSlots, out);
+  launch_slot_reduce(partials, grid.x * grid.y, kGradSlots, &V.ctr->reduce_done, out, s);
 }
 
 void launch_batch_raycast(const BatchDev& B, float* depth, float* vertex, float* normal,
