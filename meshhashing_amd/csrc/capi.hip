@@ -954,7 +954,7 @@ int mh_primal_dual_iterate(mh_volume* v, float lambda, float sigma, float tau, d
   if (v->pd_work_gen != v->work_gen)
     return fail(MH_ERR_STATE, "worklist changed since mh_primal_dual_init");
   launch_pd_iterate(v->V, v->pd_nbr, lambda, sigma, tau, v->pd_partials, v->pd_npartials,
-                    v->pd_energy, v->stream, v->grid_wg256());
+                    energy_host ? v->pd_energy : nullptr, v->stream, v->grid_wg256());
   HIP_TRY(hipGetLastError());
   if (energy_host) {
     HIP_TRY(hipMemcpyAsync(energy_host, v->pd_energy, 3 * sizeof(double), hipMemcpyDeviceToHost,

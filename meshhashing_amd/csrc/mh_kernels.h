@@ -258,6 +258,7 @@ void launch_point_to_psdf(const View& V, const M4& wTc, int corrected, double* p
 // primal_dual.hip
 void launch_pd_neighbors(const View& V, int32_t* nbr, hipStream_t s, int grid);
 void launch_pd_init(const View& V, const int32_t* nbr, hipStream_t s, int grid);
+// energy: where the three energies go, or null if they are not wanted
 void launch_pd_iterate(const View& V, const int32_t* nbr, float lambda, float sigma, float tau,
                        double* partials, uint32_t npartials, double* energy, hipStream_t s,
                        int grid);

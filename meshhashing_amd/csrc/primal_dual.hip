@@ -102,6 +102,10 @@ __device__ __forceinline__ double block_sum(double v, double* red) {
 
 // PrimalDualIteratePass1Kernel (primal_dual.cu:45-109): energies, dual
 // ascent p += sigma grad(sdf_bar), Huber shrink, projection onto |p| <= 1.
+// The energies (ENERGY) are taken only when the caller asks for them: they
+// need the field, its start and the field's three neighbours, which the dual
+// step does not read.
+template <bool ENERGY>
 __global__ __launch_bounds__(256) void pd_pass1_kernel(View V, const int32_t* nbr, float sigma,
                                                        double* partials) {
   __shared__ double red[8];
@@ -116,10 +120,13 @@ __global__ __launch_bounds__(256) void pd_pass1_kernel(View V, const int32_t* nb
       const float w = V.weight[idx];
       if (below_eps(w)) continue;
       const i3 o = devectorize(i);
-      const float sdf = V.sdf[idx];
-      float dd = fabsf(sdf - V.pd_sdf0[idx]);
-      dd *= dd;
-      if (above_eps(w)) e_data += (double)dd;
+      float sdf = 0.0f;
+      if (ENERGY) {
+        sdf = V.sdf[idx];
+        float dd = fabsf(sdf - V.pd_sdf0[idx]);
+        dd *= dd;
+        if (above_eps(w)) e_data += (double)dd;
+      }
       // GetSDFGradient (primal_dual_query.h:88-133) and GetPrimalGradient
       // (:189-234): forward differences; any missing, unobserved or
       // unmasked neighbour zeroes the whole gradient.
@@ -131,13 +138,15 @@ __global__ __launch_bounds__(256) void pd_pass1_kernel(View V, const int32_t* nb
           ok = false;
           break;
         }
-        gs[k] = V.sdf[j];
+        if (ENERGY) gs[k] = V.sdf[j];
         gb[k] = V.pd_sdf_bar[j];
       }
       const float sb = V.pd_sdf_bar[idx];
-      const f3 grad_s = ok ? mk3(gs[0] - sdf, gs[1] - sdf, gs[2] - sdf) : mk3(0.0f, 0.0f, 0.0f);
       const f3 grad_b = ok ? mk3(gb[0] - sb, gb[1] - sb, gb[2] - sb) : mk3(0.0f, 0.0f, 0.0f);
-      e_tv += (double)huber(length(grad_s), alpha);
+      if (ENERGY) {
+        const f3 grad_s = ok ? mk3(gs[0] - sdf, gs[1] - sdf, gs[2] - sdf) : mk3(0.0f, 0.0f, 0.0f);
+        e_tv += (double)huber(length(grad_s), alpha);
+      }
       f3 p = mk3(V.pd_p[3 * idx], V.pd_p[3 * idx + 1], V.pd_p[3 * idx + 2]);
       p = p + sigma * grad_b;
       p = p / (1.0f + sigma * alpha);
@@ -147,11 +156,13 @@ __global__ __launch_bounds__(256) void pd_pass1_kernel(View V, const int32_t* nb
       V.pd_p[3 * idx + 2] = p.z;
     }
   }
-  const double sd = block_sum(e_data, red);
-  const double st = block_sum(e_tv, red);
-  if (threadIdx.x == 0) {
-    partials[2 * blockIdx.x + 0] = sd;
-    partials[2 * blockIdx.x + 1] = st;
+  if (ENERGY) {
+    const double sd = block_sum(e_data, red);
+    const double st = block_sum(e_tv, red);
+    if (threadIdx.x == 0) {
+      partials[2 * blockIdx.x + 0] = sd;
+      partials[2 * blockIdx.x + 1] = st;
+    }
   }
 }
 
@@ -195,14 +206,20 @@ __global__ __launch_bounds__(256) void pd_pass2_kernel(View V, const int32_t* nb
   }
 }
 
-// Fixed-order sum of the per-workgroup partials.
-__global__ void pd_energy_kernel(const double* partials, uint32_t n, float lambda, double* energy) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+// Sum of the per-workgroup partials, in an order fixed by n: a lane adds
+// every 256th, then the lanes are added up in order.  (One lane adding all
+// 2048 pairs was a chain of 183 us.)
+__global__ __launch_bounds__(256) void pd_energy_kernel(const double* __restrict__ partials, uint32_t n, float lambda,
+                                                        double* __restrict__ energy) {
+  __shared__ double red[8];
   double d = 0.0, t = 0.0;
-  for (uint32_t i = 0; i < n; ++i) {
+  for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) {
     d += partials[2 * i];
     t += partials[2 * i + 1];
   }
+  d = block_sum(d, red);
+  t = block_sum(t, red);
+  if (threadIdx.x != 0) return;
   energy[0] = d;
   energy[1] = t;
   energy[2] = d * (double)lambda / 2.0 + t;
@@ -218,8 +235,12 @@ void launch_pd_iterate(const View& V, const int32_t* nbr, float lambda, float si
                        double* partials, uint32_t npartials, double* energy, hipStream_t s,
                        int grid) {
   const int g = grid < (int)npartials ? grid : (int)npartials;
-  pd_pass1_kernel<<<g, 256, 0, s>>>(V, nbr, sigma, partials);
-  pd_energy_kernel<<<1, 64, 0, s>>>(partials, (uint32_t)g, lambda, energy);
+  if (energy) {
+    pd_pass1_kernel<true><<<g, 256, 0, s>>>(V, nbr, sigma, partials);
+    pd_energy_kernel<<<1, 256, 0, s>>>(partials, (uint32_t)g, lambda, energy);
+  } else {
+    pd_pass1_kernel<false><<<g, 256, 0, s>>>(V, nbr, sigma, nullptr);
+  }
   pd_pass2_kernel<<<grid, 256, 0, s>>>(V, nbr, lambda, tau);
 }
 
