@@ -450,6 +450,7 @@ int mh_volume_create(const mh_hash_params* hash, const mh_volume_params* vol,
   A(&V.block_heap, cap);
   A(&V.occ, (size_t)1 << (kOccBits - 5));
   A(&V.occ2, (size_t)1 << (kOcc2Bits - 5));
+  A(&V.oct, cap * 8);
   A(&V.ctr, 1);
   A(&V.ovf, kOverflowQueue);
   A(&V.sdf, nvox);
@@ -1435,6 +1436,7 @@ int check_tiling(int tiling, int grid_per_cu) {
 struct mh_batch {
   std::vector<mh_volume*> vols;
   uint32_t n = 0, W = 0, H = 0;
+  uint32_t max_capacity = 0;  // largest scene pool
   hipStream_t stream = nullptr;
   bool own_stream = false;
   // the raycast branch of a frame (it reads only the fused TSDF and the
@@ -1469,7 +1471,7 @@ struct mh_batch {
   hipGraphExec_t exec = nullptr;
   uint32_t graph_flags = 0;
 
-  BatchDev dev() const { return BatchDev{d_frames, d_work, d_work_count, d_dyn, n, W, H, 0}; }
+  BatchDev dev() const { return BatchDev{d_frames, d_work, d_work_count, d_dyn, n, W, H, 0, max_capacity}; }
   void drop_graph() {
     if (exec) (void)hipGraphExecDestroy(exec);
     if (graph) (void)hipGraphDestroy(graph);
@@ -1597,7 +1599,7 @@ int mh_tune_raycast(mh_volume* v, const mh_raycaster_params* p, const float cTw[
   HIP_TRY(sc.get(&d, npix));
   HIP_TRY(sc.get(&n, npix * 3));
   HIP_TRY(sc.get(&sctr, 1));
-  if (R.range) launch_ray_range_one(v->V, R, v->stream);
+  launch_ray_range_one(v->V, R, v->stream);
   HIP_TRY(hipMemcpyAsync(sctr, v->V.ctr, sizeof(Counters), hipMemcpyDeviceToDevice, v->stream));
   auto run = [&](int k) { launch_raycast_march(v->V, R, d, nullptr, n, v->stream, k); };
   auto restore = [&]() -> int {
@@ -1790,6 +1792,7 @@ int mh_batch_create(uint32_t n_scenes, const mh_hash_params* hash, const mh_volu
     v->stream = b->stream;
     b->vols.push_back(v);
     work_cap += hash[s].value_capacity;
+    b->max_capacity = std::max(b->max_capacity, hash[s].value_capacity);
   }
   const size_t npix = (size_t)b->W * b->H * n_scenes;
   if (dalloc(&b->d_frames, n_scenes) != hipSuccess || dalloc(&b->d_work, work_cap) != hipSuccess ||
@@ -2359,7 +2362,8 @@ int mh_dump_voxel_field(mh_volume* v, const float* field_dev, uint32_t capacity,
 // ------------------------------------------------------------ localisation
 namespace {
 
-// PointToSurface (localizing/point_to_psdf.cu:84-147) on the current frame.
+// PointToSurface (localizing/point_to_psdf.cu:84-147) on the current frame,
+// the block rows being filled (launch_ray_rows).
 int point_to_psdf(mh_volume* v, const float wTc[16], int jacobian, mh_point_to_psdf_result* out) {
   flush_frame(v);
   HIP_TRY(ensure_partials(v, point_to_psdf_partials(v->V)));
@@ -2393,6 +2397,7 @@ int mh_point_to_psdf(mh_volume* v, const float wTc[16], int jacobian, mh_point_t
   if (jacobian != MH_P2S_REFERENCE && jacobian != MH_P2S_CORRECTED)
     return fail(MH_ERR_ARG, "jacobian must be MH_P2S_REFERENCE or MH_P2S_CORRECTED");
   if (!v->have_frame) return fail(MH_ERR_STATE, "no frame uploaded");
+  launch_ray_rows(v->V, v->stream);
   return point_to_psdf(v, wTc, jacobian, out);
 }
 
@@ -2402,6 +2407,7 @@ int mh_localize(mh_volume* v, uint32_t iterations, float lambda, int jacobian, f
   if (jacobian != MH_P2S_REFERENCE && jacobian != MH_P2S_CORRECTED)
     return fail(MH_ERR_ARG, "jacobian must be MH_P2S_REFERENCE or MH_P2S_CORRECTED");
   if (!v->have_frame) return fail(MH_ERR_STATE, "no frame uploaded");
+  launch_ray_rows(v->V, v->stream);  // no step changes the block set
   uint32_t it = 0;
   for (; it < iterations; ++it) {
     mh_point_to_psdf_result r;

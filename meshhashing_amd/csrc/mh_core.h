@@ -15,6 +15,7 @@
 #include <stdint.h>
 
 #include "../../include/meshhashing.h"
+#include "mh_div.h"
 
 #define MH_HD __host__ __device__ __forceinline__
 
@@ -108,34 +109,33 @@ __device__ __forceinline__ int vox1(float w, float vs) {
   return f2i(p + (float)sgn(p) * 0.5f);
 }
 
-// vox1(pc, vs) from a multiply by 1/vs instead of the IEEE division;
-// accepted only when the quotient is more than 1e-3 voxel away from every
-// rounding tie and from 0 (and |q| < 2048, where the multiply is within 2 ulp
-// of the quotient), so it equals the exact result.
-__device__ __forceinline__ bool fast_corner(float pc, float inv_vs, int* c) {
-  const float q = pc * inv_vs;
-  const float aq = fabsf(q);
-  if (!(aq < 2048.0f) || aq < 1e-3f) return false;
-  const float f = aq - floorf(aq);
-  if (fabsf(f - 0.5f) < 1e-3f) return false;
-  *c = f2i(q + (float)sgn(q) * 0.5f);
-  return true;
+// vox1 with the division as a quotient by a constant (inv_vs = 1 / vs).
+// Quotients outside its range (past any voxel, infinite, not a number) take
+// the division itself.
+__device__ __forceinline__ int vox1_quot(float w, float vs, float inv_vs) {
+  const float p = fabsf(w * inv_vs) < 1e9f ? quotient(w, vs, inv_vs) : w / vs;
+  return f2i(p + (float)sgn(p) * 0.5f);
 }
 
 // The two corner voxels vox1(pc, vs) and vox1(pc + vs, vs) of a trilinear
-// sample along one axis (spatial_query.h:23-66 rounds both).  Clear of a
-// tie, the upper one is the lower + 1: pc + vs is within 1.3e-4 voxel of
-// exact, so its quotient stays clear of the next tie.
+// sample along one axis (spatial_query.h:23-66 rounds both).  Below 2048
+// voxels the product pc * inv_vs is within 2.5e-4 of the exact quotient and
+// the rounded quotient within 1.3e-4, so a product more than 1e-3 from every
+// rounding tie rounds to the same voxel; the upper corner is then the lower
+// + 1, pc + vs being within 1.3e-4 voxel of exact.
 __device__ __forceinline__ void corner_pair(float pc, float vs, float inv_vs, int* c0, int* c1) {
-  if (fast_corner(pc, inv_vs, c0)) {
-    *c1 = *c0 + 1;
-  } else {
-    *c0 = vox1(pc + 0.0f, vs);
-    *c1 = vox1(pc + vs, vs);
+  const float q = pc * inv_vs, r = rintf(q);
+  *c0 = (int)r;
+  *c1 = *c0 + 1;
+  if (!(fabsf(q) < 2048.0f && fabsf(q - r) < 0.499f)) {
+    *c0 = vox1_quot(pc, vs, inv_vs);
+    *c1 = vox1_quot(pc + vs, vs, inv_vs);
   }
 }
 
-MH_HD int voxel_to_block1(int v) { return (v - (v < 0) * (kBlockSide - 1)) / kBlockSide; }
+// floor(v / 8), what the reference's (v - (v < 0) * 7) / 8 gives
+MH_HD int voxel_to_block1(int v) { return v >> 3; }
+static_assert(kBlockSide == 8, "voxel_to_block1");
 MH_HD i3 voxel_to_block(i3 v) {
   return i3{voxel_to_block1(v.x), voxel_to_block1(v.y), voxel_to_block1(v.z)};
 }
@@ -294,6 +294,7 @@ struct View {
   uint32_t capacity;
   uint32_t* occ;         // occupancy filter, 2^kOccBits bits
   uint32_t* occ2;        // super-block (4^3 blocks) occupancy filter, 2^kOcc2Bits bits
+  int32_t* oct;          // per block b: pool indices of b + {0, 1}^3; valid within a raycast (ray_prepare_kernel)
   Counters* ctr;
   uint64_t* ovf;         // overflow queue
   // voxels, pool-index-major, 512 per block

@@ -125,6 +125,7 @@ struct BatchDev {
   uint32_t nscenes;
   uint32_t width, height;  // common image size
   int psdf;             // scenes carry PSDF fields (all or none)
+  uint32_t max_capacity;   // largest block pool
   Many src() const { return Many{frames, work, work_count, dyn}; }
 };
 
@@ -252,6 +253,9 @@ void launch_raycast_backward(const View& V, const RayConst& p, const float* obs,
 // err, count) over the current frame's depth
 constexpr int kP2SSlots = 29;
 uint32_t point_to_psdf_partials(const View& V);
+// Fills V.oct, which the point-to-PSDF pass reads (valid until the block set
+// changes).
+void launch_ray_rows(const View& V, hipStream_t s);
 void launch_point_to_psdf(const View& V, const M4& wTc, int corrected, double* partials, double* out,
                           hipStream_t s);
 

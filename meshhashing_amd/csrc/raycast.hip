@@ -11,8 +11,7 @@
 // march keeps the eight blocks around its current lowest-corner block
 // (Octant) and shares block lookups, misses included, through a per-wave LDS
 // table, so runs of samples in one block, or in one unallocated block, cost
-// no hash probe; the adjoint and localisation kernels keep a lane's last two
-// lookups in registers (BlockCache) instead.
+// no hash probe; the neighbours come from a table filled before the march.
 // The depth output is metric z (t * dir_c.z); the reference colour-maps it
 // (ray_caster.cu:96-98) and keeps metric depth only in the vertex image.
 #include "mh_kernels.h"
@@ -40,18 +39,32 @@ __device__ __forceinline__ void wave_table_init(WaveTable* t) {
   __syncthreads();
 }
 
+// A block's pool index; kFreePtr if it is absent, kAbsentSuper if no block of
+// its super-block was ever allocated either.  Both filters' words and the
+// bucket's first slot are loaded together (one round trip in the usual cases).
+constexpr int32_t kAbsentSuper = -1;
+__device__ __forceinline__ int32_t ray_probe(const View& V, i3 b) {
+  if (!coord_ok(b)) return kFreePtr;
+  const uint64_t key = pack_key(b);
+  const uint32_t bit = occ_bit(key), sbit = occ2_bit(super_key(b));
+  const uint32_t first = hash_bucket(b, V.bucket_count) * V.bucket_size;
+  const uint32_t word = V.occ[bit >> 5], sword = V.occ2[sbit >> 5];
+  const Entry e0 = V.entries[first];
+  if (!((word >> (bit & 31u)) & 1u)) return ((sword >> (sbit & 31u)) & 1u) ? kFreePtr : kAbsentSuper;
+  if (e0.key == key) return e0.ptr;
+  return hash_find_key<true>(V, b, key);
+}
+
 __device__ __forceinline__ int32_t table_find(const View& V, WaveTable* t, i3 b) {
   const int lim = 1 << 15;
-  if (b.x < -lim || b.x >= lim || b.y < -lim || b.y >= lim || b.z < -lim || b.z >= lim)
-    return coord_ok(b) ? hash_find_eager(V, b) : kFreePtr;
+  if (b.x < -lim || b.x >= lim || b.y < -lim || b.y >= lim || b.z < -lim || b.z >= lim) return ray_probe(V, b);
   const uint32_t slot = (uint32_t)(b.x & 7) | ((uint32_t)(b.y & 7) << 3) | ((uint32_t)(b.z & 3) << 6);
   const uint64_t tag = (uint64_t)((uint32_t)(b.x >> 3) & 0x1FFFu) |
                        ((uint64_t)((uint32_t)(b.y >> 3) & 0x1FFFu) << 13) |
                        ((uint64_t)((uint32_t)(b.z >> 2) & 0x3FFFu) << 26);
   const uint64_t e = t->e[slot];
   if (e != 0ull && (e >> 24) == tag) return (int32_t)(e & 0xFFFFFFu) - 3;
-  const int32_t p = coord_ok(b) ? hash_find_eager(V, b) : kFreePtr;
-  if (V.ray_mark && p >= 0) V.ray_mark[p] = V.ray_stamp;  // diagnostics: block sampled
+  const int32_t p = ray_probe(V, b);
   if (p >= (1 << 24) - 3) return p;  // does not fit the entry
   const uint32_t lane = threadIdx.x & 63u;
   volatile uint32_t* owner = t->owner;
@@ -60,164 +73,103 @@ __device__ __forceinline__ int32_t table_find(const View& V, WaveTable* t, i3 b)
   return p;
 }
 
-// The last two lookups of one ray (hits and misses), in registers.
-struct BlockCache {
-  uint64_t k0, k1;
-  int32_t p0, p1;
-  WaveTable* t;
-};
-
-__device__ __forceinline__ int32_t cached_find(const View& V, BlockCache& c, i3 b) {
-  const uint64_t k = pack_key(b);
-  if (k == c.k0) return c.p0;
-  if (k == c.k1) {
-    const uint64_t tk = c.k0;
-    const int32_t tp = c.p0;
-    c.k0 = c.k1;
-    c.p0 = c.p1;
-    c.k1 = tk;
-    c.p1 = tp;
-    return c.p0;
-  }
-  const int32_t p = table_find(V, c.t, b);
-  c.k1 = c.k0;
-  c.p1 = c.p0;
-  c.k0 = k;
-  c.p0 = p;
-  return p;
-}
-
-
-// Pool indices of the blocks holding a trilinear cell's eight corners
-// (corner i = (cx[i>>2 & 1], cy[i>>1 & 1], cz[i & 1])).  Each distinct
-// block is looked up once, lowest corner first, from a single call site (a
-// rolled loop): the probe is emitted once per caller instead of once per
-// corner.  kStop: end at the first missing block (false); otherwise every
-// block is looked up and missing ones are left negative.
-template <bool kStop>
-__device__ __forceinline__ bool corner_blocks(const View& V, BlockCache& cache, const int cx[2],
-                                              const int cy[2], const int cz[2], int32_t pb[8]) {
-  const int bx0 = voxel_to_block1(cx[0]), by0 = voxel_to_block1(cy[0]), bz0 = voxel_to_block1(cz[0]);
-  const bool xx = voxel_to_block1(cx[1]) != bx0, yy = voxel_to_block1(cy[1]) != by0,
-             zz = voxel_to_block1(cz[1]) != bz0;
-  // distinct blocks: entry e = (dx << 2 | dy << 1 | dz) for block b0 + d
-  uint32_t todo = 1;
-#pragma unroll
-  for (int e = 1; e < 8; ++e)
-    if ((!(e & 4) || xx) && (!(e & 2) || yy) && (!(e & 1) || zz)) todo |= 1u << e;
-  int32_t be[8];
-  bool ok = true;
-  while (todo) {
-    const int e = __ffs(todo) - 1;
-    todo &= todo - 1u;
-    const int32_t q = cached_find(V, cache, i3{bx0 + ((e >> 2) & 1), by0 + ((e >> 1) & 1), bz0 + (e & 1)});
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-      if (j == e) be[j] = q;
-    if (q < 0) {
-      ok = false;
-      if (kStop) return false;
-    }
-  }
-  // corner i lies in entry (i & 4 if xx) | (i & 2 if yy) | (i & 1 if zz),
-  // chosen by selects (constant indices keep be[] in registers)
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const bool sx = (i & 4) && xx, sy = (i & 2) && yy, sz = (i & 1) && zz;
-    pb[i] = sx ? (sy ? (sz ? be[7] : be[6]) : (sz ? be[5] : be[4]))
-               : (sy ? (sz ? be[3] : be[2]) : (sz ? be[1] : be[0]));
-  }
-  return ok;
-}
-
-// GetSpatialValue restricted to the SDF (the only field the march uses),
-// without the empty-space test.
-__device__ __forceinline__ bool ray_sdf_full(const View& V, BlockCache& cache, f3 pos, float* out) {
-  const float vs = V.geo.voxel_size;
-  const float hv = 0.5f * vs;
-  const float pcx = pos.x - hv, pcy = pos.y - hv, pcz = pos.z - hv;
-  const float qx = pos.x / vs, qy = pos.y / vs, qz = pos.z / vs;
-  const float rx = qx - floorf(qx), ry = qy - floorf(qy), rz = qz - floorf(qz);
-  const int cx[2] = {vox1(pcx + 0.0f, vs), vox1(pcx + vs, vs)};
-  const int cy[2] = {vox1(pcy + 0.0f, vs), vox1(pcy + vs, vs)};
-  const int cz[2] = {vox1(pcz + 0.0f, vs), vox1(pcz + vs, vs)};
-  // The sample is invalid if any corner's block is missing; in empty space
-  // the lowest corner's block already says so (one cached probe).
-  int32_t pb[8];
-  if (!corner_blocks<true>(V, cache, cx, cy, cz, pb)) return false;
-  float sdf = 0.0f;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int mx = (i >> 2) & 1, my = (i >> 1) & 1, mz = i & 1;
-    const uint32_t li = (uint32_t)((cx[mx] & 7) + 8 * (cy[my] & 7) + 64 * (cz[mz] & 7));
-    const float w = (mx ? rx : 1.0f - rx) * (my ? ry : 1.0f - ry) * (mz ? rz : 1.0f - rz);
-    sdf += w * V.sdf[(size_t)pb[i] * kBlockVoxels + li];
-  }
-  *out = sdf;
-  return true;
-}
-
-// GetSpatialValue's SDF with the empty-space test first.
-__device__ __forceinline__ bool ray_sdf(const View& V, BlockCache& cache, f3 pos, float inv_vs,
-                                        float* out) {
-  const float hv = 0.5f * V.geo.voxel_size;
-  int c0x, c0y, c0z;
-  if (fast_corner(pos.x - hv, inv_vs, &c0x) && fast_corner(pos.y - hv, inv_vs, &c0y) &&
-      fast_corner(pos.z - hv, inv_vs, &c0z) &&
-      cached_find(V, cache, i3{voxel_to_block1(c0x), voxel_to_block1(c0y), voxel_to_block1(c0z)}) < 0)
-    return false;
-  return ray_sdf_full(V, cache, pos, out);
-}
-
 // The eight blocks around a lowest-corner block b: b + (i>>2 & 1, i>>1 & 1,
-// i & 1) for entry i, each looked up when a sample first needs it and kept
-// while the march stays with b.
-constexpr int32_t kNotLooked = INT32_MIN;
+// i & 1) for entry i, kept while the march stays with b.  Entry 0 comes from
+// the wave's table, the others from the block's row of V.oct (below) in two
+// 16-byte loads.
 struct Octant {
   int bx, by, bz;
   int32_t p[8];
 };
 __device__ __forceinline__ Octant empty_octant() {
-  return Octant{INT32_MIN, INT32_MIN, INT32_MIN,
-                {kNotLooked, kNotLooked, kNotLooked, kNotLooked, kNotLooked, kNotLooked, kNotLooked, kNotLooked}};
+  return Octant{INT32_MIN, INT32_MIN, INT32_MIN, {kFreePtr, -1, -1, -1, -1, -1, -1, -1}};
+}
+__device__ __forceinline__ void octant_move(const View& V, WaveTable* t, Octant& oc, int bx, int by, int bz) {
+  if (bx == oc.bx && by == oc.by && bz == oc.bz) return;
+  oc.bx = bx;
+  oc.by = by;
+  oc.bz = bz;
+  oc.p[0] = table_find(V, t, i3{bx, by, bz});
+  if (oc.p[0] < 0) return;
+  const int4* row = reinterpret_cast<const int4*>(V.oct) + 2 * (size_t)oc.p[0];
+  const int4 lo = row[0], hi = row[1];
+  oc.p[1] = lo.y;
+  oc.p[2] = lo.z;
+  oc.p[3] = lo.w;
+  oc.p[4] = hi.x;
+  oc.p[5] = hi.y;
+  oc.p[6] = hi.z;
+  oc.p[7] = hi.w;
 }
 
-// GetSpatialValue's SDF for a march sample (spatial_query.h:23-66).  The
-// corner voxels come from a multiply by 1/vs when the quotient is more than
-// 1e-3 voxel from a rounding tie (the same integers as the reference's
-// divisions, see fast_corner; the upper corner is then the lower + 1, the
-// sum pc + vs being within 1.3e-4 voxel of exact), else from the divisions;
-// the ratios come from the division, as the reference computes them.  A
-// missing lowest-corner block ends the sample after one compare while the
-// octant is cached, which is how empty space inside the tile range costs
-// little.  Octant misses go to the wave's LDS table directly (the cache's
-// two-entry register cache is left out of the march: its registers cost
-// more than the lookups it saves).
-// The sample from its corner voxels; ratios() gives (rx, ry, rz), taken
-// only once the sample is known to be valid.
-template <class Ratios>
-__device__ __forceinline__ bool sample_corners(const View& V, BlockCache& cache, Octant& oc, int cx0, int cx1,
-                                               int cy0, int cy1, int cz0, int cz1, Ratios ratios,
-                                               float* out) {
-  const int bx = voxel_to_block1(cx0), by = voxel_to_block1(cy0), bz = voxel_to_block1(cz0);
-  if (bx != oc.bx || by != oc.by || bz != oc.bz) {
-    oc.bx = bx;
-    oc.by = by;
-    oc.bz = bz;
-    oc.p[0] = table_find(V, cache.t, i3{bx, by, bz});
-#pragma unroll
-    for (int i = 1; i < 8; ++i) oc.p[i] = kNotLooked;
+// One axis of a sample at coordinate p: the two corner voxels of its
+// trilinear cell (rounded from p - vs/2 and p + vs/2, spatial_query.h:23-66;
+// from a multiply by 1/vs when that is clear of a rounding tie, see
+// corner_pair).
+struct RCell {
+  int x0, x1, y0, y1, z0, z1;
+};
+__device__ __forceinline__ RCell ray_cell(f3 pos, float vs, float inv_vs) {
+  const float hv = 0.5f * vs;
+  RCell c;
+  // per axis, so that a wave runs the divisions only for the axes on which
+  // some lane is near a tie
+  corner_pair(pos.x - hv, vs, inv_vs, &c.x0, &c.x1);
+  corner_pair(pos.y - hv, vs, inv_vs, &c.y0, &c.y1);
+  corner_pair(pos.z - hv, vs, inv_vs, &c.z0, &c.z1);
+  return c;
+}
+// The ratio frac(p / vs) of an axis.
+__device__ __forceinline__ float ray_ratio(float p, float vs, float inv_vs) {
+  const float q = quotient(p, vs, inv_vs);
+  return q - floorf(q);
+}
+struct RAxis {
+  int c0, c1;
+  float r;
+};
+__device__ __forceinline__ RAxis ray_axis(float p, float vs, float inv_vs) {
+  RAxis a;
+  corner_pair(p - 0.5f * vs, vs, inv_vs, &a.c0, &a.c1);
+  a.r = ray_ratio(p, vs, inv_vs);
+  return a;
+}
+
+// Where the eight corner voxels of a cell lie in a voxel field (corner i: bit
+// 2 x, bit 1 y, bit 0 z set); false if one of the blocks holding them is
+// absent.  Offsets are in bytes and 32-bit, so that a load takes one address
+// register beside the field's scalar base, unless the pool is larger than
+// kNarrowCapacity blocks (kWide: 64-bit).
+constexpr uint32_t kNarrowCapacity = 1u << 21;  // x 2 KiB a block
+template <bool kWide>
+struct RayOffset { using type = uint32_t; };
+template <>
+struct RayOffset<true> { using type = uint64_t; };
+template <bool kWide>
+using ray_offset = typename RayOffset<kWide>::type;
+template <bool kWide>
+__device__ __forceinline__ float field_at(const float* __restrict__ f, ray_offset<kWide> off) {
+  return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(f) + off);
+}
+template <bool kWide>
+__device__ __forceinline__ bool cell_corners(const View& V, WaveTable* t, Octant& oc, const RCell& c,
+                                             ray_offset<kWide> off[8]) {
+  const int bx = voxel_to_block1(c.x0), by = voxel_to_block1(c.y0), bz = voxel_to_block1(c.z0);
+  octant_move(V, t, oc, bx, by, bz);
+  if (oc.p[0] < 0) {
+    return false;
   }
-  if (oc.p[0] < 0) return false;
-  const bool xx = voxel_to_block1(cx1) != bx, yy = voxel_to_block1(cy1) != by, zz = voxel_to_block1(cz1) != bz;
+  const bool xx = voxel_to_block1(c.x1) != bx, yy = voxel_to_block1(c.y1) != by, zz = voxel_to_block1(c.z1) != bz;
+  if (V.ray_mark) {  // diagnostics: blocks sampled
+    V.ray_mark[oc.p[0]] = V.ray_stamp;
 #pragma unroll
-  for (int i = 1; i < 8; ++i) {
-    const bool need = (!(i & 4) || xx) && (!(i & 2) || yy) && (!(i & 1) || zz);
-    if (!need) continue;
-    if (oc.p[i] == kNotLooked) oc.p[i] = table_find(V, cache.t, i3{bx + ((i >> 2) & 1), by + ((i >> 1) & 1), bz + (i & 1)});
-    if (oc.p[i] < 0) return false;
+    for (int i = 1; i < 8; ++i) {
+      if (!((!(i & 4) || xx) && (!(i & 2) || yy) && (!(i & 1) || zz))) continue;
+      if (oc.p[i] < 0) return false;
+      V.ray_mark[oc.p[i]] = V.ray_stamp;
+    }
   }
-  // block of each corner (bit 2: x, bit 1: y, bit 0: z set), by selects
+  // block of each corner, by selects
   const int32_t p0 = oc.p[0];
   const int32_t p1 = zz ? oc.p[1] : p0;
   const int32_t p2 = yy ? oc.p[2] : p0;
@@ -226,59 +178,86 @@ __device__ __forceinline__ bool sample_corners(const View& V, BlockCache& cache,
   const int32_t p5 = xx ? (zz ? oc.p[5] : oc.p[4]) : p1;
   const int32_t p6 = xx ? (yy ? oc.p[6] : oc.p[4]) : p2;
   const int32_t p7 = xx ? (yy ? (zz ? oc.p[7] : oc.p[6]) : (zz ? oc.p[5] : oc.p[4])) : p3;
+  if (min(min(min(p1, p2), min(p3, p4)), min(min(p5, p6), p7)) < 0) return false;
+  const uint32_t x0 = (uint32_t)(c.x0 & 7) * 4u, x1 = (uint32_t)(c.x1 & 7) * 4u;
+  const uint32_t y0 = (uint32_t)(c.y0 & 7) * 32u, y1 = (uint32_t)(c.y1 & 7) * 32u;
+  const uint32_t z0 = (uint32_t)(c.z0 & 7) * 256u, z1 = (uint32_t)(c.z1 & 7) * 256u;
   const int32_t pb[8] = {p0, p1, p2, p3, p4, p5, p6, p7};
-  const int cx[2] = {cx0, cx1}, cy[2] = {cy0, cy1}, cz[2] = {cz0, cz1};
-  const f3 r = ratios();
-  const float rx = r.x, ry = r.y, rz = r.z;
-  float sdf = 0.0f;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int mx = (i >> 2) & 1, my = (i >> 1) & 1, mz = i & 1;
-    const uint32_t li = (uint32_t)((cx[mx] & 7) + 8 * (cy[my] & 7) + 64 * (cz[mz] & 7));
-    const float w = (mx ? rx : 1.0f - rx) * (my ? ry : 1.0f - ry) * (mz ? rz : 1.0f - rz);
-    sdf += w * V.sdf[(size_t)pb[i] * kBlockVoxels + li];
-  }
-  *out = sdf;
+  for (int i = 0; i < 8; ++i)
+    off[i] = (ray_offset<kWide>)(uint32_t)pb[i] * (kBlockVoxels * 4u) +
+             (((i & 4) ? x1 : x0) + ((i & 2) ? y1 : y0) + ((i & 1) ? z1 : z0));
   return true;
 }
 
-__device__ __forceinline__ bool march_sample(const View& V, BlockCache& cache, Octant& oc, f3 pos,
-                                             float inv_vs, float* out) {
+// The trilinear sum of GetSpatialValue (spatial_query.h:23-66), corner by
+// corner in the reference's order.
+__device__ __forceinline__ float trilinear(const float v[8], float rx, float ry, float rz) {
+  float sdf = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float w = ((i & 4) ? rx : 1.0f - rx) * ((i & 2) ? ry : 1.0f - ry) * ((i & 1) ? rz : 1.0f - rz);
+    sdf += w * v[i];
+  }
+  return sdf;
+}
+
+// GetSpatialValue's SDF at a point; false if a corner's block is absent (a
+// missing lowest-corner block ends the sample after one compare while the
+// octant is kept, which is how empty space inside the tile range costs
+// little).  The ratios are the reference's quotients.
+template <bool kWide>
+__device__ __forceinline__ bool point_sample(const View& V, WaveTable* t, Octant& oc, f3 pos, float inv_vs,
+                                             float* out) {
   const float vs = V.geo.voxel_size;
-  const float hv = 0.5f * vs;
-  const float pcx = pos.x - hv, pcy = pos.y - hv, pcz = pos.z - hv;
-  // per axis, so that a wave runs the divisions only for the axes on which
-  // some lane is near a tie
-  int cx0, cy0, cz0, cx1, cy1, cz1;
-  corner_pair(pcx, vs, inv_vs, &cx0, &cx1);
-  corner_pair(pcy, vs, inv_vs, &cy0, &cy1);
-  corner_pair(pcz, vs, inv_vs, &cz0, &cz1);
-  return sample_corners(V, cache, oc, cx0, cx1, cy0, cy1, cz0, cz1, [&] {
-    const float qx = pos.x / vs, qy = pos.y / vs, qz = pos.z / vs;
-    return mk3(qx - floorf(qx), qy - floorf(qy), qz - floorf(qz));
-  }, out);
+  ray_offset<kWide> off[8];
+  if (!cell_corners<kWide>(V, t, oc, ray_cell(pos, vs, inv_vs), off)) return false;
+  float v[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = field_at<kWide>(V.sdf, off[i]);
+  *out = trilinear(v, ray_ratio(pos.x, vs, inv_vs), ray_ratio(pos.y, vs, inv_vs), ray_ratio(pos.z, vs, inv_vs));
+  return true;
 }
 
-// One axis of a sample at coordinate p: its two corner voxels (as
-// march_sample rounds them) and the ratio frac(p / vs).
-struct RAxis {
-  int c0, c1;
-  float r;
-};
-__device__ __forceinline__ RAxis ray_axis(float p, float vs, float inv_vs) {
-  RAxis a;
-  corner_pair(p - 0.5f * vs, vs, inv_vs, &a.c0, &a.c1);
-  const float q = p / vs;
-  a.r = q - floorf(q);
-  return a;
-}
-
-// march_sample from the sample's three axes (the normal's stencils share two
-// of them with the crossing point).
-__device__ __forceinline__ bool axes_sample(const View& V, BlockCache& cache, Octant& oc, const RAxis& X,
-                                            const RAxis& Y, const RAxis& Z, float* out) {
-  return sample_corners(V, cache, oc, X.c0, X.c1, Y.c0, Y.c1, Z.c0, Z.c1, [&] { return mk3(X.r, Y.r, Z.r); },
-                        out);
+// GetSpatialSDFGradient's samples at p -+ vs/2 e_k (spatial_query.h:68-97):
+// as central differences; false if any is invalid.  p -+ h e_k equals p off
+// axis k (x - 0 = x), so the stencils take p's own axes there.  One sample site
+// in a rolled loop: an axis's two samples loaded together need 128 registers
+// (four waves a SIMD) and were slower, 640 x 480 of a 5 mm desk 175 against
+// 165 us.
+template <bool kWide>
+__device__ __forceinline__ bool gradient_samples(const View& V, WaveTable* t, Octant& oc, f3 p, float inv_vs,
+                                                 float* g0, float* g1, float* g2) {
+  const float vs = V.geo.voxel_size;
+  const float h = 0.5f * vs;
+  const RAxis X = ray_axis(p.x, vs, inv_vs), Y = ray_axis(p.y, vs, inv_vs), Z = ray_axis(p.z, vs, inv_vs);
+  bool valid = true;
+  float last = 0.0f;
+  *g0 = *g1 = *g2 = 0.0f;
+  // x-, x+, y-, y+, z-, z+ from one sample site
+#pragma unroll 1
+  for (int j = 0; j < 6 && valid; ++j) {
+    const int k = j >> 1;
+    const float pk = k == 0 ? p.x : (k == 1 ? p.y : p.z);
+    const RAxis S = ray_axis((j & 1) ? pk + h : pk - h, vs, inv_vs);
+    RCell c{X.c0, X.c1, Y.c0, Y.c1, Z.c0, Z.c1};
+    if (k == 0) { c.x0 = S.c0; c.x1 = S.c1; }
+    if (k == 1) { c.y0 = S.c0; c.y1 = S.c1; }
+    if (k == 2) { c.z0 = S.c0; c.z1 = S.c1; }
+    ray_offset<kWide> off[8];
+    valid = cell_corners<kWide>(V, t, oc, c, off);
+    if (!valid) break;
+    float v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = field_at<kWide>(V.sdf, off[i]);
+    const float s = trilinear(v, k == 0 ? S.r : X.r, k == 1 ? S.r : Y.r, k == 2 ? S.r : Z.r);
+    const float gk = (s - last) / vs;
+    last = s;
+    if (j == 1) *g0 = gk;
+    if (j == 3) *g1 = gk;
+    if (j == 5) *g2 = gk;
+  }
+  return valid;
 }
 
 // A ray parameter below which every sample position o + t dir lies more
@@ -304,12 +283,11 @@ __device__ __forceinline__ float cell_exit_t(f3 o, f3 dir, int bx, int by, int b
 __device__ __forceinline__ float block_exit_t(f3 o, f3 dir, int bx, int by, int bz, float vs) {
   return cell_exit_t(o, dir, bx, by, bz, (float)kBlockSide * vs, vs);
 }
-// The same for the super-block (4^3 blocks) holding block b, when no block of
-// it was ever allocated (its filter bit is clear): every sample whose
-// lowest-corner block lies in it is invalid.  Otherwise block_exit_t.
-__device__ __forceinline__ float absent_exit_t(const View& V, f3 o, f3 dir, int bx, int by, int bz, float vs) {
-  const uint32_t sb = occ2_bit(super_key(i3{bx, by, bz}));
-  if ((V.occ2[sb >> 5] >> (sb & 31u)) & 1u) return block_exit_t(o, dir, bx, by, bz, vs);
+// The same for an absent block: over its super-block (4^3 blocks) when no
+// block of that was ever allocated, every sample whose lowest-corner block
+// lies in it being invalid.
+__device__ __forceinline__ float absent_exit_t(int32_t found, f3 o, f3 dir, int bx, int by, int bz, float vs) {
+  if (found != kAbsentSuper) return block_exit_t(o, dir, bx, by, bz, vs);
   return cell_exit_t(o, dir, bx >> kSuperShift, by >> kSuperShift, bz >> kSuperShift,
                      (float)(kBlockSide << kSuperShift) * vs, vs);
 }
@@ -363,8 +341,9 @@ struct Hit {
 // tile's block range): earlier samples are stepped over without sampling,
 // so the sample sequence t_min, t_min + step, ... stays the reference's, and
 // the march ends after t_hi.
+template <bool kWide>
 __device__ __forceinline__ bool find_surface(const View& V, const RayConst& R, f3 o, f3 dir, float t_min,
-                                             float t_max, float t_lo, float t_hi, BlockCache& cache,
+                                             float t_max, float t_lo, float t_hi, WaveTable* table,
                                              Octant& oc, Hit* hit, uint32_t* nsamp) {
   float prev_sdf = 0.0f, prev_t = 0.0f;
   bool prev_ok = false;
@@ -378,14 +357,14 @@ __device__ __forceinline__ bool find_surface(const View& V, const RayConst& R, f
     bool cross = false;
     for (; t < t_max && t <= t_hi; t += R.step) {
       float sv;
-      if (!march_sample(V, cache, oc, mk3(o.x + t * dir.x, o.y + t * dir.y, o.z + t * dir.z), R.inv_vs,
-                        &sv)) {
+      if (!point_sample<kWide>(V, table, oc, mk3(o.x + t * dir.x, o.y + t * dir.y, o.z + t * dir.z), R.inv_vs,
+                               &sv)) {
         // Lowest-corner block absent: the following samples inside its box
         // (its super-block's, if that never held a block) are invalid too
         // (an invalid sample changes nothing); step over them with the same
         // FP32 additions, so the t sequence is kept.
         if (oc.p[0] < 0) {
-          const float t_out = absent_exit_t(V, o, dir, oc.bx, oc.by, oc.bz, V.geo.voxel_size);
+          const float t_out = absent_exit_t(oc.p[0], o, dir, oc.bx, oc.by, oc.bz, V.geo.voxel_size);
           for (float tn = t + R.step; tn < t_out && tn > t; tn = t + R.step) t = tn;
         }
         continue;
@@ -405,11 +384,12 @@ __device__ __forceinline__ bool find_surface(const View& V, const RayConst& R, f
     float l = prev_t, r = t, m = (l + r) * 0.5f;
     float l_sdf = prev_sdf, r_sdf = s;
     bool found = true;
+#pragma unroll 1
     for (int k = 0; k < 3; ++k) {
       m = l + (l_sdf / (l_sdf - r_sdf)) * (r - l);
       float m_sdf;
-      if (!march_sample(V, cache, oc, mk3(o.x + m * dir.x, o.y + m * dir.y, o.z + m * dir.z), R.inv_vs,
-                        &m_sdf)) {
+      if (!point_sample<kWide>(V, table, oc, mk3(o.x + m * dir.x, o.y + m * dir.y, o.z + m * dir.z), R.inv_vs,
+                               &m_sdf)) {
         found = false;
         break;
       }
@@ -434,13 +414,9 @@ __device__ __forceinline__ bool find_surface(const View& V, const RayConst& R, f
 }
 
 // The ray parameters between which pixel (x, y) can meet an allocated block:
-// the tile's camera-z range over dir_c.z, widened by 0.1 %.  Without a range
-// pass, the whole [t_min, t_max].
+// the tile's camera-z range over dir_c.z, widened by 0.1 %.
 __device__ __forceinline__ void ray_bounds(const RayConst& R, uint32_t x, uint32_t y, float dcz, float t_min,
                                            float t_max, float* t_lo, float* t_hi) {
-  *t_lo = t_min;
-  *t_hi = t_max;
-  if (!R.range) return;
   const uint32_t tile = (y >> 3) * R.tiles_x + (x >> 3);
   const float zmin = __uint_as_float(R.range[2 * tile]);
   const float zmax = __uint_as_float(R.range[2 * tile + 1]);
@@ -449,6 +425,7 @@ __device__ __forceinline__ void ray_bounds(const RayConst& R, uint32_t x, uint32
 }
 
 // March one pixel; returns the number of valid samples taken.
+template <bool kWide>
 __device__ __forceinline__ uint32_t cast_pixel(const View& V, const RayConst& R, uint32_t x, uint32_t y,
                                WaveTable* table, float* res_d, f3* res_v, f3* res_n) {
   uint32_t nsamp = 0;
@@ -462,36 +439,19 @@ __device__ __forceinline__ uint32_t cast_pixel(const View& V, const RayConst& R,
   const f3 o = xform(R.wTc, mk3(0.0f, 0.0f, 0.0f));
   const f3 dir = normalize(xform_dir(R.wTc, dir_c));
 
-  BlockCache cache{kEmptyKey, kEmptyKey, kFreePtr, kFreePtr, table};
   Hit hit;
   float t_lo, t_hi;
   ray_bounds(R, x, y, dir_c.z, t_min, t_max, &t_lo, &t_hi);
   Octant oc = empty_octant();
-  if (find_surface(V, R, o, dir, t_min, t_max, t_lo, t_hi, cache, oc, &hit, &nsamp)) {
+  if (find_surface<kWide>(V, R, o, dir, t_min, t_max, t_lo, t_hi, table, oc, &hit, &nsamp)) {
     const float m = hit.m;
     const float d = m * dir_c.z;
     out_d = d;
     out_v = reproject(R.cam, x, y, d);
     if (R.enable_gradients) {
       const f3 iso = mk3(o.x + m * dir.x, o.y + m * dir.y, o.z + m * dir.z);
-      const float h = 0.5f * V.geo.voxel_size;
-      bool valid = true;
-      float sp[3] = {0, 0, 0}, sn[3] = {0, 0, 0};
-      const float vs = V.geo.voxel_size;
-      // iso -+ h e_k equals iso off axis k (x - 0 = x), so the stencils take
-      // the crossing point's axes there
-      const RAxis X = ray_axis(iso.x, vs, R.inv_vs), Y = ray_axis(iso.y, vs, R.inv_vs),
-                  Z = ray_axis(iso.z, vs, R.inv_vs);
-#pragma unroll
-      for (int k = 0; k < 3 && valid; ++k) {
-        const float ik = k == 0 ? iso.x : (k == 1 ? iso.y : iso.z);
-        const RAxis An = ray_axis(ik - h, vs, R.inv_vs);
-        valid = axes_sample(V, cache, oc, k == 0 ? An : X, k == 1 ? An : Y, k == 2 ? An : Z, &sn[k]);
-        if (!valid) break;
-        const RAxis Ap = ray_axis(ik + h, vs, R.inv_vs);
-        valid = axes_sample(V, cache, oc, k == 0 ? Ap : X, k == 1 ? Ap : Y, k == 2 ? Ap : Z, &sp[k]);
-      }
-      const f3 grad = mk3((sp[0] - sn[0]) / vs, (sp[1] - sn[1]) / vs, (sp[2] - sn[2]) / vs);
+      f3 grad;
+      const bool valid = gradient_samples<kWide>(V, table, oc, iso, R.inv_vs, &grad.x, &grad.y, &grad.z);
       const float l2 = length(grad);
       f3 nw = (l2 > 0.0f && valid) ? grad / l2 : mk3(0.0f, 0.0f, 0.0f);
       nw = -nw;
@@ -506,26 +466,23 @@ __device__ __forceinline__ uint32_t cast_pixel(const View& V, const RayConst& R,
 
 // ------------------------------------------------------------ adjoint
 // GetSpatialValue's SDF (same corners, weights and summation order as
-// ray_sdf, so the value is bit-identical) with the spatial gradient of the
+// point_sample, so the value is bit-identical) with the spatial gradient of the
 // trilinear interpolant: each ratio frac(pos / vs) moves at 1 / vs.
-__device__ __forceinline__ bool ray_sdf_grad(const View& V, BlockCache& cache, f3 pos, float* val,
+template <bool kWide>
+__device__ __forceinline__ bool ray_sdf_grad(const View& V, WaveTable* t, Octant& oc, f3 pos, float inv_vs, float* val,
                                              f3* grad) {
   const float vs = V.geo.voxel_size;
-  const float hv = 0.5f * vs;
-  const float pcx = pos.x - hv, pcy = pos.y - hv, pcz = pos.z - hv;
-  const float qx = pos.x / vs, qy = pos.y / vs, qz = pos.z / vs;
-  const float rx = qx - floorf(qx), ry = qy - floorf(qy), rz = qz - floorf(qz);
-  const int cx[2] = {vox1(pcx + 0.0f, vs), vox1(pcx + vs, vs)};
-  const int cy[2] = {vox1(pcy + 0.0f, vs), vox1(pcy + vs, vs)};
-  const int cz[2] = {vox1(pcz + 0.0f, vs), vox1(pcz + vs, vs)};
-  int32_t pb[8];
-  if (!corner_blocks<true>(V, cache, cx, cy, cz, pb)) return false;
+  const float rx = ray_ratio(pos.x, vs, inv_vs), ry = ray_ratio(pos.y, vs, inv_vs), rz = ray_ratio(pos.z, vs, inv_vs);
+  ray_offset<kWide> off[8];
+  if (!cell_corners<kWide>(V, t, oc, ray_cell(pos, vs, inv_vs), off)) return false;
+  float v[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = field_at<kWide>(V.sdf, off[i]);
   float sdf = 0.0f, gx = 0.0f, gy = 0.0f, gz = 0.0f;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const int mx = (i >> 2) & 1, my = (i >> 1) & 1, mz = i & 1;
-    const uint32_t li = (uint32_t)((cx[mx] & 7) + 8 * (cy[my] & 7) + 64 * (cz[mz] & 7));
-    const float c = V.sdf[(size_t)pb[i] * kBlockVoxels + li];
+    const float c = v[i];
     const float wx = mx ? rx : 1.0f - rx, wy = my ? ry : 1.0f - ry, wz = mz ? rz : 1.0f - rz;
     sdf += wx * wy * wz * c;
     gx += (mx ? c : -c) * wy * wz;
@@ -537,25 +494,20 @@ __device__ __forceinline__ bool ray_sdf_grad(const View& V, BlockCache& cache, f
   return true;
 }
 
-// Adds coef * (trilinear weight of each corner) to the corners' gradient.
-__device__ __forceinline__ void scatter_sdf(const View& V, BlockCache& cache, f3 pos, float coef,
+// Adds coef * (trilinear weight of each corner) to the corners' gradient, for
+// a sample that the forward pass accepted (all its blocks exist).
+template <bool kWide>
+__device__ __forceinline__ void scatter_sdf(const View& V, WaveTable* t, Octant& oc, f3 pos, float inv_vs, float coef,
                                             float* __restrict__ grad_sdf) {
   const float vs = V.geo.voxel_size;
-  const float hv = 0.5f * vs;
-  const float pcx = pos.x - hv, pcy = pos.y - hv, pcz = pos.z - hv;
-  const float qx = pos.x / vs, qy = pos.y / vs, qz = pos.z / vs;
-  const float rx = qx - floorf(qx), ry = qy - floorf(qy), rz = qz - floorf(qz);
-  const int cx[2] = {vox1(pcx + 0.0f, vs), vox1(pcx + vs, vs)};
-  const int cy[2] = {vox1(pcy + 0.0f, vs), vox1(pcy + vs, vs)};
-  const int cz[2] = {vox1(pcz + 0.0f, vs), vox1(pcz + vs, vs)};
-  int32_t pb[8];
-  corner_blocks<false>(V, cache, cx, cy, cz, pb);
+  const float rx = ray_ratio(pos.x, vs, inv_vs), ry = ray_ratio(pos.y, vs, inv_vs), rz = ray_ratio(pos.z, vs, inv_vs);
+  ray_offset<kWide> off[8];
+  if (!cell_corners<kWide>(V, t, oc, ray_cell(pos, vs, inv_vs), off)) return;
+#pragma unroll
   for (int i = 0; i < 8; ++i) {
     const int mx = (i >> 2) & 1, my = (i >> 1) & 1, mz = i & 1;
-    if (pb[i] < 0) continue;  // cannot happen for a sample the forward pass accepted
-    const uint32_t li = (uint32_t)((cx[mx] & 7) + 8 * (cy[my] & 7) + 64 * (cz[mz] & 7));
     const float w = (mx ? rx : 1.0f - rx) * (my ? ry : 1.0f - ry) * (mz ? rz : 1.0f - rz);
-    atomicAdd(&grad_sdf[(size_t)pb[i] * kBlockVoxels + li], coef * w);
+    atomicAdd(reinterpret_cast<float*>(reinterpret_cast<char*>(grad_sdf) + off[i]), coef * w);
   }
 }
 
@@ -577,8 +529,9 @@ __device__ __forceinline__ void sample_tangent(f3 x, f3 g, int slot, float* t) {
 // Differentiates the rendered depth of one pixel: recomputes the march
 // (same decisions as the forward pass), then carries tangents through the
 // three regula-falsi steps.  Returns false when the pixel has no hit.
+template <bool kWide>
 __device__ __forceinline__ bool depth_tangent(const View& V, const RayConst& R, uint32_t x, uint32_t y,
-                                              BlockCache& cache, float* depth, float* dd, f3* X) {
+                                              WaveTable* table, Octant& oc, float* depth, float* dd, f3* X) {
   const f3 dir_c = normalize(reproject(R.cam, x, y, 1.0f));
   const float t_min = R.min_depth / dir_c.z;
   const float t_max = R.max_depth / dir_c.z;
@@ -588,16 +541,15 @@ __device__ __forceinline__ bool depth_tangent(const View& V, const RayConst& R, 
   uint32_t ns = 0;
   float t_lo, t_hi;
   ray_bounds(R, x, y, dir_c.z, t_min, t_max, &t_lo, &t_hi);
-  Octant oc = empty_octant();
-  if (!find_surface(V, R, o, dir, t_min, t_max, t_lo, t_hi, cache, oc, &hit, &ns)) return false;
+  if (!find_surface<kWide>(V, R, o, dir, t_min, t_max, t_lo, t_hi, table, oc, &hit, &ns)) return false;
   float l = hit.tp, r = hit.tk, ls, rs;
   float dl[kTan], dr[kTan], dls[kTan], drs[kTan], dm[kTan];
   f3 g;
   X[0] = mk3(o.x + l * dir.x, o.y + l * dir.y, o.z + l * dir.z);
   X[1] = mk3(o.x + r * dir.x, o.y + r * dir.y, o.z + r * dir.z);
-  ray_sdf_grad(V, cache, X[0], &ls, &g);
+  ray_sdf_grad<kWide>(V, table, oc, X[0], R.inv_vs, &ls, &g);
   sample_tangent(X[0], g, 6, dls);
-  ray_sdf_grad(V, cache, X[1], &rs, &g);
+  ray_sdf_grad<kWide>(V, table, oc, X[1], R.inv_vs, &rs, &g);
   sample_tangent(X[1], g, 7, drs);
 #pragma unroll
   for (int k = 0; k < kTan; ++k) dl[k] = dr[k] = 0.0f;
@@ -618,7 +570,7 @@ __device__ __forceinline__ bool depth_tangent(const View& V, const RayConst& R, 
     for (int q = 0; q < 3; ++q)
       if (j == q) X[2 + q] = xm;
     float ms;
-    ray_sdf_grad(V, cache, xm, &ms, &g);
+    ray_sdf_grad<kWide>(V, table, oc, xm, R.inv_vs, &ms, &g);
     float dms[kTan];
     sample_tangent(xm, g, 8 + j, dms);
     const float gd = g.x * dir.x + g.y * dir.y + g.z * dir.z;
@@ -653,6 +605,7 @@ __device__ __forceinline__ bool depth_tangent(const View& V, const RayConst& R, 
 // wave): FP64 sums of r^2 / 2, r J, J J^T (upper triangle) and the pixel
 // count, reduced in a fixed order by raycast_grad_reduce_kernel.  With
 // grad_sdf, r * d depth / d sdf is scattered onto the voxels.
+template <bool kWide>
 __global__ __launch_bounds__(64) void raycast_backward_kernel(View V, RayConst R,
                                                               const float* __restrict__ obs,
                                                               float* __restrict__ grad_sdf,
@@ -667,11 +620,11 @@ __global__ __launch_bounds__(64) void raycast_backward_kernel(View V, RayConst R
   for (int k = 0; k < kGradSlots; ++k) acc[k] = 0.0;
   if (x < R.cam.width && y < R.cam.height) {
     const float od = obs[y * R.cam.width + x];
-    BlockCache cache{kEmptyKey, kEmptyKey, kFreePtr, kFreePtr, &table};
+    Octant oc = empty_octant();
     float d, dd[kTan];
     f3 X[5];
     acc[30] = od > 0.0f && od < INFINITY ? 1.0 : 0.0;
-    if (od > 0.0f && od < INFINITY && depth_tangent(V, R, x, y, cache, &d, dd, X) &&
+    if (od > 0.0f && od < INFINITY && depth_tangent<kWide>(V, R, x, y, &table, oc, &d, dd, X) &&
         fmaxf(fabsf(dd[3]), fmaxf(fabsf(dd[4]), fabsf(dd[5]))) <= max_slope) {
       const float res = d - od;
       if (!(fabsf(res) <= max_residual)) {
@@ -687,7 +640,18 @@ __global__ __launch_bounds__(64) void raycast_backward_kernel(View V, RayConst R
           for (int j = i; j < 6; ++j) acc[t++] = (double)dd[i] * (double)dd[j];
         acc[28] = 1.0;
         if (grad_sdf)
-          for (int e = 0; e < 5; ++e) scatter_sdf(V, cache, X[e], res * dd[6 + e], grad_sdf);
+#pragma unroll 1
+          for (int e = 0; e < 5; ++e) {
+            f3 x = X[0];
+            float c = dd[6];
+#pragma unroll
+            for (int q = 1; q < 5; ++q)
+              if (e == q) {
+                x = X[q];
+                c = dd[6 + q];
+              }
+            scatter_sdf<kWide>(V, &table, oc, x, R.inv_vs, res * c, grad_sdf);
+          }
       }
     }
   }
@@ -763,6 +727,7 @@ void launch_slot_reduce(double* partials, uint32_t n, uint32_t slots, uint32_t* 
 // mat6x6 arithmetic; they are summed in FP64 per wave and then per
 // workgroup in a fixed order instead of float atomics.  Slots: A's upper
 // triangle (21), b (6), err, count.
+template <bool kWide>
 __global__ __launch_bounds__(64) void point_to_psdf_kernel(View V, M4 wTc, float inv_vs, int corrected,
                                                            double* __restrict__ partials) {
   __shared__ WaveTable table;
@@ -776,28 +741,11 @@ __global__ __launch_bounds__(64) void point_to_psdf_kernel(View V, M4 wTc, float
     const float depth = V.depth[(size_t)y * V.cam.width + x];
     if (!(depth == -INFINITY || depth == 0.0f || depth >= V.geo.sdf_upper_bound)) {
       const f3 pw = xform(wTc, reproject(V.cam, x, y, depth));
-      BlockCache cache{kEmptyKey, kEmptyKey, kFreePtr, kFreePtr, &table};
+      Octant oc = empty_octant();
       float d;
-      if (ray_sdf(V, cache, pw, inv_vs, &d)) {
-        const float h = 0.5f * V.geo.voxel_size;
-        bool ok = true;
-        float sp[3] = {0, 0, 0}, sn[3] = {0, 0, 0};
-        // x-, x+, y-, y+, z-, z+ from one (rolled) sample site
-#pragma unroll 1
-        for (int j = 0; j < 6 && ok; ++j) {
-          const int k = j >> 1;
-          const f3 dp = mk3(k == 0 ? h : 0.0f, k == 1 ? h : 0.0f, k == 2 ? h : 0.0f);
-          float v;
-          ok = ray_sdf(V, cache, (j & 1) ? pw + dp : pw - dp, inv_vs, &v);
-#pragma unroll
-          for (int q = 0; q < 3; ++q) {
-            if (j == 2 * q) sn[q] = v;
-            if (j == 2 * q + 1) sp[q] = v;
-          }
-        }
-        if (ok) {
-          const float vs = V.geo.voxel_size;
-          const f3 g = mk3((sp[0] - sn[0]) / vs, (sp[1] - sn[1]) / vs, (sp[2] - sn[2]) / vs);
+      if (point_sample<kWide>(V, &table, oc, pw, inv_vs, &d)) {
+        f3 g;
+        if (gradient_samples<kWide>(V, &table, oc, pw, inv_vs, &g.x, &g.y, &g.z)) {
           const float J[6] = {g.x, g.y, corrected ? g.z : g.x,
                               -g.y * pw.z + g.z * pw.y,
                               -g.z * pw.x + g.x * pw.z,
@@ -835,7 +783,10 @@ uint32_t point_to_psdf_partials(const View& V) {
 void launch_point_to_psdf(const View& V, const M4& wTc, int corrected, double* partials, double* out,
                           hipStream_t s) {
   const dim3 grid((V.cam.width / 2 + 7) / 8, (V.cam.height / 2 + 7) / 8);
-  point_to_psdf_kernel<<<grid, 64, 0, s>>>(V, wTc, 1.0f / V.geo.voxel_size, corrected, partials);
+  if (V.capacity > kNarrowCapacity)
+    point_to_psdf_kernel<true><<<grid, 64, 0, s>>>(V, wTc, 1.0f / V.geo.voxel_size, corrected, partials);
+  else
+    point_to_psdf_kernel<false><<<grid, 64, 0, s>>>(V, wTc, 1.0f / V.geo.voxel_size, corrected, partials);
   launch_slot_reduce(partials, grid.x * grid.y, kP2SSlots, &V.ctr->reduce_done, out, s);
 }
 
@@ -847,10 +798,10 @@ __device__ __forceinline__ const RayConst& ray_of(const Many& m, uint32_t s, con
 // Scene = blockIdx.z; a batch's outputs are scene-major (W*H per scene).
 // At most 96 registers: five waves per SIMD hold a 640x480 frame's 4800
 // tiles at once on 256 CUs (four would leave a partial second round).
-// TW: tile width in pixels (the tile is TW x 64 / TW; every shape gives the
-// same per-pixel results, the autotuner picks the fastest).
-template <class Src, int TW = 8>
-__global__ __launch_bounds__(64, kRayWavesPerSimd) void raycast_kernel(Src src_, const SceneFrame* __restrict__ tab, RayConst R1, float* __restrict__ depth_out,
+// tw: log2 of the tile's width in pixels (the tile has 64; every shape gives
+// the same per-pixel results, the autotuner picks the fastest).
+template <class Src, bool kWide>
+__global__ __launch_bounds__(64, kRayWavesPerSimd) void raycast_kernel(Src src_, const SceneFrame* __restrict__ tab, RayConst R1, int tw, float* __restrict__ depth_out,
                                                      float* __restrict__ vertex_out,
                                                      float* __restrict__ normal_out) {
   const Src src = with_table(src_, tab);
@@ -862,15 +813,14 @@ __global__ __launch_bounds__(64, kRayWavesPerSimd) void raycast_kernel(Src src_,
   const View V = src.view(scene);
   const RayConst R = ray_of(src, scene, R1);
   if (R.boost) __builtin_amdgcn_s_setprio(2);
-  constexpr int TH = 64 / TW;
-  const uint32_t x = blockIdx.x * TW + (threadIdx.x % TW);
-  const uint32_t y = blockIdx.y * TH + (threadIdx.x / TW);
+  const uint32_t x = (blockIdx.x << tw) + (threadIdx.x & ((1u << tw) - 1u));
+  const uint32_t y = (blockIdx.y << (6 - tw)) + (threadIdx.x >> tw);
   uint32_t ns = 0;
   if (x < R.cam.width && y < R.cam.height) {
     const size_t pix = (size_t)scene * R.cam.width * R.cam.height + y * R.cam.width + x;
     float d;
     f3 vv, nn;
-    ns = cast_pixel(V, R, x, y, &table, &d, &vv, &nn);
+    ns = cast_pixel<kWide>(V, R, x, y, &table, &d, &vv, &nn);
     if (depth_out) depth_out[pix] = d;
     if (vertex_out) {
       vertex_out[3 * pix + 0] = vv.x;
@@ -898,12 +848,38 @@ __global__ __launch_bounds__(64, kRayWavesPerSimd) void raycast_kernel(Src src_,
 // such blocks beside it (a wall's, at the camera's own depth), and switching the
 // ranges off for them made every ray walk up to its surface from min_depth (5 mm
 // room at 1237 x 931: the march 854 us, 499 us with the ranges).
+//
+// Before it, one launch clears the tile ranges (its first kClearGroups
+// workgroups) and fills the blocks' rows of V.oct: the pool indices of the
+// eight blocks b + {0, 1}^3 of every allocated block b, eight lanes a block.  A
+// march sample then has its corners' blocks from two 16-byte loads instead of
+// up to seven lookups that a wave's lanes ran one after another.
+constexpr uint32_t kClearGroups = 8;
 template <class Src>
-__global__ __launch_bounds__(256) void ray_range_clear_kernel(Src src_, const SceneFrame* __restrict__ tab, RayConst R1) {
+__global__ __launch_bounds__(256) void ray_prepare_kernel(Src src_, const SceneFrame* __restrict__ tab, RayConst R1) {
   const Src src = with_table(src_, tab);
-  const RayConst& R = ray_of(src, blockIdx.y, R1);
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < 2 * R.tiles; i += gridDim.x * blockDim.x)
-    R.range[i] = (i & 1u) ? 0u : 0x7f800000u;  // zmin +inf, zmax 0
+  if (blockIdx.x < kClearGroups) {
+    const RayConst& R = ray_of(src, blockIdx.y, R1);
+    if (!R.range) return;
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < 2 * R.tiles; i += kClearGroups * blockDim.x)
+      R.range[i] = (i & 1u) ? 0u : 0x7f800000u;  // zmin +inf, zmax 0
+    return;
+  }
+  const View V = src.view(blockIdx.y);
+  const size_t n = (size_t)V.ctr->block_hwm * 8;
+  for (size_t i = (size_t)(blockIdx.x - kClearGroups) * blockDim.x + threadIdx.x; i < n;
+       i += (size_t)(gridDim.x - kClearGroups) * blockDim.x) {
+    const uint32_t p = (uint32_t)(i >> 3), e = (uint32_t)i & 7u;
+    const uint64_t key = V.block_keys[p];
+    if (key == kEmptyKey) continue;
+    const i3 b = unpack_key(key);
+    V.oct[i] = e == 0 ? (int32_t)p
+                      : hash_find_eager(V, i3{b.x + (int)(e >> 2), b.y + (int)((e >> 1) & 1u), b.z + (int)(e & 1u)});
+  }
+}
+template <class Src>
+void launch_ray_prepare(Src src, const SceneFrame* tab, const RayConst& R, uint32_t nscenes, hipStream_t s) {
+  ray_prepare_kernel<<<dim3(kClearGroups + (nscenes > 1 ? 64 : 1024), nscenes), 256, 0, s>>>(src, tab, R);
 }
 
 // The tiles that the part of block `key`'s box a ray can sample projects to,
@@ -1032,7 +1008,7 @@ __global__ __launch_bounds__(256) void ray_range_kernel(Src src_, const SceneFra
 template <class Src>
 void launch_ray_range(Src src, const SceneFrame* tab, const RayConst& R, uint32_t tiles, uint32_t nscenes,
                       hipStream_t s) {
-  ray_range_clear_kernel<<<dim3(8, nscenes), 256, 0, s>>>(src, tab, R);
+  launch_ray_prepare(src, tab, R, nscenes, s);
   if (tiles <= kRangeLdsTiles) {
     ray_range_kernel<Src, true><<<dim3(nscenes > 1 ? 64 : 128, nscenes), 256, 0, s>>>(src, tab, R);
   } else {
@@ -1044,16 +1020,17 @@ void launch_ray_range(Src src, const SceneFrame* tab, const RayConst& R, uint32_
 
 template <class Src>
 void raycast_shaped(Src src, const SceneFrame* tab, const RayConst& p, uint32_t w, uint32_t h, uint32_t nscenes,
-                    int shape, float* depth, float* vertex, float* normal, hipStream_t s) {
+                    bool wide, int shape, float* depth, float* vertex, float* normal, hipStream_t s) {
   const int tw = kRayTileWidths[shape], th = 64 / tw;
+  const int log_tw = __builtin_ctz((unsigned)tw);
   const dim3 grid((w + tw - 1) / tw, (h + th - 1) / th, nscenes);
-  switch (tw) {
-    case 16: raycast_kernel<Src, 16><<<grid, 64, 0, s>>>(src, tab, p, depth, vertex, normal); break;
-    case 4: raycast_kernel<Src, 4><<<grid, 64, 0, s>>>(src, tab, p, depth, vertex, normal); break;
-    case 32: raycast_kernel<Src, 32><<<grid, 64, 0, s>>>(src, tab, p, depth, vertex, normal); break;
-    default: raycast_kernel<Src, 8><<<grid, 64, 0, s>>>(src, tab, p, depth, vertex, normal); break;
-  }
+  if (wide)
+    raycast_kernel<Src, true><<<grid, 64, 0, s>>>(src, tab, p, log_tw, depth, vertex, normal);
+  else
+    raycast_kernel<Src, false><<<grid, 64, 0, s>>>(src, tab, p, log_tw, depth, vertex, normal);
 }
+
+void launch_ray_rows(const View& V, hipStream_t s) { launch_ray_prepare(One{V}, nullptr, RayConst{}, 1, s); }
 
 void launch_ray_range_one(const View& V, const RayConst& p, hipStream_t s) {
   launch_ray_range(One{V}, nullptr, p, p.tiles, 1, s);
@@ -1061,17 +1038,17 @@ void launch_ray_range_one(const View& V, const RayConst& p, hipStream_t s) {
 
 void launch_raycast_march(const View& V, const RayConst& p, float* depth, float* vertex, float* normal,
                           hipStream_t s, int shape) {
-  raycast_shaped(One{V}, nullptr, p, p.cam.width, p.cam.height, 1, shape, depth, vertex, normal, s);
+  raycast_shaped(One{V}, nullptr, p, p.cam.width, p.cam.height, 1, V.capacity > kNarrowCapacity, shape, depth,
+                 vertex, normal, s);
 }
 
 void launch_raycast(const View& V, const RayConst& p, float* depth, float* vertex, float* normal,
                     hipStream_t s, const KernelClock* kc, int shape) {
-  if (p.range) {
-    tick(kc, s, "ray_range_kernel");
-    launch_ray_range(One{V}, nullptr, p, p.tiles, 1, s);
-  }
+  tick(kc, s, "ray_range_kernel");
+  launch_ray_range(One{V}, nullptr, p, p.tiles, 1, s);
   tick(kc, s, "raycast_kernel");
-  raycast_shaped(One{V}, nullptr, p, p.cam.width, p.cam.height, 1, shape, depth, vertex, normal, s);
+  raycast_shaped(One{V}, nullptr, p, p.cam.width, p.cam.height, 1, V.capacity > kNarrowCapacity, shape, depth,
+                 vertex, normal, s);
   tick(kc, s, nullptr);
 }
 
@@ -1097,16 +1074,19 @@ void launch_raycast_backward(const View& V, const RayConst& p, const float* obs,
                              double* partials, double* out, float max_residual, float max_slope,
                              hipStream_t s) {
   dim3 grid((p.cam.width + 7) / 8, (p.cam.height + 7) / 8);
-  if (p.range) launch_ray_range(One{V}, nullptr, p, p.tiles, 1, s);
-  raycast_backward_kernel<<<grid, 64, 0, s>>>(V, p, obs, grad_sdf, partials, max_residual,
-                                              max_slope);
+  launch_ray_range(One{V}, nullptr, p, p.tiles, 1, s);
+  if (V.capacity > kNarrowCapacity)
+    raycast_backward_kernel<true><<<grid, 64, 0, s>>>(V, p, obs, grad_sdf, partials, max_residual, max_slope);
+  else
+    raycast_backward_kernel<false><<<grid, 64, 0, s>>>(V, p, obs, grad_sdf, partials, max_residual, max_slope);
   launch_slot_reduce(partials, grid.x * grid.y, kGradSlots, &V.ctr->reduce_done, out, s);
 }
 
 void launch_batch_raycast(const BatchDev& B, float* depth, float* vertex, float* normal,
                           hipStream_t s, int shape) {
   launch_ray_range(B.src(), B.frames, RayConst{}, ((B.width + 7) / 8) * ((B.height + 7) / 8), B.nscenes, s);
-  raycast_shaped(B.src(), B.frames, RayConst{}, B.width, B.height, B.nscenes, shape, depth, vertex, normal, s);
+  raycast_shaped(B.src(), B.frames, RayConst{}, B.width, B.height, B.nscenes, B.max_capacity > kNarrowCapacity, shape,
+                 depth, vertex, normal, s);
 }
 
 }  // namespace mh
