@@ -150,6 +150,8 @@ struct mh_volume {
   double* pd_energy = nullptr;
   uint32_t pd_npartials = 0;
   uint32_t mc_pass = 0;
+  bool fields_held = false;  // a caller has a pointer to a voxel field (and may write any slot of it)
+  bool reset_all = true;     // the next reset clears the whole pool: new memory, or fields held
   // mesh compaction (allocated on first use)
   uint32_t* cm_used = nullptr;    // per vertex slot: used by a live triangle
   uint32_t* cm_remap = nullptr;   // per vertex slot: compact index
@@ -524,7 +526,8 @@ int mh_volume_destroy(mh_volume* v) {
 
 int mh_volume_reset(mh_volume* v) {
   if (check_vol(v)) return MH_ERR_ARG;
-  launch_reset(v->V, v->stream, v->grid_wg256());
+  launch_reset(v->V, v->reset_all, v->stream, v->grid_wg256());
+  v->reset_all = v->fields_held;
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(v->stream));
   v->have_frame = false;
@@ -684,6 +687,7 @@ int mh_volume_field_device_ptr(mh_volume* v, int field, void** field_dev, uint64
   }
   if (!p) return fail(MH_ERR_STATE, "volume has no PSDF fields");
   *field_dev = p;
+  v->fields_held = v->reset_all = true;
   if (count) *count = (uint64_t)v->hp.value_capacity * kBlockVoxels;
   return MH_OK;
 }

@@ -977,8 +977,10 @@ __global__ __launch_bounds__(256) void mc_push_freed_kernel(Src src_, const Scen
   const View& V = src.view(blockIdx.y);
   // both unchanged until every workgroup of the scene has counted itself done
   const uint32_t n = V.ctr->vfree_count;
-  if (n == 0) return;  // the same for all of the scene's workgroups
   const int32_t top = V.ctr->vertex_top;
+  // no slot went back during the pass: the heap is at its lowest since the last
+  if (blockIdx.x == 0 && threadIdx.x == 0) V.ctr->vertex_low = min(V.ctr->vertex_low, top);
+  if (n == 0) return;  // the same for all of the scene's workgroups
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
     V.vertex_heap[top + 1 + (int32_t)i] = V.vfree[i];
   __syncthreads();

@@ -235,6 +235,7 @@ struct Counters {
   uint32_t cand_count;     // worklist length
   uint32_t ovf_count;      // keys queued for list insertion this frame
   int32_t vertex_top;      // vertex heap counter (mesh.h:53-59)
+  int32_t vertex_low;      // lowest vertex_top a meshing pass ended with
   uint32_t gc_count;       // blocks on the garbage list (RecycleGarbageBlockArray)
   uint32_t flags;          // MH_STATUS_* bits
   uint32_t dropped;

@@ -157,7 +157,8 @@ inline void tick(const KernelClock* c, hipStream_t s, const char* next) {
 }
 
 // mapping.hip
-void launch_reset(const View& V, hipStream_t s, int grid);
+// full: every block and vertex (else those that were ever handed out)
+void launch_reset(const View& V, bool full, hipStream_t s, int grid);
 void launch_convert_depth(const View& V, const uint16_t* raw, hipStream_t s);
 void launch_convert_color(const View& V, const uint8_t* bgra, hipStream_t s);
 void launch_alloc(const View& V, hipStream_t s, const KernelClock* kc = nullptr);
