@@ -1457,7 +1457,7 @@ struct mh_batch {
   int ring = 0;
   uint32_t* d_work = nullptr;
   uint32_t* d_work_count = nullptr;
-  uint32_t* d_dyn = nullptr;       // marching cubes' on-demand item counter
+  uint32_t* d_dyn = nullptr;       // marching cubes' on-demand item counters
   uint16_t* d_raw = nullptr;       // staging for host depth uploads
   uint32_t* d_range = nullptr;     // raycast tile ranges, ray_range_words(W, H) per scene
   int32_t* d_nbt = nullptr;        // marching cubes: 27 neighbours per concatenated-worklist item
@@ -1800,7 +1800,7 @@ int mh_batch_create(uint32_t n_scenes, const mh_hash_params* hash, const mh_volu
   }
   const size_t npix = (size_t)b->W * b->H * n_scenes;
   if (dalloc(&b->d_frames, n_scenes) != hipSuccess || dalloc(&b->d_work, work_cap) != hipSuccess ||
-      dalloc(&b->d_work_count, 1) != hipSuccess || dalloc(&b->d_dyn, 1) != hipSuccess ||
+      dalloc(&b->d_work_count, 1) != hipSuccess || dalloc(&b->d_dyn, kDynGroups * 64) != hipSuccess ||
       dalloc(&b->d_raw, npix) != hipSuccess ||
       dalloc(&b->d_nbt, work_cap * 27) != hipSuccess)
     return bail(fail(MH_ERR_HIP, "device allocation failed"));

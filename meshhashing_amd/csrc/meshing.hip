@@ -6,7 +6,7 @@
 // core/mesh.h:53-107 (vertex/triangle pools and ref counts),
 // visualization/color_util.h:13-37 (ValToRGB).
 //
-// MI355X layout: one 512-lane workgroup per block, one cube per lane.  The
+// MI355X layout: one workgroup per block, two cubes per lane.  The
 // block and its 26 neighbours are staged once as an 11^3 voxel shell in LDS
 // (local coordinates -1..9), which covers every corner, every trilinear
 // sample and every gradient stencil of the block's cubes, so the 8 + 56
@@ -74,13 +74,24 @@ __device__ __forceinline__ const McConst& mc_of(const One&, uint32_t, const McCo
 __device__ __forceinline__ const McConst& mc_of(const Many& m, uint32_t s, const McConst&) {
   return m.f[s].mc;
 }
-constexpr uint32_t kLookupLane = kBlockVoxels - 64;  // the surfel pass's last wave
+// Surfel pass: 256 lanes a workgroup (two voxels a lane).  The next block's
+// shell, cube words and vertex slots are loaded into registers while the
+// current block is worked on, which takes up to 128 registers: four workgroups
+// a CU, each a block at work and one on its way.  Bound by the latency of a
+// block's chain of LDS phases and barriers.  Measured on the replayed 640 x 480,
+// 5 mm frame and a pass over 64 rooms (76 k blocks): 358 us and 2.87 ms so,
+// 412 us and 3.35 ms with 512 lanes and two workgroups a CU, 466 us and 3.57 ms
+// with 512 lanes, three workgroups and 80 registers (spills).
+constexpr uint32_t kMcLanes = 256;
+constexpr int kMcVox = kBlockVoxels / kMcLanes;
+constexpr uint32_t kLookupLane = kMcLanes - 64;  // its last wave
 // The surfel pass hands out its first items statically (workgroup g takes
 // g, g + grid, ...) and the rest on demand from a counter, so workgroups
 // whose blocks held little surface take more of them.  static_q quarters of
 // the worklist (rounded down to whole rounds of the grid, at least one) are
-// static; the counter (cleared by the neighbour-table pass) counts the items
-// handed out after them.
+// static.  The rest goes by kDynGroups counters (cleared by the neighbour-table
+// pass), workgroup g taking every kDynGroups-th item from the one of its group:
+// on one counter, workgroups that ask at the same time wait for each other.
 __device__ __forceinline__ uint32_t mc_static_items(uint32_t n, uint32_t grid, uint32_t static_q) {
   const uint32_t k = (static_q * n / 4u) / grid;
   return (k ? k : 1u) * grid;
@@ -91,8 +102,8 @@ __global__ __launch_bounds__(256) void mc_neighbours_kernel(Src src_, const Scen
                                                              McConst mc1, int32_t* __restrict__ nbt) {
   const Src src = with_table(src_, tab);
   const uint32_t total = src.count() * 27u;
-  // the surfel pass's counter of items handed out on demand (it runs next)
-  if (blockIdx.x == 0 && threadIdx.x == 0) *src.next_ctr() = 0u;
+  // the surfel pass's counters of items handed out on demand (it runs next)
+  if (blockIdx.x == 0 && threadIdx.x < kDynGroups) src.next_ctr()[64 * threadIdx.x] = 0u;
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < total; i += gridDim.x * blockDim.x) {
     const uint32_t ci = i / 27u, t = i % 27u;
     uint32_t scene;
@@ -107,67 +118,100 @@ __global__ __launch_bounds__(256) void mc_neighbours_kernel(Src src_, const Scen
   }
 }
 
-// nbe: the lane's neighbour-table entry for this block (lanes
-// kLookupLane + t, t < 27).
+// What a lane holds of a block on its way: its share of the shell, its two
+// voxels' cube words and vertex slots.
+constexpr int kShellPer = (kShellN + (int)kMcLanes - 1) / (int)kMcLanes;
 template <bool PSDF>
-__device__ void stage_shell(const View& V, const McConst& mc, int32_t nbe, Shell<PSDF>& S, int32_t* nb,
-                            uint8_t* meshed) {
-  const uint32_t t = threadIdx.x - kLookupLane;
-  if (t < 27) {
-    nb[t] = nbe < 0 ? nbe : (nbe & (kMeshedBit - 1));
-    meshed[t] = nbe >= 0 && (nbe & kMeshedBit) != 0;
-  }
-  __syncthreads();
-  // All of a lane's loads are issued before any is stored to LDS (one
-  // memory round trip for the shell), for a 512-lane workgroup.
-  constexpr int kPer = (kShellN + 511) / 512;
-  float sd[kPer], wt[kPer], va[kPer], vb[kPer];
-  bool ok[kPer];
+struct BlockRegs {
+  float sd[kShellPer], wt[kShellPer], va[PSDF ? kShellPer : 1], vb[PSDF ? kShellPer : 1];
+  bool ok[kShellPer];
+  int32_t vps[kMcVox][3];
+  uint32_t word[kMcVox];
+};
+// Where shell voxel s lies: neighbour | local voxel << 5 | kCodeInner if it is a
+// corner of a cube at local -1..7 (its coordinates are at most 8).
+constexpr uint32_t kCodeInner = 1u << 14;
+__device__ __forceinline__ uint32_t shell_code(int s) {
+  const int lx = s % kShell - 1, ly = (s / kShell) % kShell - 1, lz = s / (kShell * kShell) - 1;
+  const int dx = lx < 0 ? -1 : (lx >= 8 ? 1 : 0), dy = ly < 0 ? -1 : (ly >= 8 ? 1 : 0),
+            dz = lz < 0 ? -1 : (lz >= 8 ? 1 : 0);
+  return (uint32_t)nb27(dx, dy, dz) | ((uint32_t)((lx - 8 * dx) + 8 * (ly - 8 * dy) + 64 * (lz - 8 * dz)) << 5) |
+         (lx <= 8 && ly <= 8 && lz <= 8 ? kCodeInner : 0u);
+}
+// A row entry's pool index (negative: absent) and mark.
+__device__ __forceinline__ int32_t row_ptr(int32_t e) { return e < 0 ? e : (e & (kMeshedBit - 1)); }
+__device__ __forceinline__ bool row_meshed(int32_t e) { return e >= 0 && (e & kMeshedBit) != 0; }
+
+// Issues the loads of block ptr (row: its neighbours, code: shell_code's table).
+template <bool PSDF>
+__device__ __forceinline__ void load_block(const View& V, int32_t ptr, const int32_t* row, const uint16_t* code,
+                                           BlockRegs<PSDF>& R) {
 #pragma unroll
-  for (int r = 0; r < kPer; ++r) {
-    const int s = (int)threadIdx.x + 512 * r;
-    ok[r] = false;
-    sd[r] = wt[r] = va[r] = vb[r] = 0.0f;
+  for (int r = 0; r < kShellPer; ++r) {
+    const int s = (int)(threadIdx.x + kMcLanes * r);
+    R.ok[r] = false;
+    R.sd[r] = R.wt[r] = 0.0f;
+    if (PSDF) R.va[r] = R.vb[r] = 0.0f;
     if (s >= kShellN) continue;
-    const int lx = s % kShell - 1, ly = (s / kShell) % kShell - 1, lz = s / (kShell * kShell) - 1;
-    const int dx = lx < 0 ? -1 : (lx >= 8 ? 1 : 0);
-    const int dy = ly < 0 ? -1 : (ly >= 8 ? 1 : 0);
-    const int dz = lz < 0 ? -1 : (lz >= 8 ? 1 : 0);
-    const int32_t p = nb[nb27(dx, dy, dz)];
+    const uint32_t c = code[s];
+    const int32_t p = row_ptr(row[c & 31u]);
     if (p < 0) continue;
-    const size_t idx = (size_t)p * kBlockVoxels + (size_t)((lx - 8 * dx) + 8 * (ly - 8 * dy) +
-                                                           64 * (lz - 8 * dz));
-    ok[r] = true;
-    sd[r] = V.sdf[idx];
-    wt[r] = V.weight[idx];
+    const size_t idx = (size_t)p * kBlockVoxels + ((c >> 5) & 511u);
+    R.ok[r] = true;
+    R.sd[r] = V.sdf[idx];
+    R.wt[r] = V.weight[idx];
     if (PSDF) {
-      va[r] = V.va[idx];
-      vb[r] = V.vb[idx];
+      R.va[r] = V.va[idx];
+      R.vb[r] = V.vb[idx];
     }
   }
 #pragma unroll
-  for (int r = 0; r < kPer; ++r) {
-    const int s = (int)threadIdx.x + 512 * r;
+  for (int r = 0; r < kMcVox; ++r) {
+    const size_t idx = (size_t)ptr * kBlockVoxels + threadIdx.x + kMcLanes * r;
+    R.word[r] = V.cube[idx];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) R.vps[r][a] = V.vptr[3 * idx + a];
+  }
+}
+
+// Puts the lane's share of the shell into LDS.  Returns whether the block may
+// hold a vertex or a triangle after this pass, or holds a vertex slot now, as
+// far as this lane can see: a negative voxel around its own and its lower
+// neighbours' cubes (local -1..8), a slot, or a lower neighbour that is not
+// meshed in this pass (its stored configurations count then).  A block of
+// which no lane says so is done: its cubes are all 0 and it has no surfels.
+template <bool PSDF>
+__device__ __forceinline__ bool stage_shell(const McConst& mc, const BlockRegs<PSDF>& R, const int32_t* row,
+                                            const uint16_t* code, Shell<PSDF>& S) {
+  const uint32_t t = threadIdx.x - kLookupLane;
+  bool keep = false;
+  if (t < 27 && t % 3 < 2 && (t / 3) % 3 < 2 && t / 9 < 2) keep = row[t] >= 0 && !row_meshed(row[t]);
+#pragma unroll
+  for (int r = 0; r < kShellPer; ++r) {
+    const int s = (int)(threadIdx.x + kMcLanes * r);
     if (s >= kShellN) continue;
     // the corner tests of IsValid (marching_cubes.cu:96-130), once per
     // voxel here instead of once per cube corner
-    const float rho = PSDF ? va[r] / (va[r] + vb[r]) : 0.0f;
-    const bool cube_ok = ok[r] && !(fabsf(sd[r]) > mc.sdf_threshold) && (!PSDF || !(rho < mc.rho_min)) &&
-                         !(wt[r] < mc.weight_min);
-    S.f[s] = (uint8_t)((ok[r] ? kShOk : 0) | (cube_ok ? kShCube : 0) | (sd[r] < 0.0f ? kShNeg : 0));
-    S.sdf[s] = sd[r];
-    S.w[s] = wt[r];
+    const float sd = R.sd[r], wt = R.wt[r];
+    const float rho = PSDF ? R.va[r] / (R.va[r] + R.vb[r]) : 0.0f;
+    const bool cube_ok = R.ok[r] && !(fabsf(sd) > mc.sdf_threshold) && (!PSDF || !(rho < mc.rho_min)) &&
+                         !(wt < mc.weight_min);
+    S.f[s] = (uint8_t)((R.ok[r] ? kShOk : 0) | (cube_ok ? kShCube : 0) | (sd < 0.0f ? kShNeg : 0));
+    S.sdf[s] = sd;
+    S.w[s] = wt;
     if (PSDF) {
-      S.a[s] = va[r];
-      S.b[s] = vb[r];
+      S.a[s] = R.va[r];
+      S.b[s] = R.vb[r];
     }
+    keep = keep || (sd < 0.0f && (code[s] & kCodeInner));
   }
-  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kMcVox; ++r) keep = keep || R.vps[r][0] >= 0 || R.vps[r][1] >= 0 || R.vps[r][2] >= 0;
+  return keep;
 }
 
-
 struct SVal {
-  float sdf, a, b, radius;
+  float sdf, a, b;
 };
 
 // One axis of a GetSpatialValue sample (spatial_query.h:23-66) at world
@@ -180,16 +224,17 @@ struct SAxis {
   int c0, c1;
   float r;
 };
-__device__ __forceinline__ SAxis shell_axis(float p, float vs, int base) {
+__device__ __forceinline__ SAxis shell_axis(float p, float vs, float inv_vs, int base) {
   const float pc = p - 0.5f * vs;
-  const float q = p / vs;
-  return SAxis{vox1(pc + 0.0f, vs) - base, vox1(pc + vs, vs) - base, q - floorf(q)};
+  const float q = quotient(p, vs, inv_vs);
+  return SAxis{vox1_quot(pc + 0.0f, vs, inv_vs) - base, vox1_quot(pc + vs, vs, inv_vs) - base, q - floorf(q)};
 }
 
-// GetSpatialValue against the staged shell, from the sample's three axes.
-template <bool PSDF, bool FULL = true>
+// GetSpatialValue against the staged shell, from the sample's three axes (full:
+// the Beta parameters too).
+template <bool PSDF>
 __device__ __forceinline__ bool shell_value(const Shell<PSDF>& S, const SAxis& X, const SAxis& Y,
-                                            const SAxis& Z, SVal* out, bool* oob) {
+                                            const SAxis& Z, bool full, SVal* out, bool* oob) {
   const int cx[2] = {X.c0, X.c1}, cy[2] = {Y.c0, Y.c1}, cz[2] = {Z.c0, Z.c1};
   const float rx = X.r, ry = Y.r, rz = Z.r;
   // Straight-line evaluation of all 8 corners (no early exit: a missing
@@ -201,7 +246,7 @@ __device__ __forceinline__ bool shell_value(const Shell<PSDF>& S, const SAxis& X
     return false;
   }
   bool ok = true;
-  float sdf = 0.0f, a = 0.0f, b = 0.0f, rad = 0.0f;
+  float sdf = 0.0f;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const int mx = (i >> 2) & 1, my = (i >> 1) & 1, mz = i & 1;
@@ -209,18 +254,22 @@ __device__ __forceinline__ bool shell_value(const Shell<PSDF>& S, const SAxis& X
     ok = ok && (S.f[s] & kShOk);
     const float w = (mx ? rx : 1.0f - rx) * (my ? ry : 1.0f - ry) * (mz ? rz : 1.0f - rz);
     sdf += w * S.sdf[s];
-    if (FULL) {
-      if (PSDF) {
-        a += w * S.a[s];
-        b += w * S.b[s];
-      }
-      rad += w * sqrtf(1.0f / S.w[s]);
-    }
   }
   out->sdf = sdf;
-  out->a = a;
-  out->b = b;
-  out->radius = rad;
+  out->a = out->b = 0.0f;
+  if (PSDF && full) {
+    float a = 0.0f, b = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int mx = (i >> 2) & 1, my = (i >> 1) & 1, mz = i & 1;
+      const int s = sidx(cx[mx], cy[my], cz[mz]);
+      const float w = (mx ? rx : 1.0f - rx) * (my ? ry : 1.0f - ry) * (mz ? rz : 1.0f - rz);
+      a += w * S.a[s];
+      b += w * S.b[s];
+    }
+    out->a = a;
+    out->b = b;
+  }
   return ok;
 }
 
@@ -246,62 +295,6 @@ __device__ __forceinline__ f3 val_to_rgb(float v, float vmin, float vmax) {
     c.z = 0.0f;
   }
   return c;
-}
-
-// AllocateVertexWithMutex's payload (marching_cubes.cu:45-72).
-template <bool PSDF>
-__device__ void vertex_payload(const Shell<PSDF>& S, const Geo& g, i3 base, f3 p, Vertex* vt,
-                               bool* oob) {
-  SVal sv{};
-  const float vs = g.voxel_size;
-  const SAxis X = shell_axis(p.x, vs, base.x), Y = shell_axis(p.y, vs, base.y), Z = shell_axis(p.z, vs, base.z);
-  const bool ok = shell_value(S, X, Y, Z, &sv, oob);
-  vt->px = p.x;
-  vt->py = p.y;
-  vt->pz = p.z;
-  if (ok) {
-    const float inv_sigma2 = 1.0f / (sv.radius * sv.radius);
-    vt->radius = sqrtf(1.0f / inv_sigma2);
-    const f3 c = val_to_rgb(sv.a / (sv.a + sv.b), 0.4f, 1.0f);
-    vt->cr = c.x;
-    vt->cg = c.y;
-    vt->cb = c.z;
-  } else {  // the reference reads an uninitialised query here
-    vt->radius = 0.0f;
-    vt->cr = vt->cg = vt->cb = 0.0f;
-  }
-  // GetSpatialSDFGradient (spatial_query.h:68-97): central differences at
-  // +-vs/2, with the reference's short-circuit on the first invalid sample.
-  // (all six samples are taken; any invalid one zeroes the normal, which is
-  // what the reference's short-circuit produces)
-  // (p -+ h e_k differs from p on axis k only: the other two axes are the
-  // centre sample's)
-  const float h = 0.5f * g.voxel_size;
-  bool valid = true;
-  float g0 = 0.0f, g1 = 0.0f, g2 = 0.0f;  // (sp[k] - sn[k]) / vs per axis, without an indexed array
-  // not unrolled: the six stencils' live registers would cost mc_surfel_kernel
-  // a workgroup per CU
-#pragma unroll 1
-  for (int k = 0; k < 3; ++k) {
-    const float pk = k == 0 ? p.x : (k == 1 ? p.y : p.z);
-    const int bk = k == 0 ? base.x : (k == 1 ? base.y : base.z);
-    SVal q{};
-    const SAxis An = shell_axis(pk - h, vs, bk);
-    valid = shell_value<PSDF, false>(S, k == 0 ? An : X, k == 1 ? An : Y, k == 2 ? An : Z, &q, oob) && valid;
-    const float sn = q.sdf;
-    const SAxis Ap = shell_axis(pk + h, vs, bk);
-    valid = shell_value<PSDF, false>(S, k == 0 ? Ap : X, k == 1 ? Ap : Y, k == 2 ? Ap : Z, &q, oob) && valid;
-    const float gk = (q.sdf - sn) / vs;
-    g0 = k == 0 ? gk : g0;
-    g1 = k == 1 ? gk : g1;
-    g2 = k == 2 ? gk : g2;
-  }
-  const f3 grad = mk3(g0, g1, g2);
-  const float l = length(grad);
-  const f3 n = (l > 0.0f && valid) ? grad / l : mk3(0.0f, 0.0f, 0.0f);
-  vt->nx = n.x;
-  vt->ny = n.y;
-  vt->nz = n.z;
 }
 
 // ---------------------------------------------------------------- pass 1
@@ -331,26 +324,40 @@ __device__ __forceinline__ int cidx(int x, int y, int z) {
   return (x + 1) + kCubeHalo * (y + 1) + kCubeHalo * kCubeHalo * (z + 1);
 }
 
+// The surfel pass queues a block's vertex writes in LDS (a block with surface
+// writes ~80): a round of slot claims adds at most one per lane, and the queue
+// is worked off when another round might not fit.
+constexpr uint32_t kQueue = 2 * kMcLanes;
+
 // Payload of vertex (owner voxel at local (key & 15, key >> 4 & 15,
 // key >> 8 & 15), axis key >> 12) into vertex record vp: VertexIntersection
 // (marching_cubes.cu:16-28) in the canonical endpoint order, then
-// AllocateVertexWithMutex's payload (:45-72).
-// The surfel pass queues a block's vertex writes in LDS (a block writes ~40
-// on average); past kQueue the lane writes its vertex itself.
-constexpr uint32_t kQueue = 1024;
+// AllocateVertexWithMutex's payload (:45-72), spread over eight lanes per
+// vertex, so that a vertex costs the latency of one trilinear sample instead of
+// seven in a row: lanes 0-5 take the gradient stencils p -+ h e_k (k = sub / 2;
+// odd: +h), lane 6 the full sample at p (radius, colour); each lane samples
+// one point, the stencils sharing all but one coordinate with p (p -+ 0 = p).
+// The eight corner radii of lane 6's cell are taken one per lane.  Stencil
+// values, validities and corner radii meet in LDS (pay_s, pay_ok, pay_r, the
+// vertex's row), from which lanes 0 and 6 finish the record after the
+// workgroup barrier (finish_normal, finish_sample).
+struct PaySample {  // lane 6's sample
+  float rx, ry, rz, a, b;
+  bool ok;
+};
 template <bool PSDF>
-// Returns true when a stencil sample fell outside the staged shell.
-__device__ __forceinline__ bool write_vertex(const Shell<PSDF>& S, const View& V, const McConst& mc, i3 base,
-                             uint32_t key, int32_t vp) {
+__device__ __forceinline__ bool payload_part(const Shell<PSDF>& S, const View& V, const McConst& mc, float inv_vs,
+                                             i3 base, uint32_t key, int32_t vp, uint32_t sub, float* pay_s,
+                                             float* pay_r, uint8_t* pay_ok, PaySample* out) {
   bool oob = false;
   const Geo& g = V.geo;
+  const float vs = g.voxel_size;
   const int ox = (int)(key & 15u), oy = (int)((key >> 4) & 15u), oz = (int)((key >> 8) & 15u);
   const int ax = (int)(key >> 12);
   const float vA = S.sdf[sidx(ox, oy, oz)];
   const float vB = S.sdf[sidx(ox + (ax == 0), oy + (ax == 1), oz + (ax == 2))];
   const f3 pA = voxel_to_world(g, i3{base.x + ox, base.y + oy, base.z + oz});
-  const f3 pB = mk3(pA.x + (ax == 0 ? g.voxel_size : 0.0f), pA.y + (ax == 1 ? g.voxel_size : 0.0f),
-                    pA.z + (ax == 2 ? g.voxel_size : 0.0f));
+  const f3 pB = mk3(pA.x + (ax == 0 ? vs : 0.0f), pA.y + (ax == 1 ? vs : 0.0f), pA.z + (ax == 2 ? vs : 0.0f));
   f3 p;
   if ((double)fabsf(vA) < mc.snap) {
     p = pA;
@@ -360,80 +367,57 @@ __device__ __forceinline__ bool write_vertex(const Shell<PSDF>& S, const View& V
     const float mu = (0.0f - vA) / (vB - vA);
     p = mk3(pA.x + mu * (pB.x - pA.x), pA.y + mu * (pB.y - pA.y), pA.z + mu * (pB.z - pA.z));
   }
-  Vertex vt;
-  vertex_payload<PSDF>(S, g, base, p, &vt, &oob);
-  Vertex* dst = &V.vertices[vp];
-  *reinterpret_cast<float4*>(&dst->px) = make_float4(vt.px, vt.py, vt.pz, vt.radius);
-  dst->nx = vt.nx;
-  dst->ny = vt.ny;
-  dst->nz = vt.nz;
-  dst->cr = vt.cr;
-  dst->cg = vt.cg;
-  dst->cb = vt.cb;
+  if (sub == 6) {
+    V.vertices[vp].px = p.x;
+    V.vertices[vp].py = p.y;
+    V.vertices[vp].pz = p.z;
+  }
+  const float h = 0.5f * vs;
+  const float d = (sub & 1u) ? h : -h;
+  const uint32_t k = sub >> 1;
+  const SAxis X = shell_axis(k == 0 ? p.x + d : p.x, vs, inv_vs, base.x);
+  const SAxis Y = shell_axis(k == 1 ? p.y + d : p.y, vs, inv_vs, base.y);
+  const SAxis Z = shell_axis(k == 2 ? p.z + d : p.z, vs, inv_vs, base.z);
+  SVal q{};
+  // lanes 6 and 7 (k = 3) sample p itself, lane 7 for nothing
+  const bool ok = shell_value<PSDF>(S, X, Y, Z, sub == 6, &q, &oob);
+  pay_s[sub] = q.sdf;
+  pay_ok[sub] = ok ? 1 : 0;
+  // lane 6's cell, corner coordinates + 1 in 4 bits each (valid: all in 0..10)
+  const uint32_t cell = (uint32_t)(X.c0 + 1) | ((uint32_t)(X.c1 + 1) << 4) | ((uint32_t)(Y.c0 + 1) << 8) |
+                        ((uint32_t)(Y.c1 + 1) << 12) | ((uint32_t)(Z.c0 + 1) << 16) | ((uint32_t)(Z.c1 + 1) << 20);
+  const uint32_t c6 = (uint32_t)__shfl((int)(ok ? cell : ~0u), 6, 8);
+  if (c6 != ~0u) {
+    const uint32_t cx = (c6 >> ((sub & 4u) ? 4 : 0)) & 15u, cy = (c6 >> ((sub & 2u) ? 12 : 8)) & 15u,
+                   cz = (c6 >> ((sub & 1u) ? 20 : 16)) & 15u;
+    pay_r[sub] = sqrtf(1.0f / S.w[cx + kShell * cy + kShell * kShell * cz]);
+  }
+  *out = PaySample{X.r, Y.r, Z.r, q.a, q.b, ok};
   return oob;
 }
 
-// The same payload spread over eight lanes per vertex, so that a vertex
-// costs the latency of one trilinear sample instead of seven in a row: lanes
-// 0-5 take the gradient stencils p -+ h e_k (k = sub / 2; odd: +h), lane 6
-// the full sample at p (radius, colour) and stores position, radius and
-// colour; lane 7 is idle.  Stencil values and validities meet in LDS
-// (pay_s, pay_ok, row jl), from which lane 0 finishes the normal after the
-// workgroup barrier (finish_normal).  Every sample is write_vertex's, with
-// the same axes and arithmetic, so the stored bits are the same.
-template <bool PSDF>
-__device__ __forceinline__ bool payload_part(const Shell<PSDF>& S, const View& V, const McConst& mc,
-                                             i3 base, uint32_t key, int32_t vp, uint32_t sub,
-                                             float* pay_s, uint8_t* pay_ok) {
-  bool oob = false;
-  const Geo& g = V.geo;
-  const int ox = (int)(key & 15u), oy = (int)((key >> 4) & 15u), oz = (int)((key >> 8) & 15u);
-  const int ax = (int)(key >> 12);
-  const float vA = S.sdf[sidx(ox, oy, oz)];
-  const float vB = S.sdf[sidx(ox + (ax == 0), oy + (ax == 1), oz + (ax == 2))];
-  const f3 pA = voxel_to_world(g, i3{base.x + ox, base.y + oy, base.z + oz});
-  const f3 pB = mk3(pA.x + (ax == 0 ? g.voxel_size : 0.0f), pA.y + (ax == 1 ? g.voxel_size : 0.0f),
-                    pA.z + (ax == 2 ? g.voxel_size : 0.0f));
-  f3 p;
-  if ((double)fabsf(vA) < mc.snap) {
-    p = pA;
-  } else if ((double)fabsf(vB) < mc.snap) {
-    p = pB;
-  } else {
-    const float mu = (0.0f - vA) / (vB - vA);
-    p = mk3(pA.x + mu * (pB.x - pA.x), pA.y + mu * (pB.y - pA.y), pA.z + mu * (pB.z - pA.z));
-  }
-  const float vs = g.voxel_size;
-  const SAxis X = shell_axis(p.x, vs, base.x), Y = shell_axis(p.y, vs, base.y), Z = shell_axis(p.z, vs, base.z);
-  if (sub < 6) {
-    const int k = (int)(sub >> 1);
-    const float pk = k == 0 ? p.x : (k == 1 ? p.y : p.z);
-    const int bk = k == 0 ? base.x : (k == 1 ? base.y : base.z);
-    const float h = 0.5f * g.voxel_size;
-    const SAxis An = shell_axis((sub & 1u) ? pk + h : pk - h, vs, bk);
-    SVal q{};
-    const bool ok = shell_value<PSDF, false>(S, k == 0 ? An : X, k == 1 ? An : Y, k == 2 ? An : Z, &q, &oob);
-    pay_s[sub] = q.sdf;
-    pay_ok[sub] = ok ? 1 : 0;
-  } else if (sub == 6) {
-    SVal sv{};
-    const bool ok = shell_value(S, X, Y, Z, &sv, &oob);
-    Vertex* dst = &V.vertices[vp];
-    float radius = 0.0f, cr = 0.0f, cg = 0.0f, cb = 0.0f;  // the reference reads an uninitialised query
-    if (ok) {
-      const float inv_sigma2 = 1.0f / (sv.radius * sv.radius);
-      radius = sqrtf(1.0f / inv_sigma2);
-      const f3 c = val_to_rgb(sv.a / (sv.a + sv.b), 0.4f, 1.0f);
-      cr = c.x;
-      cg = c.y;
-      cb = c.z;
+// Lane 6's part of the record after the exchange: radius and colour.
+__device__ __forceinline__ void finish_sample(const View& V, int32_t vp, const PaySample& q, const float* pay_r) {
+  float radius = 0.0f, cr = 0.0f, cg = 0.0f, cb = 0.0f;  // the reference reads an uninitialised query here
+  if (q.ok) {
+    float rad = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float w = ((i & 4) ? q.rx : 1.0f - q.rx) * ((i & 2) ? q.ry : 1.0f - q.ry) * ((i & 1) ? q.rz : 1.0f - q.rz);
+      rad += w * pay_r[i];
     }
-    *reinterpret_cast<float4*>(&dst->px) = make_float4(p.x, p.y, p.z, radius);
-    dst->cr = cr;
-    dst->cg = cg;
-    dst->cb = cb;
+    const float inv_sigma2 = 1.0f / (rad * rad);
+    radius = sqrtf(1.0f / inv_sigma2);
+    const f3 c = val_to_rgb(q.a / (q.a + q.b), 0.4f, 1.0f);
+    cr = c.x;
+    cg = c.y;
+    cb = c.z;
   }
-  return oob;
+  Vertex* dst = &V.vertices[vp];
+  dst->radius = radius;
+  dst->cr = cr;
+  dst->cg = cg;
+  dst->cb = cb;
 }
 
 // GetSpatialSDFGradient's normal from the six stencil values of a vertex
@@ -462,21 +446,17 @@ __device__ __forceinline__ void finish_normal(const View& V, int32_t vp, const f
 // no atomics are needed; the other cubes only make sure the vertex slot is
 // allocated.  Any writer would store the same bits (canonical vertices).
 
-// Work counters of one scene, flushed per wave.
+// Work counts of a workgroup, kept by its first lane and added to the scene's
+// counters when the scene changes.
 struct McCounts {
   uint32_t writes = 0, assigned = 0, blocks = 0;
   int delta = 0;
-  bool oob = false;
   __device__ void flush(const View& V) {
-    if (__any(oob)) {
-      if ((threadIdx.x & 63u) == 0) flag(V, MH_STATUS_STENCIL_RANGE);
-    }
-    wave_add_u64(&work_stripe(V.ctr).mc_vertex_writes, writes);
-    wave_add_u64(&work_stripe(V.ctr).mc_triangle_writes, assigned);
-    wave_add_u64(&work_stripe(V.ctr).mc_blocks, blocks);
-    for (int off = 32; off > 0; off >>= 1) delta += __shfl_xor(delta, off);
-    if ((threadIdx.x & 63u) == 0 && delta)
-      atomicAdd(&work_stripe(V.ctr).tri_live, (unsigned long long)(long long)delta);
+    WorkStripe& w = work_stripe(V.ctr);
+    if (writes) atomicAdd(&w.mc_vertex_writes, (unsigned long long)writes);
+    if (assigned) atomicAdd(&w.mc_triangle_writes, (unsigned long long)assigned);
+    if (blocks) atomicAdd(&w.mc_blocks, (unsigned long long)blocks);
+    if (delta) atomicAdd(&w.tri_live, (unsigned long long)(long long)delta);
     *this = McCounts{};
   }
 };
@@ -531,110 +511,195 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* wave_s
 __device__ __forceinline__ int32_t* edge_slot(const View& V, const int32_t* nb, i3 o, int e) {
   const int ox = o.x + edge_owner_off(e, 0), oy = o.y + edge_owner_off(e, 1), oz = o.z + edge_owner_off(e, 2);
   const int dx = ox >> 3, dy = oy >> 3, dz = oz >> 3;
-  const int32_t optr = nb[nb27(dx, dy, dz)];
+  const int32_t optr = row_ptr(nb[nb27(dx, dy, dz)]);
   const uint32_t oi = (uint32_t)((ox - 8 * dx) + 8 * (oy - 8 * dy) + 64 * (oz - 8 * dz));
   return &V.vptr[((size_t)optr * kBlockVoxels + oi) * 3 + edge_axis(e)];
 }
 
 template <bool PSDF, class Src>
-__global__ __launch_bounds__(512, 6) void mc_surfel_kernel(Src src_, const SceneFrame* __restrict__ tab, McConst mc1,
-                                                           const int32_t* __restrict__ nbt, uint32_t static_q) {
+__global__ __launch_bounds__(kMcLanes, PSDF ? 3 : 4) void mc_surfel_kernel(Src src_, const SceneFrame* __restrict__ tab, McConst mc1,
+                                                                const int32_t* __restrict__ nbt, uint32_t static_q) {
   const Src src = with_table(src_, tab);
   __shared__ Shell<PSDF> S;
-  __shared__ int32_t nb[27];
-  __shared__ uint8_t meshed[27];
+  __shared__ uint16_t code[kShellN];
+  __shared__ int32_t row_[2][27];  // the neighbour-table rows of the block at work and of the next one
   __shared__ uint8_t cv[kCubeHalo * kCubeHalo * kCubeHalo];
-  __shared__ uint8_t own_cube[kBlockVoxels];
   __shared__ int surfels[2];
+  __shared__ int tri_sum[2];  // the block's change of live triangles, and the triangles of its changed cubes
+  // Flags of a block, three in turn: a block without surface ends without a
+  // further barrier, so a fast wave may set the next block's while a slow one
+  // still reads this one's; after a block's first barrier every wave is done
+  // with the one before it, whose flags are then cleared for the one after next.
+  __shared__ uint32_t busy_[3][2];
+  __shared__ uint32_t next_[2];
   __shared__ uint32_t free_base;
   __shared__ int32_t qptr[kQueue];
   __shared__ uint16_t qkey[kQueue];
   __shared__ uint32_t qn;
   __shared__ uint32_t scan_wave[8];
   __shared__ int32_t pop_top;
-  // One LDS region, three uses that never overlap in time: the
-  // configurations of the cubes at local -1..7 (this block and its lower
-  // neighbours) from the halo loop to the recycling test; the item list from
-  // the item scan to the end of the slot claims; the payload exchange (eight
-  // lanes per vertex, kPayRound vertices a round) in the payload rounds.
-  // Barriers separate each use from the next.
-  constexpr uint32_t kPayRound = kLookupLane / 8;
+  // One LDS region, two uses that never overlap in time: the configurations
+  // of the cubes at local -1..7 (this block and its lower neighbours) from the
+  // halo loop to the recycling test; the item list from the item scan to the
+  // end of the slot claims.  Barriers separate the uses.
   __shared__ uint32_t region[6 * kBlockVoxels];
   uint16_t* const items = reinterpret_cast<uint16_t*>(region);  // up to 12 per cube
   uint8_t* const hcfg = reinterpret_cast<uint8_t*>(region);
-  float* const pay_s = reinterpret_cast<float*>(region);
-  uint8_t* const pay_ok = reinterpret_cast<uint8_t*>(region + kPayRound * 8);
-  static_assert(kCfg * kCfg * kCfg <= 4 * 6 * kBlockVoxels && kPayRound * 8 * 5 <= 4 * 6 * kBlockVoxels, "region");
+  static_assert(sizeof(region) >= 12 * kBlockVoxels * sizeof(uint16_t) && sizeof(region) >= kCfg * kCfg * kCfg, "region");
+  // the payload exchange (eight lanes per vertex, kPayRound vertices a round)
+  constexpr uint32_t kPayRound = kMcLanes / 8;
+  __shared__ float pay_s[kPayRound * 8], pay_r[kPayRound * 8];
+  __shared__ uint8_t pay_ok[kPayRound * 8];
   __shared__ uint32_t nitems;
   // per-configuration crossed edges and triangle counts, read per lane with
   // divergent indices: from LDS rather than the constant tables
   __shared__ uint16_t etab[256];
   __shared__ uint8_t ntab[256];
-  if (threadIdx.x < 256) {
-    etab[threadIdx.x] = kMc.edges[threadIdx.x];
-    ntab[threadIdx.x] = (uint8_t)kMc.ntri[threadIdx.x];
-  }
   const uint32_t n = src.count();
+  if (blockIdx.x >= n) return;
+  for (uint32_t k = threadIdx.x; k < 256u; k += kMcLanes) {
+    etab[k] = kMc.edges[k];
+    ntab[k] = (uint8_t)kMc.ntri[k];
+  }
+  for (int s = (int)threadIdx.x; s < kShellN; s += (int)kMcLanes) code[s] = (uint16_t)shell_code(s);
   McCounts cnt;
   uint32_t cur_scene = ~0u;
-  // lanes kLookupLane + t hold neighbour t's table entry of the next block
+  // items: ci at work, nx next (its loads under way), the one after it in
+  // next_; lanes kLookupLane + t hold neighbour t's table entry of item nx
   const uint32_t nb_lane = threadIdx.x - kLookupLane;
-  int32_t nbe = kFreePtr;
-  if (nb_lane < 27 && blockIdx.x < n) nbe = nbt[(size_t)blockIdx.x * 27u + nb_lane];
   const uint32_t n_static = mc_static_items(n, gridDim.x, static_q);
-  __shared__ uint32_t s_next;
-  for (uint32_t ci = blockIdx.x; ci < n;) {
-    // the next item, read by every lane after the shell's barriers and
-    // rewritten only after the next barrier
-    if (threadIdx.x == 0)
-      s_next = ci + gridDim.x < n_static ? ci + gridDim.x : n_static + atomicAdd(src.next_ctr(), 1u);
-    uint32_t scene;
-    const int32_t ptr = src.item(ci, &scene);
+  auto item_after = [&](uint32_t c) -> uint32_t {
+    if (c + gridDim.x < n_static) return c + gridDim.x;
+    if (n_static >= n) return n;
+    const uint32_t groups = min(kDynGroups, gridDim.x), group = blockIdx.x % groups;
+    return n_static + groups * atomicAdd(src.next_ctr() + 64 * group, 1u) + group;
+  };
+  uint32_t ci = blockIdx.x;
+  if (threadIdx.x == 0) {
+    next_[1] = item_after(ci);
+    for (int k = 0; k < 3; ++k) busy_[k][0] = busy_[k][1] = 0u;
+  }
+  if (nb_lane < 27) row_[0][nb_lane] = nbt[(size_t)ci * 27u + nb_lane];
+  __syncthreads();
+  uint32_t nx = next_[1];
+  int32_t nbe = nb_lane < 27 && nx < n ? nbt[(size_t)nx * 27u + nb_lane] : kFreePtr;
+  uint32_t scene, scene_n = 0;
+  int32_t ptr = src.item(ci, &scene), ptr_n = 0;
+  uint64_t key = src.view(scene).block_keys[ptr], key_n = 0;
+  if (nx < n) {
+    ptr_n = src.item(nx, &scene_n);
+    key_n = src.view(scene_n).block_keys[ptr_n];
+  }
+  BlockRegs<PSDF> R;
+  load_block<PSDF>(src.view(scene), ptr, row_[0], code, R);
+  for (uint32_t turn = 0, third = 0; ci < n; turn ^= 1u, third = third == 2 ? 0 : third + 1) {
     if (scene != cur_scene) {
-      if (cur_scene != ~0u) cnt.flush(src.view(cur_scene));
+      if (cur_scene != ~0u && threadIdx.x == 0) cnt.flush(src.view(cur_scene));
       cur_scene = scene;
     }
     const View& V = src.view(scene);
     const McConst& mc = mc_of(src, scene, mc1);
     cnt.blocks += threadIdx.x == 0;
-    const i3 b = unpack_key(V.block_keys[ptr]);
-    const uint32_t i = threadIdx.x;
-    const size_t idx = (size_t)ptr * kBlockVoxels + i;
-    const uint32_t prev = V.cube[idx] & 255u;  // in flight with the shell loads
-    stage_shell<PSDF>(V, mc, nbe, S, nb, meshed);
-    const uint32_t next = s_next;
-    int32_t vps[3];  // this voxel's vertex slots (x, y, z edges)
+    const int32_t* const nb = row_[turn];
+    if (threadIdx.x == 0) next_[turn] = nx < n ? item_after(nx) : n;
+    if (nb_lane < 27) row_[turn ^ 1u][nb_lane] = nbe;
+    if (__any(stage_shell<PSDF>(mc, R, nb, code, S)) && (threadIdx.x & 63u) == 0) busy_[third][0] = 1u;
+    int32_t vps[kMcVox][3];
+    uint32_t word[kMcVox];
 #pragma unroll
-    for (int a = 0; a < 3; ++a) vps[a] = V.vptr[3 * idx + a];
-    if (threadIdx.x == 0) {
-      qn = 0;
-      surfels[0] = surfels[1] = 0;
+    for (int r = 0; r < kMcVox; ++r) {
+      word[r] = R.word[r];
+#pragma unroll
+      for (int a = 0; a < 3; ++a) vps[r][a] = R.vps[r][a];
     }
     __syncthreads();
+    // every wave is past the previous block: its flags and counts can go, and
+    // the next block's loads start
+    if (threadIdx.x == 0) {
+      const uint32_t before = third == 0 ? 2 : third - 1;
+      busy_[before][0] = busy_[before][1] = 0u;
+      qn = 0;
+      surfels[0] = surfels[1] = 0;
+      tri_sum[0] = tri_sum[1] = 0;
+    }
+    const uint32_t nn = next_[turn];
+    if (nx < n) load_block<PSDF>(src.view(scene_n), ptr_n, row_[turn ^ 1u], code, R);
+    nbe = nb_lane < 27 && nn < n ? nbt[(size_t)nn * 27u + nb_lane] : kFreePtr;
+    uint32_t scene_nn = 0;
+    int32_t ptr_nn = 0;
+    uint64_t key_nn = 0;
+    if (nn < n) {
+      ptr_nn = src.item(nn, &scene_nn);
+      key_nn = src.view(scene_nn).block_keys[ptr_nn];
+    }
+    const int32_t self = ptr;
+    const i3 b = unpack_key(key);
+    auto advance = [&] {
+      ci = nx;
+      nx = nn;
+      ptr = ptr_n;
+      ptr_n = ptr_nn;
+      scene = scene_n;
+      scene_n = scene_nn;
+      key = key_n;
+      key_n = key_nn;
+    };
+    // A block that keeps and gets no vertex: its cubes' words, its counts.
+    auto finish_empty = [&](const uint32_t* c) {
+      int lost = 0;
+#pragma unroll
+      for (int r = 0; r < kMcVox; ++r) {
+        const uint32_t prev = word[r] & 255u, nw = c[r] | (prev << 8);
+        if (nw != word[r]) V.cube[(size_t)self * kBlockVoxels + threadIdx.x + kMcLanes * r] = (uint16_t)nw;
+        lost += ntab[prev];  // c is 0 or 255: no triangle
+      }
+      // (rare: a block that lost its surface)
+      if (lost) atomicAdd(&work_stripe(V.ctr).tri_live, (unsigned long long)(long long)-lost);
+      if (threadIdx.x == 0) V.surfel[2 * self] = V.surfel[2 * self + 1] = 0;
+      advance();
+    };
+    uint32_t cube[kMcVox] = {};
+    if (!busy_[third][0]) {  // uniform
+      finish_empty(cube);
+      continue;
+    }
     // every cube of the 10^3 halo, the block's own among them: validity for
     // the writer rule, and the configuration of the block's own cubes
-    for (int s = (int)threadIdx.x; s < kCubeHalo * kCubeHalo * kCubeHalo; s += kBlockVoxels) {
+    bool crossing = false;
+#pragma unroll
+    for (int r = 0; r < kMcVox; ++r) crossing = crossing || vps[r][0] >= 0 || vps[r][1] >= 0 || vps[r][2] >= 0;
+    for (int s = (int)threadIdx.x; s < kCubeHalo * kCubeHalo * kCubeHalo; s += (int)kMcLanes) {
       const int x = s % kCubeHalo - 1, y = (s / kCubeHalo) % kCubeHalo - 1, z = s / (kCubeHalo * kCubeHalo) - 1;
       const int dx = x < 0 ? -1 : (x >= 8 ? 1 : 0), dy = y < 0 ? -1 : (y >= 8 ? 1 : 0),
                 dz = z < 0 ? -1 : (z >= 8 ? 1 : 0);
       int c;
       const bool valid = cube_index(S, x, y, z, &c);
-      const int q = nb27(dx, dy, dz);
-      cv[s] = meshed[q] && valid;
-      if ((dx | dy | dz) == 0) own_cube[x + 8 * y + 64 * z] = (uint8_t)(valid ? c : 0);
+      const int32_t q = nb[nb27(dx, dy, dz)];
+      cv[s] = row_meshed(q) && valid;
       if (dx <= 0 && dy <= 0 && dz <= 0) {
         // what the block's cube word holds after this pass: computed here
         // for a block meshed in it (its own pass computes the same bits from
         // the same voxels), stored for one that is not
         uint32_t hc = 0;
-        if (meshed[q])
+        if (row_meshed(q))
           hc = valid ? (uint32_t)c : 0u;
-        else if (nb[q] >= 0)
-          hc = V.cube[(size_t)nb[q] * kBlockVoxels + (x - 8 * dx) + 8 * (y - 8 * dy) + 64 * (z - 8 * dz)] & 255u;
+        else if (q >= 0)
+          hc = V.cube[(size_t)q * kBlockVoxels + (x - 8 * dx) + 8 * (y - 8 * dy) + 64 * (z - 8 * dz)] & 255u;
         hcfg[(x + 1) + kCfg * (y + 1) + kCfg * kCfg * (z + 1)] = (uint8_t)hc;
+        crossing = crossing || (hc != 0 && hc != 255);
       }
     }
+    if (__any(crossing) && (threadIdx.x & 63u) == 0) busy_[third][1] = 1u;
     __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kMcVox; ++r) {
+      const i3 o = devectorize(threadIdx.x + kMcLanes * r);
+      cube[r] = hcfg[(o.x + 1) + kCfg * (o.y + 1) + kCfg * kCfg * (o.z + 1)];
+    }
+    if (!busy_[third][1]) {  // uniform: no crossed edge here or below, no slot held
+      finish_empty(cube);
+      continue;
+    }
     // RecycleVerticesKernel on this block's own slots (marching_cubes.cu:
     // 303-321): a slot is referenced iff one of the four cubes around its edge
     // (this block and its lower neighbours, whose configurations are all
@@ -645,73 +710,90 @@ __global__ __launch_bounds__(512, 6) void mc_surfel_kernel(Src src_, const Scene
     // referenced free slot is claimed in this pass, here or by a lower
     // neighbour).  No other workgroup touches an unreferenced slot.
     unsigned release = 0;
+    unsigned em[kMcVox];
     {
-      const i3 o = devectorize(i);
-      const bool is_inner = o.x >= 1 && o.y >= 1 && o.z >= 1 && o.x < 7 && o.y < 7 && o.z < 7;
       int inner = 0, boundary = 0;
 #pragma unroll
-      for (int a = 0; a < 3; ++a) {
-        const int b1 = a == 0 ? 1 : 0, b2 = a == 2 ? 1 : 2;
-        bool used = false;
+      for (int r = 0; r < kMcVox; ++r) {
+        const i3 o = devectorize(threadIdx.x + kMcLanes * r);
+        const bool is_inner = o.x >= 1 && o.y >= 1 && o.z >= 1 && o.x < 7 && o.y < 7 && o.z < 7;
+        // the crossed edges of the eight cubes at o - {0, 1}^3
+        unsigned m8[8];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          int d[3] = {0, 0, 0};
-          d[b1] = k & 1;
-          d[b2] = k >> 1;
-          const unsigned m = etab[hcfg[(o.x - d[0] + 1) + kCfg * (o.y - d[1] + 1) + kCfg * kCfg * (o.z - d[2] + 1)]];
-          used = used || ((m >> edge_with(d[0], d[1], d[2], a)) & 1u) != 0;
+        for (int k = 0; k < 8; ++k)
+          m8[k] = etab[hcfg[(o.x - (k & 1) + 1) + kCfg * (o.y - ((k >> 1) & 1) + 1) + kCfg * kCfg * (o.z - (k >> 2) + 1)]];
+        em[r] = m8[0];  // 0 for configurations 0 and 255
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+          const int b1 = a == 0 ? 1 : 0, b2 = a == 2 ? 1 : 2;
+          bool used = false;
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            int d[3] = {0, 0, 0};
+            d[b1] = k & 1;
+            d[b2] = k >> 1;
+            used = used || ((m8[d[0] + 2 * d[1] + 4 * d[2]] >> edge_with(d[0], d[1], d[2], a)) & 1u) != 0;
+          }
+          if (vps[r][a] >= 0 || used) {
+            if (is_inner) ++inner;
+            else ++boundary;
+          }
+          if (vps[r][a] >= 0 && !used) release |= 1u << (3 * r + a);
         }
-        if (vps[a] >= 0 || used) {
-          if (is_inner) ++inner;
-          else ++boundary;
-        }
-        if (vps[a] >= 0 && !used) release |= 1u << a;
       }
       if (inner) atomicAdd(&surfels[0], inner);
       if (boundary) atomicAdd(&surfels[1], boundary);
     }
     const i3 base = i3{b.x * kBlockSide, b.y * kBlockSide, b.z * kBlockSide};
-    const int cube = own_cube[i];
-    V.cube[idx] = (uint16_t)((uint32_t)cube | (prev << 8));
-    // live triangles of a cube = its configuration's table row
-    const int nt = ntab[cube];
-    cnt.delta += nt - ntab[prev];
-    if ((uint32_t)cube != prev) cnt.assigned += (uint32_t)nt;
-    const unsigned em = etab[cube];  // 0 for configurations 0 and 255
+    const float inv_vs = 1.0f / V.geo.voxel_size;
+    {
+      int delta = 0, assigned = 0;
+#pragma unroll
+      for (int r = 0; r < kMcVox; ++r) {
+        const uint32_t prev = word[r] & 255u, nw = cube[r] | (prev << 8);
+        if (nw != word[r]) V.cube[(size_t)self * kBlockVoxels + threadIdx.x + kMcLanes * r] = (uint16_t)nw;
+        // live triangles of a cube = its configuration's table row
+        const int nt = ntab[cube[r]];
+        delta += nt - ntab[prev];
+        if (cube[r] != prev) assigned += nt;
+      }
+      if (delta) atomicAdd(&tri_sum[0], delta);
+      if (assigned) atomicAdd(&tri_sum[1], assigned);
+    }
     // The crossed edges of the block's cubes become a dense item list
     // (voxel | edge << 9), so the slot work below runs one item per lane
     // instead of twelve edge rounds on every cube.  The same scan ranks the
     // freed slots (bits 13 and up: the item counts sum to at most 6144).
-    uint32_t free_rank;
+    uint32_t free_rank, n_freed;
     {
-      const uint32_t mine = (uint32_t)__popc(em) | ((uint32_t)__popc(release) << 13);  // <= 12, <= 3
+      static_assert(kMcVox <= 2, "at most 24 items and 6 freed slots a lane");
+      uint32_t mine = (uint32_t)__popc(release) << 13;
+#pragma unroll
+      for (int r = 0; r < kMcVox; ++r) mine += (uint32_t)__popc(em[r]);
       uint32_t total;
-      const uint32_t at2 = block_excl_scan_planes<0xFu | (0x3u << 13)>(mine, scan_wave, &total);
+      const uint32_t at2 =
+          block_excl_scan_planes<kMcVox == 2 ? 0x1Fu | (0x7u << 13) : 0xFu | (0x3u << 13)>(mine, scan_wave, &total);
       uint32_t at = at2 & 8191u;
       free_rank = at2 >> 13;
-      for (unsigned m = em; m; m &= m - 1u) items[at++] = (uint16_t)(i | ((uint32_t)(__ffs(m) - 1) << 9));
-      if (threadIdx.x == 0) {
-        nitems = total & 8191u;
-        if (total >> 13) free_base = atomicAdd(&V.ctr->vfree_count, total >> 13);
-      }
+#pragma unroll
+      for (int r = 0; r < kMcVox; ++r)
+        for (unsigned m = em[r]; m; m &= m - 1u)
+          items[at++] = (uint16_t)((threadIdx.x + kMcLanes * r) | ((uint32_t)(__ffs(m) - 1) << 9));
+      if (threadIdx.x == 0) nitems = total & 8191u;
+      n_freed = total >> 13;
     }
+    // the freed slots' place on the list, waited for after the claims
+    uint32_t base_got = 0;
+    if (threadIdx.x == 0 && n_freed) base_got = atomicAdd(&V.ctr->vfree_count, n_freed);
     __syncthreads();
     const uint32_t n_items = nitems;
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-      if (!((release >> a) & 1u)) continue;
-      const int32_t vp = vps[a];
-      Vertex zv{};
-      V.vertices[vp] = zv;
-      V.vptr[3 * idx + a] = kFreePtr;
-      V.vfree[free_base + free_rank] = vp;
-      ++free_rank;
-    }
     if (threadIdx.x == 0) {
-      V.surfel[2 * ptr + 0] = surfels[0];
-      V.surfel[2 * ptr + 1] = surfels[1];
+      V.surfel[2 * self + 0] = surfels[0];
+      V.surfel[2 * self + 1] = surfels[1];
+      cnt.delta += tri_sum[0];
+      cnt.assigned += (uint32_t)tri_sum[1];
     }
-    for (uint32_t c0 = 0; c0 < n_items; c0 += kBlockVoxels) {
+    for (uint32_t c0 = 0;; c0 += kMcLanes) {
       // Vertex slot of each item: read it; claim it if free (CAS to the
       // lock value); pop fresh vertices for all claims of the workgroup
       // with one heap operation; publish them.
@@ -754,59 +836,72 @@ __global__ __launch_bounds__(512, 6) void mc_surfel_kernel(Src src_, const Scene
           cur = fresh;
         }
       }
-      if (!has || cur < 0) continue;
-      const int ax = edge_axis(e);
-      const int offx = edge_owner_off(e, 0), offy = edge_owner_off(e, 1), offz = edge_owner_off(e, 2);
-      const int ox = oo.x + offx, oy = oo.y + offy, oz = oo.z + offz;
-      // writer rule: offsets across the edge in the two other axes (b1 < b2;
-      // selected without indexing, e being a run-time value here)
-      const int b1 = ax == 0 ? 1 : 0, b2 = ax == 2 ? 1 : 2;
-      const int own1 = b1 == 0 ? offx : offy, own2 = b2 == 1 ? offy : offz;
-      const int kself = own1 + 2 * own2;
-      // A slot claimed in this pass is also written by its claimer: the
-      // designated cube may have read it while still locked and skipped it.
-      bool writer = true;
-      for (int k = 0; k < kself && writer && !claimed; ++k) {
-        const int d1 = k & 1, d2 = k >> 1;
-        const int qx = ox - (b1 == 0 ? d1 : 0);
-        const int qy = oy - (b1 == 1 ? d1 : 0) - (b2 == 1 ? d2 : 0);
-        const int qz = oz - (b2 == 2 ? d2 : 0);
-        if (cv[cidx(qx, qy, qz)]) writer = false;
+      if (has && cur >= 0) {
+        const int ax = edge_axis(e);
+        const int offx = edge_owner_off(e, 0), offy = edge_owner_off(e, 1), offz = edge_owner_off(e, 2);
+        const int ox = oo.x + offx, oy = oo.y + offy, oz = oo.z + offz;
+        // writer rule: offsets across the edge in the two other axes (b1 < b2;
+        // selected without indexing, e being a run-time value here)
+        const int b1 = ax == 0 ? 1 : 0, b2 = ax == 2 ? 1 : 2;
+        const int own1 = b1 == 0 ? offx : offy, own2 = b2 == 1 ? offy : offz;
+        const int kself = own1 + 2 * own2;
+        // A slot claimed in this pass is also written by its claimer: the
+        // designated cube may have read it while still locked and skipped it.
+        bool writer = true;
+        for (int k = 0; k < kself && writer && !claimed; ++k) {
+          const int d1 = k & 1, d2 = k >> 1;
+          const int qx = ox - (b1 == 0 ? d1 : 0);
+          const int qy = oy - (b1 == 1 ? d1 : 0) - (b2 == 1 ? d2 : 0);
+          const int qz = oz - (b2 == 2 ? d2 : 0);
+          if (cv[cidx(qx, qy, qz)]) writer = false;
+        }
+        if (writer) {  // queue the payload; all lanes of the block work the queue
+          const uint32_t q = atomicAdd(&qn, 1u);
+          qptr[q] = cur;
+          qkey[q] = (uint16_t)((uint32_t)ox | ((uint32_t)oy << 4) | ((uint32_t)oz << 8) | ((uint32_t)ax << 12));
+        }
       }
-      if (!writer) continue;
-      // queue the payload; all lanes of the block work the queue below
-      const uint32_t q = atomicAdd(&qn, 1u);
-      const uint32_t key = (uint32_t)ox | ((uint32_t)oy << 4) | ((uint32_t)oz << 8) | ((uint32_t)ax << 12);
-      if (q < kQueue) {
-        qptr[q] = cur;
-        qkey[q] = (uint16_t)key;
-      } else {
-        cnt.oob = write_vertex<PSDF>(S, V, mc, base, key, cur) || cnt.oob;
-        ++cnt.writes;
+      if (threadIdx.x == 0 && c0 == 0 && n_freed) free_base = base_got;
+      __syncthreads();
+      if (c0 == 0 && n_freed) {  // uniform
+#pragma unroll
+        for (int r = 0; r < kMcVox; ++r)
+#pragma unroll
+          for (int a = 0; a < 3; ++a) {
+            if (!((release >> (3 * r + a)) & 1u)) continue;
+            const int32_t vp = vps[r][a];
+            Vertex zv{};
+            V.vertices[vp] = zv;
+            V.vptr[3 * ((size_t)self * kBlockVoxels + threadIdx.x + kMcLanes * r) + a] = kFreePtr;
+            V.vfree[free_base + free_rank] = vp;
+            ++free_rank;
+          }
       }
-    }
-    __syncthreads();
-    if (nb_lane < 27 && next < n) nbe = nbt[(size_t)next * 27u + nb_lane];
-    const uint32_t nq = qn < kQueue ? qn : kQueue;
-    // payloads, eight lanes per vertex, on the waves before the last one
-    // (which looks up the next block's neighbours meanwhile)
-    for (uint32_t j0 = 0; j0 < nq; j0 += kPayRound) {  // uniform
+      const bool last = c0 + kMcLanes >= n_items;  // uniform
+      if (!last && qn + kMcLanes <= kQueue) continue;
+      // payloads, eight lanes per vertex
+      const uint32_t nq = qn;
+      cnt.writes += nq;
       const uint32_t jl = threadIdx.x >> 3, sub = threadIdx.x & 7u;
-      const uint32_t j = j0 + jl;
-      const bool act = threadIdx.x < kLookupLane && j < nq;
-      if (act)
-        cnt.oob = payload_part<PSDF>(S, V, mc, base, qkey[j], qptr[j], sub, &pay_s[8 * jl], &pay_ok[8 * jl]) ||
-                  cnt.oob;
-      __syncthreads();
-      if (act && sub == 0) {
-        finish_normal(V, qptr[j], &pay_s[8 * jl], &pay_ok[8 * jl]);
-        ++cnt.writes;
+      for (uint32_t j0 = 0; j0 < nq; j0 += kPayRound) {  // uniform
+        const uint32_t j = j0 + jl;
+        const bool act = j < nq;  // the same for a vertex's eight lanes
+        PaySample q;
+        if (act && payload_part<PSDF>(S, V, mc, inv_vs, base, qkey[j], qptr[j], sub, &pay_s[8 * jl], &pay_r[8 * jl],
+                                      &pay_ok[8 * jl], &q))
+          flag(V, MH_STATUS_STENCIL_RANGE);
+        __syncthreads();
+        if (act && sub == 0) finish_normal(V, qptr[j], &pay_s[8 * jl], &pay_ok[8 * jl]);
+        if (act && sub == 6) finish_sample(V, qptr[j], q, &pay_r[8 * jl]);
+        __syncthreads();
       }
+      if (last) break;
+      if (threadIdx.x == 0) qn = 0;
       __syncthreads();
     }
-    ci = next;
+    advance();
   }
-  if (cur_scene != ~0u) cnt.flush(src.view(cur_scene));
+  if (threadIdx.x == 0) cnt.flush(src.view(cur_scene));
 }
 
 // Meshed-in-this-pass marks for the writer rule.
@@ -1213,7 +1308,7 @@ int resident_grid(int cus) {
 // resident), at most the resident count.
 template <auto K>
 int surfel_grid(int cus, const McShape& shape) {
-  const int resident = resident_grid<K, kBlockVoxels>(cus);
+  const int resident = resident_grid<K, (int)kMcLanes>(cus);
   const int g = shape.grid_per_cu > 0 ? shape.grid_per_cu * cus : resident;
   return g < resident ? g : resident;
 }
@@ -1229,9 +1324,9 @@ void launch_marching_cubes(const View& V, const McConst& p, int32_t* nbt, hipStr
   mc_neighbours_kernel<<<cus * 8, 256, 0, s>>>(One{V}, nullptr, p, nbt);
   tick(kc, s, "mc_surfel_kernel");
   if (V.va)
-    mc_surfel_kernel<true><<<grid, kBlockVoxels, 0, s>>>(One{V}, nullptr, p, nbt, q);
+    mc_surfel_kernel<true><<<grid, kMcLanes, 0, s>>>(One{V}, nullptr, p, nbt, q);
   else
-    mc_surfel_kernel<false><<<grid, kBlockVoxels, 0, s>>>(One{V}, nullptr, p, nbt, q);
+    mc_surfel_kernel<false><<<grid, kMcLanes, 0, s>>>(One{V}, nullptr, p, nbt, q);
   tick(kc, s, "mc_push_freed_kernel");
   mc_push_freed_kernel<<<kPushGrid, 256, 0, s>>>(One{V}, nullptr);
   tick(kc, s, nullptr);
@@ -1251,9 +1346,9 @@ void launch_batch_marching_cubes(const BatchDev& B, int32_t* nbt, hipStream_t s,
   if (!marks_stamped) mc_mark_kernel<<<cus, 256, 0, s>>>(B.src(), B.frames, unused);
   mc_neighbours_kernel<<<cus * 8, 256, 0, s>>>(B.src(), B.frames, unused, nbt);
   if (B.psdf)
-    mc_surfel_kernel<true><<<grid, kBlockVoxels, 0, s>>>(B.src(), B.frames, unused, nbt, q);
+    mc_surfel_kernel<true><<<grid, kMcLanes, 0, s>>>(B.src(), B.frames, unused, nbt, q);
   else
-    mc_surfel_kernel<false><<<grid, kBlockVoxels, 0, s>>>(B.src(), B.frames, unused, nbt, q);
+    mc_surfel_kernel<false><<<grid, kMcLanes, 0, s>>>(B.src(), B.frames, unused, nbt, q);
   mc_push_freed_kernel<<<dim3(kPushGrid, B.nscenes), 256, 0, s>>>(B.src(), B.frames);
 }
 

@@ -58,7 +58,7 @@ struct One {
   View V;
   __device__ __forceinline__ const View& view(uint32_t) const { return V; }
   __device__ __forceinline__ uint32_t count() const { return V.ctr->cand_count; }
-  __device__ __forceinline__ uint32_t* next_ctr() const { return &V.ctr->mc_next; }
+  __device__ __forceinline__ uint32_t* next_ctr() const { return V.ctr->mc_next[0]; }
   __device__ __forceinline__ int32_t item(uint32_t ci, uint32_t* scene) const {
     *scene = 0;
     return V.cand[ci];
@@ -72,7 +72,7 @@ struct Many {
   const SceneFrame* __restrict__ f;
   const uint32_t* __restrict__ work;
   const uint32_t* work_count;
-  uint32_t* dyn;  // items handed out on demand (marching cubes), after the static ones
+  uint32_t* dyn;  // items handed out on demand (marching cubes), after the static ones: kDynGroups lines of 64
   __device__ __forceinline__ const View& view(uint32_t s) const { return f[s].V; }
   __device__ __forceinline__ uint32_t count() const { return *work_count; }
   __device__ __forceinline__ uint32_t* next_ctr() const { return dyn; }
@@ -121,7 +121,7 @@ struct BatchDev {
   SceneFrame* frames;   // device table, nscenes entries
   uint32_t* work;       // concatenated worklist
   uint32_t* work_count;
-  uint32_t* dyn;        // marching cubes' on-demand item counter
+  uint32_t* dyn;        // marching cubes' on-demand item counters (kDynGroups lines of 64)
   uint32_t nscenes;
   uint32_t width, height;  // common image size
   int psdf;             // scenes carry PSDF fields (all or none)
