@@ -894,10 +894,10 @@ int mh_raycast(mh_volume* v, const mh_raycaster_params* p, const float cTw[16], 
     View Vr = v->V;  // lookups record the blocks they find; then they are counted
     Vr.ray_mark = v->ray_mark;
     Vr.ray_stamp = ++v->ray_stamp;
-    launch_raycast(Vr, R, depth_dev, vertex_dev, normal_dev, v->stream, v->kc(), v->ray_shape);
+    launch_raycast(Vr, R, depth_dev, vertex_dev, normal_dev, v->stream, v->cus, v->kc(), v->ray_shape);
     launch_ray_mark_count(Vr, v->stream, v->cus * 2);
   } else {
-    launch_raycast(v->V, R, depth_dev, vertex_dev, normal_dev, v->stream, v->kc(), v->ray_shape);
+    launch_raycast(v->V, R, depth_dev, vertex_dev, normal_dev, v->stream, v->cus, v->kc(), v->ray_shape);
   }
   HIP_TRY(hipGetLastError());
   return MH_OK;
@@ -1533,14 +1533,14 @@ int batch_chain(mh_batch* b, uint32_t flags, bool integrate) {
   if (batch_overlaps(b, flags)) {
     HIP_TRY(hipEventRecord(b->fork, b->stream));
     HIP_TRY(hipStreamWaitEvent(b->side, b->fork, 0));
-    launch_batch_raycast(B, b->out_depth, b->out_vertex, b->out_normal, b->side, b->ray_shape);
+    launch_batch_raycast(B, b->out_depth, b->out_vertex, b->out_normal, b->side, b->cus, b->ray_shape);
     launch_batch_marching_cubes(B, b->d_nbt, b->stream, b->cus, kMcShapes[b->mc_shape], true);
     HIP_TRY(hipEventRecord(b->join, b->side));
     HIP_TRY(hipStreamWaitEvent(b->stream, b->join, 0));
     return MH_OK;
   }
   if (flags & MH_RUN_MESH) launch_batch_marching_cubes(B, b->d_nbt, b->stream, b->cus, kMcShapes[b->mc_shape], true);
-  if (flags & MH_RUN_RAYCAST) launch_batch_raycast(B, b->out_depth, b->out_vertex, b->out_normal, b->stream, b->ray_shape);
+  if (flags & MH_RUN_RAYCAST) launch_batch_raycast(B, b->out_depth, b->out_vertex, b->out_normal, b->stream, b->cus, b->ray_shape);
   return MH_OK;
 }
 
@@ -1605,7 +1605,7 @@ int mh_tune_raycast(mh_volume* v, const mh_raycaster_params* p, const float cTw[
   HIP_TRY(sc.get(&sctr, 1));
   launch_ray_range_one(v->V, R, v->stream);
   HIP_TRY(hipMemcpyAsync(sctr, v->V.ctr, sizeof(Counters), hipMemcpyDeviceToDevice, v->stream));
-  auto run = [&](int k) { launch_raycast_march(v->V, R, d, nullptr, n, v->stream, k); };
+  auto run = [&](int k) { launch_raycast_march(v->V, R, d, nullptr, n, v->stream, v->cus, k); };
   auto restore = [&]() -> int {
     HIP_TRY(hipMemcpyAsync(v->V.ctr, sctr, sizeof(Counters), hipMemcpyDeviceToDevice, v->stream));
     return MH_OK;
@@ -2002,7 +2002,7 @@ int mh_batch_run(mh_batch* b, const mh_mc_params* mc, uint32_t flags, mh_tune_re
       for (uint32_t s = 0; s < b->n; ++s)
         HIP_TRY(hipMemcpyAsync(sctr + s, b->vols[s]->V.ctr, sizeof(Counters), hipMemcpyDeviceToDevice,
                                b->stream));
-      auto run = [&](int k) { launch_batch_raycast(B, b->out_depth, b->out_vertex, b->out_normal, b->stream, k); };
+      auto run = [&](int k) { launch_batch_raycast(B, b->out_depth, b->out_vertex, b->out_normal, b->stream, b->cus, k); };
       auto restore = [&]() -> int {
         for (uint32_t s = 0; s < b->n; ++s)
           HIP_TRY(hipMemcpyAsync(b->vols[s]->V.ctr, sctr + s, sizeof(Counters), hipMemcpyDeviceToDevice,
@@ -2014,7 +2014,7 @@ int mh_batch_run(mh_batch* b, const mh_mc_params* mc, uint32_t flags, mh_tune_re
       if (rc2) return rc2;
       b->ray_shape = best;
       if (tune_out) tune_out->ray_shape = best;
-      launch_batch_raycast(B, b->out_depth, b->out_vertex, b->out_normal, b->stream, b->ray_shape);
+      launch_batch_raycast(B, b->out_depth, b->out_vertex, b->out_normal, b->stream, b->cus, b->ray_shape);
     }
   } else if (flags & MH_RUN_GRAPH) {
     McTune& t = b->mct;

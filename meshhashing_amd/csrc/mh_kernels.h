@@ -233,16 +233,16 @@ constexpr int kNumRayShapes = sizeof(kRayTileWidths) / sizeof(kRayTileWidths[0])
 // raycast waves resident per SIMD (the kernel is held to 96 registers)
 constexpr int kRayWavesPerSimd = 5;
 void launch_raycast(const View& V, const RayConst& p, float* depth, float* vertex, float* normal,
-                    hipStream_t s, const KernelClock* kc = nullptr, int shape = 0);
+                    hipStream_t s, int cus, const KernelClock* kc = nullptr, int shape = 0);
 // the march alone (the tile ranges already filled)
 void launch_raycast_march(const View& V, const RayConst& p, float* depth, float* vertex, float* normal,
-                          hipStream_t s, int shape);
+                          hipStream_t s, int cus, int shape);
 void launch_ray_range_one(const View& V, const RayConst& p, hipStream_t s);
 // diagnostics: add the distinct blocks the last raycast sampled (V.ray_mark
 // == V.ray_stamp) to the work counters
 void launch_ray_mark_count(const View& V, hipStream_t s, int grid);
 void launch_batch_raycast(const BatchDev& B, float* depth, float* vertex, float* normal,
-                          hipStream_t s, int shape = 0);
+                          hipStream_t s, int cus, int shape = 0);
 // adjoint: 31 FP64 sums (loss, dL/dxi[6], J^T J upper triangle[21], pixels,
 // gated-out pixels, observed pixels)
 constexpr int kGradSlots = 31;

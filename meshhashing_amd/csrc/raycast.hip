@@ -6,7 +6,8 @@
 // BisectionIntersection), geometry/spatial_query.h:23-97 (trilinear value and
 // gradient), geometry/voxel_query.h:102-129 (world-point voxel lookup).
 //
-// One lane per pixel, 8x8 pixels per wave.  Samples, the crossing test and
+// One lane per pixel, 8x8 pixels per wave (two or four lanes per pixel for
+// small images).  Samples, the crossing test and
 // the three regula-falsi steps follow the reference's FP32 expressions.  The
 // march keeps the eight blocks around its current lowest-corner block
 // (Octant) and shares block lookups, misses included, through a per-wave LDS
@@ -415,6 +416,139 @@ __device__ __forceinline__ bool find_surface(const View& V, const RayConst& R, f
   }
 }
 
+// Lane j of the L lanes that share a ray, as seen by all of them (L: 2 or 4,
+// neighbouring lanes; they run one path except inside a sample).
+template <int L, int J>
+__device__ __forceinline__ uint32_t ray_lane(uint32_t x) {
+  constexpr int ctrl = L == 4 ? J * 0x55 : (J | (J << 2) | ((2 + J) << 4) | ((2 + J) << 6));
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, ctrl, 0xF, 0xF, true);
+}
+template <int L, int J>
+__device__ __forceinline__ float ray_lane(float x) {
+  return __uint_as_float(ray_lane<L, J>(__float_as_uint(x)));
+}
+
+// find_surface by L lanes a ray: lane q takes every L-th sample, from the q-th
+// on; the samples of a round are then walked through in the ray's order by all
+// of its lanes, so that the crossing, the acceptance and the count are
+// find_surface's.  A round ends with the last lane's sample; where that lies
+// in an absent block, the next round starts behind the block.
+template <bool kWide, int L>
+__device__ __forceinline__ bool find_surface_split(const View& V, const RayConst& R, f3 o, f3 dir, float t_min,
+                                                   float t_max, float t_lo, float t_hi, WaveTable* table,
+                                                   Octant& oc, Hit* hit, uint32_t* nsamp) {
+  float prev_sdf = 0.0f, prev_t = 0.0f;
+  bool prev_ok = false;
+  if (!(t_lo < t_max) || t_hi < t_lo) return false;  // no block along this ray
+  float t = advance_steps(t_min, R.step, t_lo);
+  const uint32_t q = threadIdx.x & (L - 1);
+  while (true) {
+    float s = 0.0f, tc = 0.0f;
+    bool cross = false;
+    while (t < t_max && t <= t_hi) {
+      float ts[L];
+      ts[0] = t;
+#pragma unroll
+      for (int j = 1; j < L; ++j) ts[j] = ts[j - 1] + R.step;
+      float tq = ts[0];
+#pragma unroll
+      for (int j = 1; j < L; ++j) tq = q == (uint32_t)j ? ts[j] : tq;
+      float sv = 0.0f, t_out = 0.0f;
+      bool ok = false;
+      if (tq < t_max && tq <= t_hi) {
+        ok = point_sample<kWide>(V, table, oc, mk3(o.x + tq * dir.x, o.y + tq * dir.y, o.z + tq * dir.z), R.inv_vs, &sv);
+        if (!ok && oc.p[0] < 0) t_out = absent_exit_t(oc.p[0], o, dir, oc.bx, oc.by, oc.bz, V.geo.voxel_size);
+      }
+      const uint32_t oku = ok ? 1u : 0u;
+      auto take = [&](float v, uint32_t k, float tj) {
+        if (cross || !k) return;
+        ++*nsamp;
+        if (prev_ok && prev_sdf > 0.0f && v < 0.0f) {
+          s = v;
+          tc = tj;
+          cross = true;
+          return;
+        }
+        prev_sdf = v;
+        prev_t = tj;
+        prev_ok = true;
+      };
+      take(ray_lane<L, 0>(sv), ray_lane<L, 0>(oku), ts[0]);
+      take(ray_lane<L, 1>(sv), ray_lane<L, 1>(oku), ts[1]);
+      if constexpr (L == 4) {
+        take(ray_lane<L, 2>(sv), ray_lane<L, 2>(oku), ts[2]);
+        take(ray_lane<L, 3>(sv), ray_lane<L, 3>(oku), ts[3]);
+      }
+      if (cross) break;
+      const float out = ray_lane<L, L - 1>(t_out);
+      t = ts[L - 1];
+      for (float tn = t + R.step; tn < out && tn > t; tn = t + R.step) t = tn;
+      t += R.step;
+    }
+    if (!cross) return false;
+    // BisectionIntersection: three regula-falsi steps.
+    float l = prev_t, r = tc, m = (l + r) * 0.5f;
+    float l_sdf = prev_sdf, r_sdf = s;
+    bool found = true;
+#pragma unroll 1
+    for (int k = 0; k < 3; ++k) {
+      m = l + (l_sdf / (l_sdf - r_sdf)) * (r - l);
+      float m_sdf;
+      if (!point_sample<kWide>(V, table, oc, mk3(o.x + m * dir.x, o.y + m * dir.y, o.z + m * dir.z), R.inv_vs,
+                               &m_sdf)) {
+        found = false;
+        break;
+      }
+      if (l_sdf * m_sdf > 0.0f) {
+        l = m;
+        l_sdf = m_sdf;
+      } else {
+        r = m;
+        r_sdf = m_sdf;
+      }
+    }
+    if (found && fabsf(prev_sdf - s) < R.sample_sdf_threshold && fabsf(s) < R.sdf_threshold) {
+      *hit = Hit{prev_t, prev_sdf, tc, s, m};
+      return true;
+    }
+    prev_sdf = s;
+    prev_t = tc;
+    prev_ok = true;
+    t = tc + R.step;
+  }
+}
+
+// gradient_samples by L lanes a ray, each taking one stencil sample a round.
+template <bool kWide, int L>
+__device__ __forceinline__ bool gradient_samples_split(const View& V, WaveTable* t, Octant& oc, f3 p, float inv_vs,
+                                                       float* g0, float* g1, float* g2) {
+  const float vs = V.geo.voxel_size, h = 0.5f * vs;
+  const uint32_t q = threadIdx.x & (L - 1);
+  bool valid = true;
+  *g0 = *g1 = *g2 = 0.0f;
+#pragma unroll 1
+  for (int j0 = 0; j0 < 6; j0 += L) {
+    const int j = min(j0 + (int)q, 5), k = j >> 1;  // x-, x+, y-, y+, z-, z+
+    const float d = (j & 1) ? h : -h;
+    float s = 0.0f;
+    // (p - 0 = p: the other two coordinates are p's)
+    const bool ok = point_sample<kWide>(V, t, oc, mk3(k == 0 ? p.x + d : p.x, k == 1 ? p.y + d : p.y, k == 2 ? p.z + d : p.z),
+                                        inv_vs, &s);
+    const uint32_t oku = ok ? 1u : 0u;
+    valid = valid && ray_lane<L, 0>(oku) && ray_lane<L, 1>(oku);
+    const float ga = (ray_lane<L, 1>(s) - ray_lane<L, 0>(s)) / vs;
+    if (j0 == 0) *g0 = ga;
+    if (j0 == 2) *g1 = ga;
+    if (j0 == 4) *g2 = ga;
+    if constexpr (L == 4) {
+      valid = valid && ray_lane<L, 2>(oku) && ray_lane<L, 3>(oku);
+      const float gb = (ray_lane<L, 3>(s) - ray_lane<L, 2>(s)) / vs;
+      if (j0 == 0) *g1 = gb;
+    }
+  }
+  return valid;
+}
+
 // The ray parameters between which pixel (x, y) can meet an allocated block:
 // the tile's camera-z range over dir_c.z, widened by 0.1 %.
 __device__ __forceinline__ void ray_bounds(const RayConst& R, uint32_t x, uint32_t y, float dcz, float t_min,
@@ -427,7 +561,7 @@ __device__ __forceinline__ void ray_bounds(const RayConst& R, uint32_t x, uint32
 }
 
 // March one pixel; returns the number of valid samples taken.
-template <bool kWide>
+template <bool kWide, int L>
 __device__ __forceinline__ uint32_t cast_pixel(const View& V, const RayConst& R, uint32_t x, uint32_t y,
                                WaveTable* table, float* res_d, f3* res_v, f3* res_n) {
   uint32_t nsamp = 0;
@@ -445,7 +579,12 @@ __device__ __forceinline__ uint32_t cast_pixel(const View& V, const RayConst& R,
   float t_lo, t_hi;
   ray_bounds(R, x, y, dir_c.z, t_min, t_max, &t_lo, &t_hi);
   Octant oc = empty_octant();
-  if (find_surface<kWide>(V, R, o, dir, t_min, t_max, t_lo, t_hi, table, oc, &hit, &nsamp)) {
+  bool found;
+  if constexpr (L == 1)
+    found = find_surface<kWide>(V, R, o, dir, t_min, t_max, t_lo, t_hi, table, oc, &hit, &nsamp);
+  else
+    found = find_surface_split<kWide, L>(V, R, o, dir, t_min, t_max, t_lo, t_hi, table, oc, &hit, &nsamp);
+  if (found) {
     const float m = hit.m;
     const float d = m * dir_c.z;
     out_d = d;
@@ -453,7 +592,11 @@ __device__ __forceinline__ uint32_t cast_pixel(const View& V, const RayConst& R,
     if (R.enable_gradients) {
       const f3 iso = mk3(o.x + m * dir.x, o.y + m * dir.y, o.z + m * dir.z);
       f3 grad;
-      const bool valid = gradient_samples<kWide>(V, table, oc, iso, R.inv_vs, &grad.x, &grad.y, &grad.z);
+      bool valid;
+      if constexpr (L == 1)
+        valid = gradient_samples<kWide>(V, table, oc, iso, R.inv_vs, &grad.x, &grad.y, &grad.z);
+      else
+        valid = gradient_samples_split<kWide, L>(V, table, oc, iso, R.inv_vs, &grad.x, &grad.y, &grad.z);
       const float l2 = length(grad);
       f3 nw = (l2 > 0.0f && valid) ? grad / l2 : mk3(0.0f, 0.0f, 0.0f);
       nw = -nw;
@@ -856,7 +999,8 @@ __device__ __forceinline__ const RayConst& ray_of(const Many& m, uint32_t s, con
 // tiles at once on 256 CUs (four would leave a partial second round).
 // tw: log2 of the tile's width in pixels (the tile has 64; every shape gives
 // the same per-pixel results, the autotuner picks the fastest).
-template <class Src, bool kWide>
+// L lanes a ray (64 / L pixels a wave): see ray_lanes.
+template <class Src, bool kWide, int L>
 __global__ __launch_bounds__(64, kRayWavesPerSimd) void raycast_kernel(Src src_, const SceneFrame* __restrict__ tab, RayConst R1, int tw, float* __restrict__ depth_out,
                                                      float* __restrict__ vertex_out,
                                                      float* __restrict__ normal_out) {
@@ -869,24 +1013,30 @@ __global__ __launch_bounds__(64, kRayWavesPerSimd) void raycast_kernel(Src src_,
   const View V = src.view(scene);
   const RayConst R = ray_of(src, scene, R1);
   if (R.boost) __builtin_amdgcn_s_setprio(2);
-  const uint32_t x = (blockIdx.x << tw) + (threadIdx.x & ((1u << tw) - 1u));
-  const uint32_t y = (blockIdx.y << (6 - tw)) + (threadIdx.x >> tw);
+  constexpr int kLog = L == 4 ? 2 : (L == 2 ? 1 : 0);
+  const uint32_t ray = threadIdx.x >> kLog;
+  const uint32_t x = (blockIdx.x << tw) + (ray & ((1u << tw) - 1u));
+  const uint32_t y = (blockIdx.y << (6 - kLog - tw)) + (ray >> tw);
   uint32_t ns = 0;
   if (x < R.cam.width && y < R.cam.height) {
     const size_t pix = (size_t)scene * R.cam.width * R.cam.height + y * R.cam.width + x;
     float d;
     f3 vv, nn;
-    ns = cast_pixel<kWide>(V, R, x, y, &table, &d, &vv, &nn);
-    if (depth_out) depth_out[pix] = d;
-    if (vertex_out) {
-      vertex_out[3 * pix + 0] = vv.x;
-      vertex_out[3 * pix + 1] = vv.y;
-      vertex_out[3 * pix + 2] = vv.z;
-    }
-    if (normal_out) {
-      normal_out[3 * pix + 0] = nn.x;
-      normal_out[3 * pix + 1] = nn.y;
-      normal_out[3 * pix + 2] = nn.z;
+    ns = cast_pixel<kWide, L>(V, R, x, y, &table, &d, &vv, &nn);
+    if (L == 1 || (threadIdx.x & (L - 1)) == 0) {
+      if (depth_out) depth_out[pix] = d;
+      if (vertex_out) {
+        vertex_out[3 * pix + 0] = vv.x;
+        vertex_out[3 * pix + 1] = vv.y;
+        vertex_out[3 * pix + 2] = vv.z;
+      }
+      if (normal_out) {
+        normal_out[3 * pix + 0] = nn.x;
+        normal_out[3 * pix + 1] = nn.y;
+        normal_out[3 * pix + 2] = nn.z;
+      }
+    } else {
+      ns = 0;  // the ray's first lane has counted its samples
     }
   }
   wave_add_u64(&work_stripe(V.ctr).ray_samples, ns);
@@ -1074,16 +1224,29 @@ void launch_ray_range(Src src, const SceneFrame* tab, const RayConst& R, uint32_
   }
 }
 
+// Lanes a ray: an image of few pixels leaves the chip nearly empty, a wave a
+// SIMD at 333 x 251, and each wave's time is the latency of its rays' samples
+// in a row; four (two) lanes a ray then take a quarter (half) of the rounds.
+// As many as fit the chip in one round of waves; past that the extra lanes only
+// add work.  Measured (5 mm desk, whole call, 1 / 2 / 4 lanes): 160 x 120
+// 155 / 128 / 92 us, 320 x 240 138 / 124 / 98, 400 x 300 147 / 130 / 137,
+// 480 x 360 149 / 155 / 152, 640 x 480 142 / 162 / 189.
+inline int ray_lanes(uint64_t pixels, int cus) {
+  const uint64_t waves = (pixels + 63) / 64, room = (uint64_t)kRayWavesPerSimd * 4 * (uint64_t)cus;
+  return 4 * waves <= room ? 4 : (2 * waves <= room ? 2 : 1);
+}
 template <class Src>
 void raycast_shaped(Src src, const SceneFrame* tab, const RayConst& p, uint32_t w, uint32_t h, uint32_t nscenes,
-                    bool wide, int shape, float* depth, float* vertex, float* normal, hipStream_t s) {
-  const int tw = kRayTileWidths[shape], th = 64 / tw;
+                    bool wide, int shape, int cus, float* depth, float* vertex, float* normal, hipStream_t s) {
+  const int lanes = wide || shape != 0 ? 1 : ray_lanes((uint64_t)w * h * nscenes, cus);
+  const int px = 64 / lanes;
+  const int tw = lanes == 1 ? kRayTileWidths[shape] : (lanes == 2 ? 8 : 4), th = px / tw;
   const int log_tw = __builtin_ctz((unsigned)tw);
   const dim3 grid((w + tw - 1) / tw, (h + th - 1) / th, nscenes);
-  if (wide)
-    raycast_kernel<Src, true><<<grid, 64, 0, s>>>(src, tab, p, log_tw, depth, vertex, normal);
-  else
-    raycast_kernel<Src, false><<<grid, 64, 0, s>>>(src, tab, p, log_tw, depth, vertex, normal);
+  const auto k = wide ? raycast_kernel<Src, true, 1>
+                      : (lanes == 4 ? raycast_kernel<Src, false, 4>
+                                    : (lanes == 2 ? raycast_kernel<Src, false, 2> : raycast_kernel<Src, false, 1>));
+  k<<<grid, 64, 0, s>>>(src, tab, p, log_tw, depth, vertex, normal);
 }
 
 void launch_ray_rows(const View& V, hipStream_t s) { launch_ray_prepare(One{V}, nullptr, RayConst{}, 1, s); }
@@ -1093,18 +1256,18 @@ void launch_ray_range_one(const View& V, const RayConst& p, hipStream_t s) {
 }
 
 void launch_raycast_march(const View& V, const RayConst& p, float* depth, float* vertex, float* normal,
-                          hipStream_t s, int shape) {
-  raycast_shaped(One{V}, nullptr, p, p.cam.width, p.cam.height, 1, V.capacity > kNarrowCapacity, shape, depth,
-                 vertex, normal, s);
+                          hipStream_t s, int cus, int shape) {
+  raycast_shaped(One{V}, nullptr, p, p.cam.width, p.cam.height, 1, V.capacity > kNarrowCapacity, shape, cus,
+                 depth, vertex, normal, s);
 }
 
 void launch_raycast(const View& V, const RayConst& p, float* depth, float* vertex, float* normal,
-                    hipStream_t s, const KernelClock* kc, int shape) {
+                    hipStream_t s, int cus, const KernelClock* kc, int shape) {
   tick(kc, s, "ray_range_kernel");
   launch_ray_range(One{V}, nullptr, p, p.tiles, 1, s);
   tick(kc, s, "raycast_kernel");
-  raycast_shaped(One{V}, nullptr, p, p.cam.width, p.cam.height, 1, V.capacity > kNarrowCapacity, shape, depth,
-                 vertex, normal, s);
+  raycast_shaped(One{V}, nullptr, p, p.cam.width, p.cam.height, 1, V.capacity > kNarrowCapacity, shape, cus,
+                 depth, vertex, normal, s);
   tick(kc, s, nullptr);
 }
 
@@ -1139,10 +1302,10 @@ void launch_raycast_backward(const View& V, const RayConst& p, const float* obs,
 }
 
 void launch_batch_raycast(const BatchDev& B, float* depth, float* vertex, float* normal,
-                          hipStream_t s, int shape) {
+                          hipStream_t s, int cus, int shape) {
   launch_ray_range(B.src(), B.frames, RayConst{}, ((B.width + 7) / 8) * ((B.height + 7) / 8), B.nscenes, s);
   raycast_shaped(B.src(), B.frames, RayConst{}, B.width, B.height, B.nscenes, B.max_capacity > kNarrowCapacity, shape,
-                 depth, vertex, normal, s);
+                 cus, depth, vertex, normal, s);
 }
 
 }  // namespace mh
