@@ -139,8 +139,7 @@ struct mh_volume {
   const uint16_t* pending_raw = nullptr;
   const uint8_t* pending_color = nullptr;
   bool have_frame = false;
-  int32_t* pd_nbr = nullptr;
-  uint32_t pd_nbr_cap = 0;
+  PdTables pd{};
   // Bumped by every call that rebuilds or clears the worklist; the
   // primal-dual neighbour table records the value it was built at.
   uint64_t work_gen = 0;
@@ -911,14 +910,17 @@ static int ensure_pd(mh_volume* v) {
   Scratch sc;
   float *s0 = nullptr, *sb = nullptr, *w = nullptr, *p = nullptr;
   uint8_t* m = nullptr;
-  int32_t* nbr = nullptr;
+  PdTables T{};
   double *part = nullptr, *en = nullptr;
   HIP_TRY(sc.get(&s0, nvox));
   HIP_TRY(sc.get(&sb, nvox));
   HIP_TRY(sc.get(&w, nvox));
   HIP_TRY(sc.get(&p, nvox * 3));
   HIP_TRY(sc.get(&m, nvox));
-  HIP_TRY(sc.get(&nbr, (size_t)v->hp.value_capacity * 6));
+  HIP_TRY(sc.get(&T.nbr, (size_t)v->hp.value_capacity * 6));
+  HIP_TRY(sc.get(&T.index, (size_t)v->hp.value_capacity));
+  HIP_TRY(sc.get(&T.bits, nvox / 8));
+  HIP_TRY(sc.get(&T.dual, nvox / 8));
   HIP_TRY(sc.get(&part, (size_t)np * 2));
   HIP_TRY(sc.get(&en, 4));
   HIP_TRY(hipMemsetAsync(m, 0, nvox, v->stream));
@@ -926,6 +928,8 @@ static int ensure_pd(mh_volume* v) {
   HIP_TRY(hipMemsetAsync(sb, 0, nvox * 4, v->stream));
   HIP_TRY(hipMemsetAsync(w, 0, nvox * 4, v->stream));
   HIP_TRY(hipMemsetAsync(p, 0, nvox * 12, v->stream));
+  HIP_TRY(hipMemsetAsync(T.index, 0, (size_t)v->hp.value_capacity * 4, v->stream));
+  HIP_TRY(hipMemsetAsync(T.dual, 0, nvox / 8, v->stream));  // p is +0
   // every buffer exists: publish them together
   sc.release_to(v->owned);
   V.pd_sdf0 = s0;
@@ -933,7 +937,7 @@ static int ensure_pd(mh_volume* v) {
   V.pd_w = w;
   V.pd_p = p;
   V.pd_mask = m;
-  v->pd_nbr = nbr;
+  v->pd = T;
   v->pd_partials = part;
   v->pd_energy = en;
   v->pd_npartials = np;
@@ -944,8 +948,7 @@ int mh_primal_dual_init(mh_volume* v) {
   if (check_vol(v)) return MH_ERR_ARG;
   const int rc = ensure_pd(v);
   if (rc != MH_OK) return rc;
-  launch_pd_neighbors(v->V, v->pd_nbr, v->stream, v->grid_wg256());
-  launch_pd_init(v->V, v->pd_nbr, v->stream, v->grid_wg256());
+  launch_pd_init(v->V, v->pd, v->stream, v->grid_wg256());
   HIP_TRY(hipGetLastError());
   v->pd_work_gen = v->work_gen;
   return MH_OK;
@@ -958,7 +961,7 @@ int mh_primal_dual_iterate(mh_volume* v, float lambda, float sigma, float tau, d
   // call that has rebuilt the worklist since makes it stale.
   if (v->pd_work_gen != v->work_gen)
     return fail(MH_ERR_STATE, "worklist changed since mh_primal_dual_init");
-  launch_pd_iterate(v->V, v->pd_nbr, lambda, sigma, tau, v->pd_partials, v->pd_npartials,
+  launch_pd_iterate(v->V, v->pd, lambda, sigma, tau, v->pd_partials, v->pd_npartials,
                     energy_host ? v->pd_energy : nullptr, v->stream, v->grid_wg256());
   HIP_TRY(hipGetLastError());
   if (energy_host) {

@@ -261,10 +261,17 @@ void launch_point_to_psdf(const View& V, const M4& wTc, int corrected, double* p
                           hipStream_t s);
 
 // primal_dual.hip
-void launch_pd_neighbors(const View& V, int32_t* nbr, hipStream_t s, int grid);
-void launch_pd_init(const View& V, const int32_t* nbr, hipStream_t s, int grid);
+// A solver's tables: the worklist blocks' face neighbours, where a block stands
+// on the worklist, and two bits and one bit a voxel, by block (64 rows each).
+struct PdTables {
+  int32_t* nbr;
+  uint32_t* index;
+  uint16_t* bits;
+  uint8_t* dual;
+};
+void launch_pd_init(const View& V, const PdTables& T, hipStream_t s, int grid);
 // energy: where the three energies go, or null if they are not wanted
-void launch_pd_iterate(const View& V, const int32_t* nbr, float lambda, float sigma, float tau,
+void launch_pd_iterate(const View& V, const PdTables& T, float lambda, float sigma, float tau,
                        double* partials, uint32_t npartials, double* energy, hipStream_t s,
                        int grid);
 
