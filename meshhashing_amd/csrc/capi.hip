@@ -166,6 +166,7 @@ struct mh_volume {
   double* rgrad_partials = nullptr;     // raycast adjoint: per-workgroup sums
   uint32_t rgrad_cap = 0;
   double* rgrad_out = nullptr;
+  LocalizeState* localize = nullptr;
   uint32_t* ray_range = nullptr;        // raycast: camera-z range per 8x8 tile
   uint32_t ray_range_words = 0;
   int tiling = kDefaultIntegrateTiling;  // integration tiling (kIntegrateTilings)
@@ -514,6 +515,7 @@ int mh_volume_destroy(mh_volume* v) {
   for (void* p : v->owned) (void)hipFree(p);
   if (v->rgrad_partials) (void)hipFree(v->rgrad_partials);
   if (v->rgrad_out) (void)hipFree(v->rgrad_out);
+  if (v->localize) (void)hipFree(v->localize);
   if (v->ray_range) (void)hipFree(v->ray_range);
   if (v->ray_mark) (void)hipFree(v->ray_mark);
   for (hipEvent_t e : v->ev_pool) (void)hipEventDestroy(e);
@@ -2161,42 +2163,6 @@ int scratch_address(int dev, unsigned char** out) {
   return MH_OK;
 }
 
-// exp of xi = (omega, upsilon) in se(3) as a row-major 4x4 (Rodrigues, and
-// V = I + (1 - cos)/th^2 W + (th - sin)/th^3 W^2 for the translation).
-void se3_exp(const double xi[6], double T[16]) {
-  const double wx = xi[0], wy = xi[1], wz = xi[2];
-  const double th2 = wx * wx + wy * wy + wz * wz, th = std::sqrt(th2);
-  double A, B, C;
-  if (th < 1e-6) {
-    A = 1.0 - th2 / 6.0;
-    B = 0.5 - th2 / 24.0;
-    C = 1.0 / 6.0 - th2 / 120.0;
-  } else {
-    A = std::sin(th) / th;
-    B = (1.0 - std::cos(th)) / th2;
-    C = (th - std::sin(th)) / (th2 * th);
-  }
-  const double W[9] = {0, -wz, wy, wz, 0, -wx, -wy, wx, 0};
-  double W2[9];
-  for (int i = 0; i < 3; ++i)
-    for (int j = 0; j < 3; ++j) {
-      double a = 0;
-      for (int k = 0; k < 3; ++k) a += W[3 * i + k] * W[3 * k + j];
-      W2[3 * i + j] = a;
-    }
-  for (int i = 0; i < 3; ++i) {
-    double t = 0;
-    for (int j = 0; j < 3; ++j) {
-      const double I = i == j ? 1.0 : 0.0;
-      T[4 * i + j] = I + A * W[3 * i + j] + B * W2[3 * i + j];
-      t += (I + B * W[3 * i + j] + C * W2[3 * i + j]) * xi[3 + j];
-    }
-    T[4 * i + 3] = t;
-  }
-  T[12] = T[13] = T[14] = 0.0;
-  T[15] = 1.0;
-}
-
 void matmul4(const double* a, const double* b, double* c) {
   for (int i = 0; i < 4; ++i)
     for (int j = 0; j < 4; ++j) {
@@ -2377,7 +2343,7 @@ int point_to_psdf(mh_volume* v, const float wTc[16], int jacobian, mh_point_to_p
   M4 T;
   std::memcpy(T.m, wTc, sizeof(T.m));
   launch_point_to_psdf(v->V, T, jacobian == MH_P2S_CORRECTED ? 1 : 0, v->rgrad_partials,
-                       v->rgrad_out, v->stream);
+                       v->rgrad_out, LocalizeStep{}, v->stream, v->cus);
   HIP_TRY(hipGetLastError());
   double h[kP2SSlots];
   HIP_TRY(hipMemcpyAsync(h, v->rgrad_out, sizeof(h), hipMemcpyDeviceToHost, v->stream));
@@ -2415,25 +2381,29 @@ int mh_localize(mh_volume* v, uint32_t iterations, float lambda, int jacobian, f
     return fail(MH_ERR_ARG, "jacobian must be MH_P2S_REFERENCE or MH_P2S_CORRECTED");
   if (!v->have_frame) return fail(MH_ERR_STATE, "no frame uploaded");
   launch_ray_rows(v->V, v->stream);  // no step changes the block set
+  flush_frame(v);
+  HIP_TRY(ensure_partials(v, point_to_psdf_partials(v->V)));
+  if (!v->localize) HIP_TRY(dalloc(&v->localize, 1));
+  M4 T;
+  std::memcpy(T.m, wTc, sizeof(T.m));
   uint32_t it = 0;
-  for (; it < iterations; ++it) {
-    mh_point_to_psdf_result r;
-    const int rc = point_to_psdf(v, wTc, jacobian, &r);
-    if (rc) return rc;
-    if (err_trace) err_trace[it] = r.err;
-    if (count_trace) count_trace[it] = r.count;
-    if (r.count == 0) break;
-    // SolveAndConvertDeltaXi (main_engine.cc:28-54): (A + lambda I) dxi = -b,
-    // dT = exp(dxi) with dxi = (translation, rotation), wTc <- dT wTc.
-    double H[36], x[6];
-    for (int k = 0; k < 36; ++k) H[k] = r.A[k] + (k % 7 == 0 ? (double)lambda : 0.0);
-    if (!solve6(H, r.b, 0.0, x)) break;
-    const double xi[6] = {x[3], x[4], x[5], x[0], x[1], x[2]};
-    double E[16], T[16], Tn[16];
-    se3_exp(xi, E);
-    for (int k = 0; k < 16; ++k) T[k] = wTc[k];
-    matmul4(E, T, Tn);
-    for (int k = 0; k < 16; ++k) wTc[k] = (float)Tn[k];
+  bool done = false;
+  while (it < iterations && !done) {
+    const uint32_t n = std::min(iterations - it, kLocalizeChunk);
+    for (uint32_t k = 0; k < n; ++k)
+      launch_point_to_psdf(v->V, T, jacobian == MH_P2S_CORRECTED ? 1 : 0, v->rgrad_partials, nullptr,
+                           LocalizeStep{v->localize, (double)lambda, k, it + k == 0}, v->stream, v->cus);
+    HIP_TRY(hipGetLastError());
+    LocalizeState st;
+    HIP_TRY(hipMemcpyAsync(&st, v->localize, sizeof(st), hipMemcpyDeviceToHost, v->stream));
+    HIP_TRY(hipStreamSynchronize(v->stream));
+    done = st.done != 0;
+    for (uint32_t k = 0; k < st.steps + (done ? 1u : 0u); ++k) {
+      if (err_trace) err_trace[it + k] = st.err[k];
+      if (count_trace) count_trace[it + k] = st.count[k];
+    }
+    it += st.steps;
+    std::memcpy(wTc, st.wTc, sizeof(st.wTc));
   }
   if (iterations_done) *iterations_done = it;
   set_pose(v, wTc);  // Sensor::set_transform

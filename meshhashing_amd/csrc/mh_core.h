@@ -471,6 +471,42 @@ __device__ __forceinline__ int32_t alloc_block(const View& V) {
   return p;
 }
 
+// exp of xi = (omega, upsilon) in se(3) as a row-major 4x4 (Rodrigues, and
+// V = I + (1 - cos)/th^2 W + (th - sin)/th^3 W^2 for the translation).
+MH_HD void se3_exp(const double xi[6], double T[16]) {
+  const double wx = xi[0], wy = xi[1], wz = xi[2];
+  const double th2 = wx * wx + wy * wy + wz * wz, th = sqrt(th2);
+  double A, B, C;
+  if (th < 1e-6) {
+    A = 1.0 - th2 / 6.0;
+    B = 0.5 - th2 / 24.0;
+    C = 1.0 / 6.0 - th2 / 120.0;
+  } else {
+    A = sin(th) / th;
+    B = (1.0 - cos(th)) / th2;
+    C = (th - sin(th)) / (th2 * th);
+  }
+  const double W[9] = {0, -wz, wy, wz, 0, -wx, -wy, wx, 0};
+  double W2[9];
+  for (int i = 0; i < 3; ++i)
+    for (int j = 0; j < 3; ++j) {
+      double a = 0;
+      for (int k = 0; k < 3; ++k) a += W[3 * i + k] * W[3 * k + j];
+      W2[3 * i + j] = a;
+    }
+  for (int i = 0; i < 3; ++i) {
+    double t = 0;
+    for (int j = 0; j < 3; ++j) {
+      const double I = i == j ? 1.0 : 0.0;
+      T[4 * i + j] = I + A * W[3 * i + j] + B * W2[3 * i + j];
+      t += (I + B * W[3 * i + j] + C * W2[3 * i + j]) * xi[3 + j];
+    }
+    T[4 * i + 3] = t;
+  }
+  T[12] = T[13] = T[14] = 0.0;
+  T[15] = 1.0;
+}
+
 // Local voxel index <-> offset, geometry_helper.h:111-129.
 MH_HD i3 devectorize(uint32_t i) {
   return i3{(int)(i % 8u), (int)((i % 64u) / 8u), (int)(i / 64u)};

@@ -253,12 +253,30 @@ void launch_raycast_backward(const View& V, const RayConst& p, const float* obs,
 // point-to-PSDF normal equations: 29 FP64 sums (A upper triangle[21], b[6],
 // err, count) over the current frame's depth
 constexpr int kP2SSlots = 29;
+// mh_localize's steps run one after another on the device, kLocalizeChunk of
+// them between two looks of the host at this.
+constexpr uint32_t kLocalizeChunk = 32;
+struct LocalizeState {
+  float wTc[16];
+  uint32_t done;   // no further step: no point in sight, or a singular system
+  uint32_t steps;  // of the chunk, taken
+  double err[kLocalizeChunk];
+  uint32_t count[kLocalizeChunk];
+};
+// A step (`slot` of its chunk; the very first starts from a pose by value), or
+// none (st null).
+struct LocalizeStep {
+  LocalizeState* st;
+  double lambda;
+  uint32_t slot;
+  int fresh;
+};
 uint32_t point_to_psdf_partials(const View& V);
 // Fills V.oct, which the point-to-PSDF pass reads (valid until the block set
 // changes).
 void launch_ray_rows(const View& V, hipStream_t s);
 void launch_point_to_psdf(const View& V, const M4& wTc, int corrected, double* partials, double* out,
-                          hipStream_t s);
+                          const LocalizeStep& step, hipStream_t s, int cus);
 
 // primal_dual.hip
 // A solver's tables: the worklist blocks' face neighbours, where a block stands

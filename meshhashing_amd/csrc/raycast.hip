@@ -873,49 +873,80 @@ __global__ __launch_bounds__(64) void raycast_backward_kernel(View V, RayConst R
 // first of its rows; the workgroup that finishes last adds those up the same
 // way.  A lane's chain is then kReduceRows / 8 loads rather than n: a lane
 // per column walking every row took 1135 us for a 640 x 480 image's 4800 rows
-// (71 us for 300 rows) against 9 us (5 us) here.
+// against 9 us here.  Up to kReduceOneRows rows go to one workgroup of 32 rows at
+// a time, whose two round trips are less than the fence, the count and the
+// second stage (a localiser's step with its 300 rows: 10.0 us by eights, 7.2 us).
 constexpr uint32_t kReduceRows = 64;
+constexpr uint32_t kReduceOneRows = 512;
+template <uint32_t kGroups>
 __device__ __forceinline__ double reduce_rows(const double* rows, uint32_t n, size_t stride,
                                               uint32_t slots, double (*red)[32]) {
-  const uint32_t k = threadIdx.x & 31u, g = threadIdx.x >> 5;
+  const uint32_t k = threadIdx.x & 31, g = threadIdx.x >> 5;
   double s = 0.0;
   if (k < slots)
 #pragma unroll 8
-    for (uint32_t i = g; i < n; i += 8) s += rows[i * stride + k];
+    for (uint32_t i = g; i < n; i += kGroups) s += rows[i * stride + k];
   red[g][k] = s;
   __syncthreads();
   double all = 0.0;
 #pragma unroll
-  for (int j = 0; j < 8; ++j) all += red[j][k];
+  for (uint32_t j = 0; j < kGroups; ++j) all += red[j][k];
   __syncthreads();
   return all;
 }
-__global__ __launch_bounds__(256) void slot_reduce_kernel(double* partials, uint32_t n, uint32_t slots,
-                                                          uint32_t* done, double* __restrict__ out) {
-  __shared__ double red[8][32];
+// (-> the whole sum in the first `slots` lanes of one workgroup, true there;
+// kOne: the only workgroup, of 1024 lanes)
+template <bool kOne>
+__device__ __forceinline__ bool slot_reduce(double* partials, uint32_t n, uint32_t slots, uint32_t* done, double* sum) {
+  constexpr uint32_t kGroups = kOne ? 32 : 8;
+  __shared__ double red[kGroups][32];
+  if (kOne) {
+    *sum = reduce_rows<kGroups>(partials, n, slots, slots, red);
+    return true;
+  }
   __shared__ bool last;
   const uint32_t r0 = blockIdx.x * kReduceRows;
   double* const mine = partials + (size_t)r0 * slots;
-  const double s = reduce_rows(mine, min(kReduceRows, n - r0), slots, slots, red);
-  if (threadIdx.x < slots) (gridDim.x == 1 ? out : mine)[threadIdx.x] = s;
-  if (gridDim.x == 1) return;
+  const double s = reduce_rows<kGroups>(mine, min(kReduceRows, n - r0), slots, slots, red);
+  if (threadIdx.x < slots) mine[threadIdx.x] = s;
   __threadfence();  // the row before the count that announces it
   __syncthreads();
   if (threadIdx.x == 0) last = atomicAdd(done, 1u) == gridDim.x - 1;
   __syncthreads();
-  if (!last) return;
+  if (!last) return false;
   __threadfence();  // the other workgroups' rows after their counts
-  const double a = reduce_rows(partials, gridDim.x, (size_t)kReduceRows * slots, slots, red);
-  if (threadIdx.x < slots) out[threadIdx.x] = a;
+  *sum = reduce_rows<kGroups>(partials, gridDim.x, (size_t)kReduceRows * slots, slots, red);
   if (threadIdx.x == 0) *done = 0u;  // for the next call
+  return true;
+}
+inline uint32_t reduce_groups(uint32_t n) { return n <= kReduceOneRows ? 1 : (n + kReduceRows - 1) / kReduceRows; }
+inline uint32_t reduce_lanes(uint32_t n) { return n <= kReduceOneRows ? 1024 : 256; }
+template <bool kOne>
+__global__ __launch_bounds__(kOne ? 1024 : 256) void slot_reduce_kernel(double* partials, uint32_t n, uint32_t slots,
+                                                                         uint32_t* done, double* __restrict__ out) {
+  double a;
+  if (slot_reduce<kOne>(partials, n, slots, done, &a) && threadIdx.x < slots) out[threadIdx.x] = a;
 }
 void launch_slot_reduce(double* partials, uint32_t n, uint32_t slots, uint32_t* done, double* out, hipStream_t s) {
-  slot_reduce_kernel<<<(n + kReduceRows - 1) / kReduceRows, 256, 0, s>>>(partials, n, slots, done, out);
+  const auto k = n <= kReduceOneRows ? slot_reduce_kernel<true> : slot_reduce_kernel<false>;
+  k<<<reduce_groups(n), reduce_lanes(n), 0, s>>>(partials, n, slots, done, out);
+}
+
+// Lanes a ray: an image of few pixels leaves the chip nearly empty, a wave a
+// SIMD at 333 x 251, and each wave's time is the latency of its rays' samples
+// in a row; four (two) lanes a ray then take a quarter (half) of the rounds.
+// As many as fit the chip in one round of waves; past that the extra lanes only
+// add work.  Measured (5 mm desk, whole call, 1 / 2 / 4 lanes): 160 x 120
+// 155 / 128 / 92 us, 320 x 240 138 / 124 / 98, 400 x 300 147 / 130 / 137,
+// 480 x 360 149 / 155 / 152, 640 x 480 142 / 162 / 189.
+inline int ray_lanes(uint64_t pixels, int cus) {
+  const uint64_t waves = (pixels + 63) / 64, room = (uint64_t)kRayWavesPerSimd * 4 * (uint64_t)cus;
+  return 4 * waves <= room ? 4 : (2 * waves <= room ? 2 : 1);
 }
 
 // ------------------------------------------------------------ localisation
-// PointToSurfaceKernel (localizing/point_to_psdf.cu:19-82): one lane per odd
-// pixel (both coordinates odd), 8 x 8 of them per 64-lane workgroup, i.e.
+// PointToSurfaceKernel (localizing/point_to_psdf.cu:19-82): the odd pixels
+// (both coordinates odd), 8 x 8 of them per workgroup, i.e.
 // a 16 x 16 pixel tile as in the reference.  A depth that is -inf, 0 or at
 // least sdf_upper_bound is skipped; the world point wTc * p, the SDF
 // (GetSpatialValue) and its central difference at +-vs/2
@@ -926,16 +957,28 @@ void launch_slot_reduce(double* partials, uint32_t n, uint32_t slots, uint32_t* 
 // mat6x6 arithmetic; they are summed in FP64 per wave and then per
 // workgroup in a fixed order instead of float atomics.  Slots: A's upper
 // triangle (21), b (6), err, count.
-template <bool kWide>
-__global__ __launch_bounds__(64) void point_to_psdf_kernel(View V, M4 wTc, float inv_vs, int corrected,
-                                                           double* __restrict__ partials) {
+//
+// L lanes a point (1 or 4; 64 L lanes a workgroup): a tracked frame's points are
+// a wave or two a SIMD, and the pass then lasts as long as its seven samples in
+// a row; four lanes take the gradient's six in two rounds, and add up eight
+// slots each.  320 x 240 over a 2 cm room: 14 us with one, 10.3 with four.
+template <bool kWide, int L>
+__global__ __launch_bounds__(64 * L) void point_to_psdf_kernel(View V, M4 T0, float inv_vs, int corrected,
+                                                               double* __restrict__ partials, LocalizeStep step) {
+  if (step.st && !step.fresh && step.st->done) return;
   __shared__ WaveTable table;
+  __shared__ double part[L][32];
   wave_table_init(&table);
-  const uint32_t x = 2 * (blockIdx.x * 8 + (threadIdx.x & 7)) + 1;
-  const uint32_t y = 2 * (blockIdx.y * 8 + (threadIdx.x >> 3)) + 1;
-  double acc[kP2SSlots];
+  const uint32_t point = threadIdx.x / L;
+  const uint32_t x = 2 * (blockIdx.x * 8 + (point & 7)) + 1;
+  const uint32_t y = 2 * (blockIdx.y * 8 + (point >> 3)) + 1;
+  M4 wTc = T0;
+  if (step.st && !step.fresh)
 #pragma unroll
-  for (int k = 0; k < kP2SSlots; ++k) acc[k] = 0.0;
+    for (int k = 0; k < 16; ++k) wTc.m[k] = step.st->wTc[k];
+  double acc[32];
+#pragma unroll
+  for (int k = 0; k < 32; ++k) acc[k] = 0.0;
   if (x < V.cam.width && y < V.cam.height) {
     const float depth = V.depth[(size_t)y * V.cam.width + x];
     if (!(depth == -INFINITY || depth == 0.0f || depth >= V.geo.sdf_upper_bound)) {
@@ -944,7 +987,12 @@ __global__ __launch_bounds__(64) void point_to_psdf_kernel(View V, M4 wTc, float
       float d;
       if (point_sample<kWide>(V, &table, oc, pw, inv_vs, &d)) {
         f3 g;
-        if (gradient_samples<kWide>(V, &table, oc, pw, inv_vs, &g.x, &g.y, &g.z)) {
+        bool valid;
+        if constexpr (L == 1)
+          valid = gradient_samples<kWide>(V, &table, oc, pw, inv_vs, &g.x, &g.y, &g.z);
+        else
+          valid = gradient_samples_split<kWide, L>(V, &table, oc, pw, inv_vs, &g.x, &g.y, &g.z);
+        if (valid) {
           const float J[6] = {g.x, g.y, corrected ? g.z : g.x,
                               -g.y * pw.z + g.z * pw.y,
                               -g.z * pw.x + g.x * pw.z,
@@ -962,16 +1010,114 @@ __global__ __launch_bounds__(64) void point_to_psdf_kernel(View V, M4 wTc, float
       }
     }
   }
+  // lane q of a point adds up slots [32 / L * q, 32 / L * (q + 1))
+  constexpr int kOwn = 32 / L;
+  const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, q = lane & (L - 1);
 #pragma unroll
-  for (int k = 0; k < kP2SSlots; ++k) {
+  for (int k = 0; k < (kOwn < kP2SSlots ? kOwn : kP2SSlots); ++k) {
     double v = acc[k];
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-    acc[k] = v;
-  }
-  if (threadIdx.x == 0) {
-    const size_t wg = (size_t)blockIdx.y * gridDim.x + blockIdx.x;
 #pragma unroll
-    for (int k = 0; k < kP2SSlots; ++k) partials[wg * kP2SSlots + k] = acc[k];
+    for (int j = 1; j < L; ++j) v = q == (uint32_t)j ? acc[kOwn * j + k] : v;
+    for (int off = 32; off >= L; off >>= 1) v += __shfl_xor(v, off);
+    if (lane < L) part[wave][kOwn * q + k] = v;
+  }
+  __syncthreads();
+  if (threadIdx.x < kP2SSlots) {
+    const size_t wg = (size_t)blockIdx.y * gridDim.x + blockIdx.x;
+    double s = part[0][threadIdx.x];
+#pragma unroll
+    for (int w = 1; w < L; ++w) s += part[w][threadIdx.x];
+    partials[wg * kP2SSlots + threadIdx.x] = s;
+  }
+}
+
+// SolveAndConvertDeltaXi (main_engine.cc:28-54) on the sums of one step, by one
+// wave: (A + lambda I) dxi = -b, dT = exp(dxi) with dxi = (translation,
+// rotation), wTc <- dT wTc.  Gaussian elimination with partial pivoting, an
+// entry a lane; false if no point was in sight or the matrix is singular.
+__device__ __forceinline__ bool localize_solve(const double* sums, double lambda, float* wTc) {
+  __shared__ double A[6][8], E[16];
+  const uint32_t lane = threadIdx.x, r = lane / 7, j = lane % 7;
+  auto wave_sync = [] { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); };
+  if (sums[28] < 1.0) return false;
+  if (r < 6) {
+    if (j < 6) {
+      const uint32_t lo = min(r, j), hi = max(r, j);
+      const double h = sums[lo * 6 - lo * (lo - 1) / 2 + (hi - lo)] + (r == j ? lambda : 0.0);
+      A[r][j] = h + (r == j ? 0.0 * h : 0.0);  // an infinite diagonal is singular
+    } else {
+      A[r][6] = -sums[21 + r];
+    }
+  }
+  wave_sync();
+  for (uint32_t c = 0; c < 6; ++c) {
+    uint32_t piv = c;
+    for (uint32_t i = c + 1; i < 6; ++i)
+      if (fabs(A[i][c]) > fabs(A[piv][c])) piv = i;
+    if (!(fabs(A[piv][c]) > 0.0)) return false;
+    if (lane < 7) {
+      const double a = A[c][lane], b = A[piv][lane];
+      A[c][lane] = b;
+      A[piv][lane] = a;
+    }
+    wave_sync();
+    if (r > c && r < 6 && j >= c) {
+      const double f = A[r][c] / A[c][c];
+      const double v = A[r][j] - f * A[c][j];
+      wave_sync();
+      A[r][j] = v;
+    }
+    wave_sync();
+  }
+  double x[6];
+#pragma unroll
+  for (int i = 5; i >= 0; --i) {
+    double s = A[i][6];
+#pragma unroll
+    for (int k = i + 1; k < 6; ++k) s -= A[i][k] * x[k];
+    x[i] = s / A[i][i];
+  }
+  const double xi[6] = {x[3], x[4], x[5], x[0], x[1], x[2]};
+  double e[16];
+  se3_exp(xi, e);
+  if (lane == 0)
+#pragma unroll
+    for (int k = 0; k < 16; ++k) E[k] = e[k];
+  wave_sync();
+  if (lane < 16) {
+    double s = 0.0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) s += E[4 * (lane >> 2) + k] * (double)wTc[4 * k + (lane & 3)];
+    wave_sync();
+    wTc[lane] = (float)s;
+  }
+  return true;
+}
+// The sums of a step and the step itself, by the workgroup that finishes them,
+// so that the steps of a call follow each other without the host: 20 of them at
+// 320 x 240 took 810 us with a copy, a wait and a launch from the host between
+// two (17 us each), 417 us so.
+template <bool kOne>
+__global__ __launch_bounds__(kOne ? 1024 : 256) void localize_step_kernel(double* partials, uint32_t n, uint32_t* done, M4 T0,
+                                                            LocalizeStep step) {
+  LocalizeState* const st = step.st;
+  if (!step.fresh && st->done) return;
+  __shared__ double sums[32];
+  __shared__ float wTc[16];
+  double a;
+  if (!slot_reduce<kOne>(partials, n, kP2SSlots, done, &a)) return;
+  if (threadIdx.x < kP2SSlots) sums[threadIdx.x] = a;
+  if (threadIdx.x < 16) wTc[threadIdx.x] = step.fresh ? T0.m[threadIdx.x] : st->wTc[threadIdx.x];
+  __syncthreads();
+  if (threadIdx.x >= 64) return;
+  const bool ok = localize_solve(sums, step.lambda, wTc);
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  if (threadIdx.x < 16) st->wTc[threadIdx.x] = wTc[threadIdx.x];
+  if (threadIdx.x == 0) {
+    st->err[step.slot] = sums[27];
+    st->count[step.slot] = (uint32_t)sums[28];
+    st->done = ok ? 0u : 1u;
+    st->steps = step.slot + (ok ? 1u : 0u);
   }
 }
 
@@ -980,13 +1126,18 @@ uint32_t point_to_psdf_partials(const View& V) {
 }
 
 void launch_point_to_psdf(const View& V, const M4& wTc, int corrected, double* partials, double* out,
-                          hipStream_t s) {
+                          const LocalizeStep& step, hipStream_t s, int cus) {
   const dim3 grid((V.cam.width / 2 + 7) / 8, (V.cam.height / 2 + 7) / 8);
-  if (V.capacity > kNarrowCapacity)
-    point_to_psdf_kernel<true><<<grid, 64, 0, s>>>(V, wTc, 1.0f / V.geo.voxel_size, corrected, partials);
+  const bool wide = V.capacity > kNarrowCapacity;
+  const int lanes = !wide && ray_lanes((uint64_t)grid.x * grid.y * 64, cus) == 4 ? 4 : 1;
+  const auto k = wide ? point_to_psdf_kernel<true, 1> : (lanes == 4 ? point_to_psdf_kernel<false, 4> : point_to_psdf_kernel<false, 1>);
+  k<<<grid, 64 * lanes, 0, s>>>(V, wTc, 1.0f / V.geo.voxel_size, corrected, partials, step);
+  const uint32_t n = grid.x * grid.y;
+  const auto finish = n <= kReduceOneRows ? localize_step_kernel<true> : localize_step_kernel<false>;
+  if (step.st)
+    finish<<<reduce_groups(n), reduce_lanes(n), 0, s>>>(partials, n, &V.ctr->reduce_done, wTc, step);
   else
-    point_to_psdf_kernel<false><<<grid, 64, 0, s>>>(V, wTc, 1.0f / V.geo.voxel_size, corrected, partials);
-  launch_slot_reduce(partials, grid.x * grid.y, kP2SSlots, &V.ctr->reduce_done, out, s);
+    launch_slot_reduce(partials, n, kP2SSlots, &V.ctr->reduce_done, out, s);
 }
 
 __device__ __forceinline__ const RayConst& ray_of(const One&, uint32_t, const RayConst& r) { return r; }
@@ -1224,17 +1375,6 @@ void launch_ray_range(Src src, const SceneFrame* tab, const RayConst& R, uint32_
   }
 }
 
-// Lanes a ray: an image of few pixels leaves the chip nearly empty, a wave a
-// SIMD at 333 x 251, and each wave's time is the latency of its rays' samples
-// in a row; four (two) lanes a ray then take a quarter (half) of the rounds.
-// As many as fit the chip in one round of waves; past that the extra lanes only
-// add work.  Measured (5 mm desk, whole call, 1 / 2 / 4 lanes): 160 x 120
-// 155 / 128 / 92 us, 320 x 240 138 / 124 / 98, 400 x 300 147 / 130 / 137,
-// 480 x 360 149 / 155 / 152, 640 x 480 142 / 162 / 189.
-inline int ray_lanes(uint64_t pixels, int cus) {
-  const uint64_t waves = (pixels + 63) / 64, room = (uint64_t)kRayWavesPerSimd * 4 * (uint64_t)cus;
-  return 4 * waves <= room ? 4 : (2 * waves <= room ? 2 : 1);
-}
 template <class Src>
 void raycast_shaped(Src src, const SceneFrame* tab, const RayConst& p, uint32_t w, uint32_t h, uint32_t nscenes,
                     bool wide, int shape, int cus, float* depth, float* vertex, float* normal, hipStream_t s) {
