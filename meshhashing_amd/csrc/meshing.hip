@@ -197,7 +197,7 @@ __device__ __forceinline__ bool stage_shell(const McConst& mc, const BlockRegs<P
     const bool cube_ok = R.ok[r] && !(fabsf(sd) > mc.sdf_threshold) && (!PSDF || !(rho < mc.rho_min)) &&
                          !(wt < mc.weight_min);
     S.f[s] = (uint8_t)((R.ok[r] ? kShOk : 0) | (cube_ok ? kShCube : 0) | (sd < 0.0f ? kShNeg : 0));
-    S.sdf[s] = sd;
+    S.sdf[s] = R.ok[r] ? sd : NAN;  // a sample with an absent corner is none: NaN
     S.w[s] = wt;
     if (PSDF) {
       S.a[s] = R.va[r];
@@ -210,10 +210,6 @@ __device__ __forceinline__ bool stage_shell(const McConst& mc, const BlockRegs<P
   return keep;
 }
 
-struct SVal {
-  float sdf, a, b;
-};
-
 // One axis of a GetSpatialValue sample (spatial_query.h:23-66) at world
 // coordinate p: the two corner voxels (rounded from p - vs/2 and p + vs/2,
 // exactly as the reference, so ties and negative coordinates pick the same
@@ -225,52 +221,31 @@ struct SAxis {
   float r;
 };
 __device__ __forceinline__ SAxis shell_axis(float p, float vs, float inv_vs, int base) {
-  const float pc = p - 0.5f * vs;
+  SAxis a;
+  corner_pair(p - 0.5f * vs, vs, inv_vs, &a.c0, &a.c1);
+  a.c0 -= base;
+  a.c1 -= base;
   const float q = quotient(p, vs, inv_vs);
-  return SAxis{vox1_quot(pc + 0.0f, vs, inv_vs) - base, vox1_quot(pc + vs, vs, inv_vs) - base, q - floorf(q)};
+  a.r = q - floorf(q);
+  return a;
 }
 
-// GetSpatialValue against the staged shell, from the sample's three axes (full:
-// the Beta parameters too).
-template <bool PSDF>
-__device__ __forceinline__ bool shell_value(const Shell<PSDF>& S, const SAxis& X, const SAxis& Y,
-                                            const SAxis& Z, bool full, SVal* out, bool* oob) {
+// GetSpatialValue against a staged field, from the sample's three axes; `in`:
+// its corners lie in the shell (local -1..9).
+__device__ __forceinline__ bool axes_in(const SAxis& X, const SAxis& Y, const SAxis& Z) {
+  return min(min(min(X.c0, X.c1), min(Y.c0, Y.c1)), min(Z.c0, Z.c1)) >= -1 &&
+         max(max(max(X.c0, X.c1), max(Y.c0, Y.c1)), max(Z.c0, Z.c1)) <= 9;
+}
+__device__ __forceinline__ float shell_value(const float* f, const SAxis& X, const SAxis& Y, const SAxis& Z) {
   const int cx[2] = {X.c0, X.c1}, cy[2] = {Y.c0, Y.c1}, cz[2] = {Z.c0, Z.c1};
-  const float rx = X.r, ry = Y.r, rz = Z.r;
-  // Straight-line evaluation of all 8 corners (no early exit: a missing
-  // corner makes the result invalid, and the sums are then discarded).
-  const bool in = cx[0] >= -1 && cx[1] <= 9 && cy[0] >= -1 && cy[1] <= 9 && cz[0] >= -1 && cz[1] <= 9 &&
-                  cx[1] >= -1 && cx[0] <= 9 && cy[1] >= -1 && cy[0] <= 9 && cz[1] >= -1 && cz[0] <= 9;
-  if (!in) {
-    *oob = true;
-    return false;
-  }
-  bool ok = true;
-  float sdf = 0.0f;
+  float v = 0.0f;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const int mx = (i >> 2) & 1, my = (i >> 1) & 1, mz = i & 1;
-    const int s = sidx(cx[mx], cy[my], cz[mz]);
-    ok = ok && (S.f[s] & kShOk);
-    const float w = (mx ? rx : 1.0f - rx) * (my ? ry : 1.0f - ry) * (mz ? rz : 1.0f - rz);
-    sdf += w * S.sdf[s];
+    const float w = (mx ? X.r : 1.0f - X.r) * (my ? Y.r : 1.0f - Y.r) * (mz ? Z.r : 1.0f - Z.r);
+    v += w * f[sidx(cx[mx], cy[my], cz[mz])];
   }
-  out->sdf = sdf;
-  out->a = out->b = 0.0f;
-  if (PSDF && full) {
-    float a = 0.0f, b = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int mx = (i >> 2) & 1, my = (i >> 1) & 1, mz = i & 1;
-      const int s = sidx(cx[mx], cy[my], cz[mz]);
-      const float w = (mx ? rx : 1.0f - rx) * (my ? ry : 1.0f - ry) * (mz ? rz : 1.0f - rz);
-      a += w * S.a[s];
-      b += w * S.b[s];
-    }
-    out->a = a;
-    out->b = b;
-  }
-  return ok;
+  return v;
 }
 
 // ValToRGB (color_util.h:13-37); the 0.25/0.5/0.75 literals are doubles
@@ -330,32 +305,45 @@ __device__ __forceinline__ int cidx(int x, int y, int z) {
 constexpr uint32_t kQueue = 2 * kMcLanes;
 
 // Payload of vertex (owner voxel at local (key & 15, key >> 4 & 15,
-// key >> 8 & 15), axis key >> 12) into vertex record vp: VertexIntersection
-// (marching_cubes.cu:16-28) in the canonical endpoint order, then
-// AllocateVertexWithMutex's payload (:45-72), spread over eight lanes per
-// vertex, so that a vertex costs the latency of one trilinear sample instead of
-// seven in a row: lanes 0-5 take the gradient stencils p -+ h e_k (k = sub / 2;
-// odd: +h), lane 6 the full sample at p (radius, colour); each lane samples
-// one point, the stencils sharing all but one coordinate with p (p -+ 0 = p).
-// The eight corner radii of lane 6's cell are taken one per lane.  Stencil
-// values, validities and corner radii meet in LDS (pay_s, pay_ok, pay_r, the
-// vertex's row), from which lanes 0 and 6 finish the record after the
-// workgroup barrier (finish_normal, finish_sample).
-struct PaySample {  // lane 6's sample
-  float rx, ry, rz, a, b;
-  bool ok;
-};
+// key >> 8 & 15), axis key >> 12): VertexIntersection (marching_cubes.cu:16-28)
+// in the canonical endpoint order, then AllocateVertexWithMutex's payload
+// (:45-72).  Four lanes sample a vertex: lanes 0-2 the gradient stencils p -+ h e_k
+// of an axis each, which share two axes with p, lane 3 the ratios of p itself
+// (p -+ 0 = p), and each two of the eight corner radii of lane 3's cell.  What they
+// found meets in LDS, a row a value (Payload), and one lane a vertex each then
+// takes the normal from it (finish_normal) and the radius and colour
+// (finish_sample).
+//
+// The pass is bound by the instructions it issues (VALU busy three quarters of
+// the time), so the lanes that share a vertex are few and the record's end,
+// with its divisions and square roots, has 64 vertices a wave.  Eight lanes a
+// vertex, two of which also finished the record (eight vertices a wave there),
+// took 9140 wave instructions a block of 64 rooms' pass (1385 us); 7940 so (1245
+// us), and a 320 x 240 room's frame 62 us instead of 71.
+constexpr uint32_t kPayRound = kMcLanes / 4;
+constexpr uint32_t kPayPitch = kPayRound + 16;  // the four lanes' rows in other banks
+enum PayRow { kPayS = 0, kPayR = 6, kPayRatio = 14, kPayPos = 17, kPayOk = 20, kPayA = 21, kPayB = 22 };
 template <bool PSDF>
-__device__ __forceinline__ bool payload_part(const Shell<PSDF>& S, const View& V, const McConst& mc, float inv_vs,
-                                             i3 base, uint32_t key, int32_t vp, uint32_t sub, float* pay_s,
-                                             float* pay_r, uint8_t* pay_ok, PaySample* out) {
-  bool oob = false;
-  const Geo& g = V.geo;
+struct Payload {
+  float v[PSDF ? 23 : 21][kPayPitch];
+};
+// The value of lane 3 of four.
+__device__ __forceinline__ uint32_t quad_last(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0xFF, 0xF, 0xF, true);
+}
+template <int CTRL>
+__device__ __forceinline__ uint32_t quad_swap(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xF, 0xF, true);
+}
+// Lane sub's part for vertex j of the round; true if a sample lies outside the shell.
+template <bool PSDF>
+__device__ __forceinline__ bool payload_part(const Shell<PSDF>& S, const Geo& g, const McConst& mc, float inv_vs,
+                                             i3 base, uint32_t key, uint32_t sub, uint32_t j, Payload<PSDF>& P) {
   const float vs = g.voxel_size;
   const int ox = (int)(key & 15u), oy = (int)((key >> 4) & 15u), oz = (int)((key >> 8) & 15u);
   const int ax = (int)(key >> 12);
-  const float vA = S.sdf[sidx(ox, oy, oz)];
-  const float vB = S.sdf[sidx(ox + (ax == 0), oy + (ax == 1), oz + (ax == 2))];
+  const int sA = sidx(ox, oy, oz);
+  const float vA = S.sdf[sA], vB = S.sdf[sA + (ax == 0 ? 1 : (ax == 1 ? kShell : kShell * kShell))];
   const f3 pA = voxel_to_world(g, i3{base.x + ox, base.y + oy, base.z + oz});
   const f3 pB = mk3(pA.x + (ax == 0 ? vs : 0.0f), pA.y + (ax == 1 ? vs : 0.0f), pA.z + (ax == 2 ? vs : 0.0f));
   f3 p;
@@ -367,69 +355,95 @@ __device__ __forceinline__ bool payload_part(const Shell<PSDF>& S, const View& V
     const float mu = (0.0f - vA) / (vB - vA);
     p = mk3(pA.x + mu * (pB.x - pA.x), pA.y + mu * (pB.y - pA.y), pA.z + mu * (pB.z - pA.z));
   }
-  if (sub == 6) {
-    V.vertices[vp].px = p.x;
-    V.vertices[vp].py = p.y;
-    V.vertices[vp].pz = p.z;
-  }
   const float h = 0.5f * vs;
-  const float d = (sub & 1u) ? h : -h;
-  const uint32_t k = sub >> 1;
-  const SAxis X = shell_axis(k == 0 ? p.x + d : p.x, vs, inv_vs, base.x);
-  const SAxis Y = shell_axis(k == 1 ? p.y + d : p.y, vs, inv_vs, base.y);
-  const SAxis Z = shell_axis(k == 2 ? p.z + d : p.z, vs, inv_vs, base.z);
-  SVal q{};
-  // lanes 6 and 7 (k = 3) sample p itself, lane 7 for nothing
-  const bool ok = shell_value<PSDF>(S, X, Y, Z, sub == 6, &q, &oob);
-  pay_s[sub] = q.sdf;
-  pay_ok[sub] = ok ? 1 : 0;
-  // lane 6's cell, corner coordinates + 1 in 4 bits each (valid: all in 0..10)
+  // the first stencil's axes (lane 3: p's), and the one that the second differs in
+  SAxis X = shell_axis(sub == 0 ? p.x - h : p.x, vs, inv_vs, base.x);
+  SAxis Y = shell_axis(sub == 1 ? p.y - h : p.y, vs, inv_vs, base.y);
+  SAxis Z = shell_axis(sub == 2 ? p.z - h : p.z, vs, inv_vs, base.z);
+  bool oob = !axes_in(X, Y, Z);
+  // lane 3's cell, corner coordinates + 1 in 4 bits each (inside: all in 0..10)
   const uint32_t cell = (uint32_t)(X.c0 + 1) | ((uint32_t)(X.c1 + 1) << 4) | ((uint32_t)(Y.c0 + 1) << 8) |
                         ((uint32_t)(Y.c1 + 1) << 12) | ((uint32_t)(Z.c0 + 1) << 16) | ((uint32_t)(Z.c1 + 1) << 20);
-  const uint32_t c6 = (uint32_t)__shfl((int)(ok ? cell : ~0u), 6, 8);
-  if (c6 != ~0u) {
-    const uint32_t cx = (c6 >> ((sub & 4u) ? 4 : 0)) & 15u, cy = (c6 >> ((sub & 2u) ? 12 : 8)) & 15u,
-                   cz = (c6 >> ((sub & 1u) ? 20 : 16)) & 15u;
-    pay_r[sub] = sqrtf(1.0f / S.w[cx + kShell * cy + kShell * kShell * cz]);
+  const uint32_t c3 = quad_last(oob ? ~0u : cell);
+  uint32_t ok = c3 != ~0u ? kShOk : 0u;
+  if (c3 != ~0u) {
+    const uint32_t cx = (c3 >> ((sub & 2u) ? 4 : 0)) & 15u, cy = (c3 >> ((sub & 1u) ? 12 : 8)) & 15u;
+#pragma unroll
+    for (uint32_t i = 0; i < 2; ++i) {  // corners 2 sub and 2 sub + 1
+      const uint32_t s = cx + kShell * cy + kShell * kShell * ((c3 >> (i ? 20 : 16)) & 15u);
+      ok &= S.f[s];
+      P.v[kPayR + 2 * sub + i][j] = sqrtf(1.0f / S.w[s]);
+    }
   }
-  *out = PaySample{X.r, Y.r, Z.r, q.a, q.b, ok};
+  ok &= quad_swap<0xB1>(ok);
+  ok &= quad_swap<0x4E>(ok);
+  if (sub == 3) {
+    P.v[kPayRatio][j] = X.r;
+    P.v[kPayRatio + 1][j] = Y.r;
+    P.v[kPayRatio + 2][j] = Z.r;
+    P.v[kPayPos][j] = p.x;
+    P.v[kPayPos + 1][j] = p.y;
+    P.v[kPayPos + 2][j] = p.z;
+    P.v[kPayOk][j] = ok ? 1.0f : 0.0f;
+    if (PSDF && ok) {
+      P.v[kPayA][j] = shell_value(S.a, X, Y, Z);
+      P.v[kPayB][j] = shell_value(S.b, X, Y, Z);
+    }
+  } else {
+#pragma unroll 1
+    for (uint32_t i = 0;; ++i) {
+      P.v[kPayS + 2 * sub + i][j] = axes_in(X, Y, Z) ? shell_value(S.sdf, X, Y, Z) : NAN;
+      if (i) break;
+      const SAxis A = sub == 0 ? shell_axis(p.x + h, vs, inv_vs, base.x)
+                               : (sub == 1 ? shell_axis(p.y + h, vs, inv_vs, base.y) : shell_axis(p.z + h, vs, inv_vs, base.z));
+      if (sub == 0) X = A;
+      if (sub == 1) Y = A;
+      if (sub == 2) Z = A;
+      oob = oob || !axes_in(X, Y, Z);
+    }
+  }
   return oob;
 }
 
-// Lane 6's part of the record after the exchange: radius and colour.
-__device__ __forceinline__ void finish_sample(const View& V, int32_t vp, const PaySample& q, const float* pay_r) {
+// Position, radius and colour of vertex j of the round.
+template <bool PSDF>
+__device__ __forceinline__ void finish_sample(const View& V, int32_t vp, uint32_t j, const Payload<PSDF>& P) {
   float radius = 0.0f, cr = 0.0f, cg = 0.0f, cb = 0.0f;  // the reference reads an uninitialised query here
-  if (q.ok) {
+  if (P.v[kPayOk][j] != 0.0f) {
+    const float rx = P.v[kPayRatio][j], ry = P.v[kPayRatio + 1][j], rz = P.v[kPayRatio + 2][j];
     float rad = 0.0f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      const float w = ((i & 4) ? q.rx : 1.0f - q.rx) * ((i & 2) ? q.ry : 1.0f - q.ry) * ((i & 1) ? q.rz : 1.0f - q.rz);
-      rad += w * pay_r[i];
+      const float w = ((i & 4) ? rx : 1.0f - rx) * ((i & 2) ? ry : 1.0f - ry) * ((i & 1) ? rz : 1.0f - rz);
+      rad += w * P.v[kPayR + i][j];
     }
     const float inv_sigma2 = 1.0f / (rad * rad);
     radius = sqrtf(1.0f / inv_sigma2);
-    const f3 c = val_to_rgb(q.a / (q.a + q.b), 0.4f, 1.0f);
+    const float a = PSDF ? P.v[PSDF ? kPayA : 0][j] : 0.0f, b = PSDF ? P.v[PSDF ? kPayB : 0][j] : 0.0f;
+    const f3 c = val_to_rgb(a / (a + b), 0.4f, 1.0f);
     cr = c.x;
     cg = c.y;
     cb = c.z;
   }
   Vertex* dst = &V.vertices[vp];
+  dst->px = P.v[kPayPos][j];
+  dst->py = P.v[kPayPos + 1][j];
+  dst->pz = P.v[kPayPos + 2][j];
   dst->radius = radius;
   dst->cr = cr;
   dst->cg = cg;
   dst->cb = cb;
 }
 
-// GetSpatialSDFGradient's normal from the six stencil values of a vertex
-// (pay_s: -x, +x, -y, +y, -z, +z); any invalid sample zeroes it, which is
-// what the reference's short-circuit produces.
-__device__ __forceinline__ void finish_normal(const View& V, int32_t vp, const float* pay_s,
-                                              const uint8_t* pay_ok) {
+// GetSpatialSDFGradient's normal from the six stencil values of a vertex (-x,
+// +x, -y, +y, -z, +z).  An invalid sample, which is NaN, zeroes it, which is what
+// the reference's short-circuit produces.
+template <bool PSDF>
+__device__ __forceinline__ void finish_normal(const View& V, int32_t vp, uint32_t j, const Payload<PSDF>& P) {
   const float vs = V.geo.voxel_size;
-  const bool valid = pay_ok[0] && pay_ok[1] && pay_ok[2] && pay_ok[3] && pay_ok[4] && pay_ok[5];
-  const f3 grad = mk3((pay_s[1] - pay_s[0]) / vs, (pay_s[3] - pay_s[2]) / vs, (pay_s[5] - pay_s[4]) / vs);
+  const f3 grad = mk3((P.v[1][j] - P.v[0][j]) / vs, (P.v[3][j] - P.v[2][j]) / vs, (P.v[5][j] - P.v[4][j]) / vs);
   const float l = length(grad);
-  const f3 n = (l > 0.0f && valid) ? grad / l : mk3(0.0f, 0.0f, 0.0f);
+  const f3 n = l > 0.0f ? grad / l : mk3(0.0f, 0.0f, 0.0f);
   Vertex* dst = &V.vertices[vp];
   dst->nx = n.x;
   dst->ny = n.y;
@@ -546,10 +560,7 @@ __global__ __launch_bounds__(kMcLanes, PSDF ? 3 : 4) void mc_surfel_kernel(Src s
   uint16_t* const items = reinterpret_cast<uint16_t*>(region);  // up to 12 per cube
   uint8_t* const hcfg = reinterpret_cast<uint8_t*>(region);
   static_assert(sizeof(region) >= 12 * kBlockVoxels * sizeof(uint16_t) && sizeof(region) >= kCfg * kCfg * kCfg, "region");
-  // the payload exchange (eight lanes per vertex, kPayRound vertices a round)
-  constexpr uint32_t kPayRound = kMcLanes / 8;
-  __shared__ float pay_s[kPayRound * 8], pay_r[kPayRound * 8];
-  __shared__ uint8_t pay_ok[kPayRound * 8];
+  __shared__ Payload<PSDF> pay;
   __shared__ uint32_t nitems;
   // per-configuration crossed edges and triangle counts, read per lane with
   // divergent indices: from LDS rather than the constant tables
@@ -563,7 +574,7 @@ __global__ __launch_bounds__(kMcLanes, PSDF ? 3 : 4) void mc_surfel_kernel(Src s
   }
   for (int s = (int)threadIdx.x; s < kShellN; s += (int)kMcLanes) code[s] = (uint16_t)shell_code(s);
   McCounts cnt;
-  uint32_t cur_scene = ~0u;
+  uint32_t cur_scene = ~0u, turns = 0;
   // items: ci at work, nx next (its loads under way), the one after it in
   // next_; lanes kLookupLane + t hold neighbour t's table entry of item nx
   const uint32_t nb_lane = threadIdx.x - kLookupLane;
@@ -879,20 +890,22 @@ __global__ __launch_bounds__(kMcLanes, PSDF ? 3 : 4) void mc_surfel_kernel(Src s
       }
       const bool last = c0 + kMcLanes >= n_items;  // uniform
       if (!last && qn + kMcLanes <= kQueue) continue;
-      // payloads, eight lanes per vertex
+      // payloads, four lanes per vertex, kPayRound vertices a round; then a wave
+      // for their normals and one for the rest (other waves each time)
       const uint32_t nq = qn;
       cnt.writes += nq;
-      const uint32_t jl = threadIdx.x >> 3, sub = threadIdx.x & 7u;
-      for (uint32_t j0 = 0; j0 < nq; j0 += kPayRound) {  // uniform
+      const uint32_t jl = threadIdx.x >> 2, lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+      for (uint32_t j0 = 0; j0 < nq; j0 += kPayRound, turns += 2) {  // uniform
         const uint32_t j = j0 + jl;
-        const bool act = j < nq;  // the same for a vertex's eight lanes
-        PaySample q;
-        if (act && payload_part<PSDF>(S, V, mc, inv_vs, base, qkey[j], qptr[j], sub, &pay_s[8 * jl], &pay_r[8 * jl],
-                                      &pay_ok[8 * jl], &q))
+        if (j < nq &&  // the same for a vertex's four lanes
+            payload_part<PSDF>(S, V.geo, mc, inv_vs, base, qkey[j], threadIdx.x & 3u, jl, pay))
           flag(V, MH_STATUS_STENCIL_RANGE);
         __syncthreads();
-        if (act && sub == 0) finish_normal(V, qptr[j], &pay_s[8 * jl], &pay_ok[8 * jl]);
-        if (act && sub == 6) finish_sample(V, qptr[j], q, &pay_r[8 * jl]);
+        const uint32_t role = (wave + turns) & 3u;
+        if (j0 + lane < nq) {
+          if (role == 0) finish_normal<PSDF>(V, qptr[j0 + lane], lane, pay);
+          if (role == 1) finish_sample<PSDF>(V, qptr[j0 + lane], lane, pay);
+        }
         __syncthreads();
       }
       if (last) break;
