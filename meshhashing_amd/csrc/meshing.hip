@@ -26,6 +26,7 @@ __constant__ McTables kMc = build_mc_tables();
 
 constexpr int kShell = 11;
 constexpr int kShellN = kShell * kShell * kShell;
+constexpr int kShellWords = 48;  // 32 of its bits each, the whole waves that stage it
 
 template <bool PSDF>
 struct Shell {
@@ -33,12 +34,12 @@ struct Shell {
   float w[kShellN];
   float a[PSDF ? kShellN : 1];
   float b[PSDF ? kShellN : 1];
-  uint8_t f[kShellN];  // kShOk | kShCube | kShNeg per voxel
+  // Three bit strings over the shell's voxels (bit sidx): the SDF is negative;
+  // the voxel passes the cube tests of a corner (|sdf| <= threshold,
+  // rho >= rho_min, weight >= weight_min); it exists (its block is allocated).
+  alignas(16) uint32_t bits[3][kShellWords];
 };
-// Shell voxel flags: the voxel exists (its block is allocated); it passes
-// the cube tests of a corner (|sdf| <= threshold, rho >= rho_min,
-// weight >= weight_min); its SDF is negative.
-constexpr uint8_t kShOk = 1, kShCube = 2, kShNeg = 4;
+enum ShellBits { kNeg = 0, kCorner = 1, kThere = 2 };
 
 __device__ __forceinline__ int sidx(int x, int y, int z) {
   return (x + 1) + kShell * (y + 1) + kShell * kShell * (z + 1);
@@ -48,6 +49,12 @@ __device__ __forceinline__ int nb27(int dx, int dy, int dz) {
 }
 
 constexpr int kCfg = 9;  // local cube coordinates -1..7
+// 32 bits of a shell bit string from bit `at` on.  A row of the shell is eleven
+// of them, the next row (y + 1) follows, the next layer (z + 1) begins 121 on.
+__device__ __forceinline__ uint32_t shell_bits(const uint32_t* b, uint32_t at) {
+  const uint32_t w = at >> 5;
+  return __builtin_amdgcn_alignbit(b[w + 1], b[w], at & 31u);
+}
 
 // The edge with owner offset (dx, dy, dz) and axis ax (a constant for
 // constant arguments).
@@ -181,29 +188,35 @@ __device__ __forceinline__ void load_block(const View& V, int32_t ptr, const int
 // meshed in this pass (its stored configurations count then).  A block of
 // which no lane says so is done: its cubes are all 0 and it has no surfels.
 template <bool PSDF>
-__device__ __forceinline__ bool stage_shell(const McConst& mc, const BlockRegs<PSDF>& R, const int32_t* row,
-                                            const uint16_t* code, Shell<PSDF>& S) {
-  const uint32_t t = threadIdx.x - kLookupLane;
+__device__ __forceinline__ bool stage_shell(const McConst& mc, const BlockRegs<PSDF>& R, const uint16_t* code,
+                                            Shell<PSDF>& S) {
   bool keep = false;
-  if (t < 27 && t % 3 < 2 && (t / 3) % 3 < 2 && t / 9 < 2) keep = row[t] >= 0 && !row_meshed(row[t]);
 #pragma unroll
   for (int r = 0; r < kShellPer; ++r) {
     const int s = (int)(threadIdx.x + kMcLanes * r);
-    if (s >= kShellN) continue;
-    // the corner tests of IsValid (marching_cubes.cu:96-130), once per
-    // voxel here instead of once per cube corner
-    const float sd = R.sd[r], wt = R.wt[r];
-    const float rho = PSDF ? R.va[r] / (R.va[r] + R.vb[r]) : 0.0f;
-    const bool cube_ok = R.ok[r] && !(fabsf(sd) > mc.sdf_threshold) && (!PSDF || !(rho < mc.rho_min)) &&
-                         !(wt < mc.weight_min);
-    S.f[s] = (uint8_t)((R.ok[r] ? kShOk : 0) | (cube_ok ? kShCube : 0) | (sd < 0.0f ? kShNeg : 0));
-    S.sdf[s] = R.ok[r] ? sd : NAN;  // a sample with an absent corner is none: NaN
-    S.w[s] = wt;
-    if (PSDF) {
-      S.a[s] = R.va[r];
-      S.b[s] = R.vb[r];
+    bool neg = false, corner = false, there = false;
+    if (s < kShellN) {
+      // the corner tests of IsValid (marching_cubes.cu:96-130), once per
+      // voxel here instead of once per cube corner
+      const float sd = R.sd[r], wt = R.wt[r];
+      const float rho = PSDF ? R.va[r] / (R.va[r] + R.vb[r]) : 0.0f;
+      const bool cube_ok = R.ok[r] && !(fabsf(sd) > mc.sdf_threshold) && (!PSDF || !(rho < mc.rho_min)) &&
+                           !(wt < mc.weight_min);
+      neg = sd < 0.0f;
+      corner = cube_ok;
+      there = R.ok[r];
+      S.sdf[s] = R.ok[r] ? sd : NAN;  // a sample with an absent corner is none: NaN
+      S.w[s] = wt;
+      if (PSDF) {
+        S.a[s] = R.va[r];
+        S.b[s] = R.vb[r];
+      }
+      keep = keep || (neg && (code[s] & kCodeInner));
     }
-    keep = keep || (sd < 0.0f && (code[s] & kCodeInner));
+    const uint64_t bn = __ballot(neg), bc = __ballot(corner), bt = __ballot(there);
+    const uint32_t lane = threadIdx.x & 63u;
+    if (lane < 3)
+      reinterpret_cast<uint64_t*>(S.bits[lane])[kMcLanes / 64 * r + (threadIdx.x >> 6)] = lane == 0 ? bn : (lane == 1 ? bc : bt);
   }
 #pragma unroll
   for (int r = 0; r < kMcVox; ++r) keep = keep || R.vps[r][0] >= 0 || R.vps[r][1] >= 0 || R.vps[r][2] >= 0;
@@ -273,31 +286,35 @@ __device__ __forceinline__ f3 val_to_rgb(float v, float vmin, float vmax) {
 }
 
 // ---------------------------------------------------------------- pass 1
-// Corner checks of the cube at local voxel (x, y, z) (marching_cubes.cu:
-// 96-130): every corner must exist, |sdf| <= threshold, rho >= rho_min and
-// weight >= weight_min; returns validity and the cube index.
-template <bool PSDF>
-__device__ __forceinline__ bool cube_index(const Shell<PSDF>& S, int x, int y, int z, int* cube) {
-  // The corners' flags (tested once per voxel when the shell was staged),
-  // all eight read without early exits, so the lanes of a wave do not
-  // diverge on which corner fails first.
-  int c = 0;
-  uint32_t all = kShCube;
-#pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    const uint32_t fl = S.f[sidx(x + corner_off(k, 0), y + corner_off(k, 1), z + corner_off(k, 2))];
-    all &= fl;
-    c |= (int)((fl >> 2) & 1u) << k;
-  }
-  *cube = c;
-  return all != 0;
+// A cube of a block, from the shell's bits: `a` those of its layer from its own
+// voxel on (0 and 1 its two corners there, 11 and 12 those of the next row), `b`
+// those of the next layer.
+constexpr uint32_t kCubeBits = 0x1803u;
+__device__ __forceinline__ uint32_t cube_of(uint32_t a, uint32_t b) {
+  // corners 0-7 (corner_off): 011 111 110 010 001 101 100 000
+  const uint32_t swap = 0xD8u;  // two bits exchanged: 0, 2, 1, 3
+  return ((b >> 11) & 3u) | ((swap >> (2 * ((a >> 11) & 3u))) & 3u) << 2 | (b & 3u) << 4 | ((swap >> (2 * (a & 3u))) & 3u) << 6;
 }
+constexpr bool corner_order_is(int i, int x, int y, int z) {
+  return corner_off(i, 0) == x && corner_off(i, 1) == y && corner_off(i, 2) == z;
+}
+static_assert(corner_order_is(0, 0, 1, 1) && corner_order_is(1, 1, 1, 1) && corner_order_is(2, 1, 1, 0) &&
+                  corner_order_is(3, 0, 1, 0) && corner_order_is(4, 0, 0, 1) && corner_order_is(5, 1, 0, 1) &&
+                  corner_order_is(6, 1, 0, 0) && corner_order_is(7, 0, 0, 0),
+              "cube_of");
+// A configuration uses exactly the edges whose ends differ in sign.
+constexpr bool edges_are_crossings() {
+  const McTables t = build_mc_tables();
+  for (int c = 0; c < 256; ++c)
+    for (int e = 0; e < 12; ++e)
+      if (((t.edges[c] >> e) & 1) != (((c >> edge_a(e)) ^ (c >> edge_b(e))) & 1)) return false;
+  return true;
+}
+static_assert(edges_are_crossings(), "an edge is used where its ends differ in sign");
 
-// Cubes at local coordinates -1..8 (10^3), for the writer rule below.
+// Cubes at local coordinates -1..8: a row of ten bits for each y, z.
 constexpr int kCubeHalo = 10;
-__device__ __forceinline__ int cidx(int x, int y, int z) {
-  return (x + 1) + kCubeHalo * (y + 1) + kCubeHalo * kCubeHalo * (z + 1);
-}
+__device__ __forceinline__ int crow(int y, int z) { return (y + 1) + kCubeHalo * (z + 1); }
 
 // The surfel pass queues a block's vertex writes in LDS (a block with surface
 // writes ~80): a round of slot claims adds at most one per lane, and the queue
@@ -365,13 +382,13 @@ __device__ __forceinline__ bool payload_part(const Shell<PSDF>& S, const Geo& g,
   const uint32_t cell = (uint32_t)(X.c0 + 1) | ((uint32_t)(X.c1 + 1) << 4) | ((uint32_t)(Y.c0 + 1) << 8) |
                         ((uint32_t)(Y.c1 + 1) << 12) | ((uint32_t)(Z.c0 + 1) << 16) | ((uint32_t)(Z.c1 + 1) << 20);
   const uint32_t c3 = quad_last(oob ? ~0u : cell);
-  uint32_t ok = c3 != ~0u ? kShOk : 0u;
+  uint32_t ok = c3 != ~0u ? 1u : 0u;
   if (c3 != ~0u) {
     const uint32_t cx = (c3 >> ((sub & 2u) ? 4 : 0)) & 15u, cy = (c3 >> ((sub & 1u) ? 12 : 8)) & 15u;
 #pragma unroll
     for (uint32_t i = 0; i < 2; ++i) {  // corners 2 sub and 2 sub + 1
       const uint32_t s = cx + kShell * cy + kShell * kShell * ((c3 >> (i ? 20 : 16)) & 15u);
-      ok &= S.f[s];
+      ok &= S.bits[kThere][s >> 5] >> (s & 31u);
       P.v[kPayR + 2 * sub + i][j] = sqrtf(1.0f / S.w[s]);
     }
   }
@@ -520,16 +537,6 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* wave_s
   return block_excl_scan_planes<(1u << BITS) - 1u>(v, wave_sums, total);
 }
 
-// Vertex slot of edge e of the cube at local voxel o: the slot of the edge's
-// owner voxel (o + the edge's owner offset, possibly in a +x/+y/+z neighbour).
-__device__ __forceinline__ int32_t* edge_slot(const View& V, const int32_t* nb, i3 o, int e) {
-  const int ox = o.x + edge_owner_off(e, 0), oy = o.y + edge_owner_off(e, 1), oz = o.z + edge_owner_off(e, 2);
-  const int dx = ox >> 3, dy = oy >> 3, dz = oz >> 3;
-  const int32_t optr = row_ptr(nb[nb27(dx, dy, dz)]);
-  const uint32_t oi = (uint32_t)((ox - 8 * dx) + 8 * (oy - 8 * dy) + 64 * (oz - 8 * dz));
-  return &V.vptr[((size_t)optr * kBlockVoxels + oi) * 3 + edge_axis(e)];
-}
-
 template <bool PSDF, class Src>
 __global__ __launch_bounds__(kMcLanes, PSDF ? 3 : 4) void mc_surfel_kernel(Src src_, const SceneFrame* __restrict__ tab, McConst mc1,
                                                                 const int32_t* __restrict__ nbt, uint32_t static_q) {
@@ -537,14 +544,15 @@ __global__ __launch_bounds__(kMcLanes, PSDF ? 3 : 4) void mc_surfel_kernel(Src s
   __shared__ Shell<PSDF> S;
   __shared__ uint16_t code[kShellN];
   __shared__ int32_t row_[2][27];  // the neighbour-table rows of the block at work and of the next one
-  __shared__ uint8_t cv[kCubeHalo * kCubeHalo * kCubeHalo];
+  // the halo's cubes that are valid and belong to a block meshed in this pass
+  __shared__ uint16_t cv[kCubeHalo * kCubeHalo];
   __shared__ int surfels[2];
   __shared__ int tri_sum[2];  // the block's change of live triangles, and the triangles of its changed cubes
   // Flags of a block, three in turn: a block without surface ends without a
   // further barrier, so a fast wave may set the next block's while a slow one
   // still reads this one's; after a block's first barrier every wave is done
   // with the one before it, whose flags are then cleared for the one after next.
-  __shared__ uint32_t busy_[3][2];
+  __shared__ uint32_t busy_[3][3];
   __shared__ uint32_t next_[2];
   __shared__ uint32_t free_base;
   __shared__ int32_t qptr[kQueue];
@@ -552,14 +560,14 @@ __global__ __launch_bounds__(kMcLanes, PSDF ? 3 : 4) void mc_surfel_kernel(Src s
   __shared__ uint32_t qn;
   __shared__ uint32_t scan_wave[8];
   __shared__ int32_t pop_top;
-  // One LDS region, two uses that never overlap in time: the configurations
-  // of the cubes at local -1..7 (this block and its lower neighbours) from the
-  // halo loop to the recycling test; the item list from the item scan to the
-  // end of the slot claims.  Barriers separate the uses.
-  __shared__ uint32_t region[6 * kBlockVoxels];
-  uint16_t* const items = reinterpret_cast<uint16_t*>(region);  // up to 12 per cube
-  uint8_t* const hcfg = reinterpret_cast<uint8_t*>(region);
-  static_assert(sizeof(region) >= 12 * kBlockVoxels * sizeof(uint16_t) && sizeof(region) >= kCfg * kCfg * kCfg, "region");
+  // One LDS region, two uses that never overlap in time: the slots that stored
+  // configurations use, up to the recycling test; the item list from the item
+  // scan to the end of the slot claims.  Barriers separate the uses.
+  constexpr uint32_t kMaxItems = 3 * kBlockSide * (kBlockSide + 1) * (kBlockSide + 1);
+  __shared__ uint32_t region[(kMaxItems + 1) / 2];
+  uint16_t* const items = reinterpret_cast<uint16_t*>(region);
+  uint32_t* const stored = region;  // axis, row (y + 8 z): a bit per x
+  static_assert(sizeof(region) >= 3 * 64 * sizeof(uint32_t) && 3 * 64 <= kMcLanes, "region");
   __shared__ Payload<PSDF> pay;
   __shared__ uint32_t nitems;
   // per-configuration crossed edges and triangle counts, read per lane with
@@ -588,7 +596,7 @@ __global__ __launch_bounds__(kMcLanes, PSDF ? 3 : 4) void mc_surfel_kernel(Src s
   uint32_t ci = blockIdx.x;
   if (threadIdx.x == 0) {
     next_[1] = item_after(ci);
-    for (int k = 0; k < 3; ++k) busy_[k][0] = busy_[k][1] = 0u;
+    for (int k = 0; k < 3; ++k) busy_[k][0] = busy_[k][1] = busy_[k][2] = 0u;
   }
   if (nb_lane < 27) row_[0][nb_lane] = nbt[(size_t)ci * 27u + nb_lane];
   __syncthreads();
@@ -604,6 +612,10 @@ __global__ __launch_bounds__(kMcLanes, PSDF ? 3 : 4) void mc_surfel_kernel(Src s
   BlockRegs<PSDF> R;
   load_block<PSDF>(src.view(scene), ptr, row_[0], code, R);
   for (uint32_t turn = 0, third = 0; ci < n; turn ^= 1u, third = third == 2 ? 0 : third + 1) {
+    // The lane's own places are worked out anew for each block: kept across them
+    // they do not fit the registers (100 bytes a lane spilled).
+    uint32_t tid = threadIdx.x;
+    asm("" : "+v"(tid));
     if (scene != cur_scene) {
       if (cur_scene != ~0u && threadIdx.x == 0) cnt.flush(src.view(cur_scene));
       cur_scene = scene;
@@ -614,7 +626,11 @@ __global__ __launch_bounds__(kMcLanes, PSDF ? 3 : 4) void mc_surfel_kernel(Src s
     const int32_t* const nb = row_[turn];
     if (threadIdx.x == 0) next_[turn] = nx < n ? item_after(nx) : n;
     if (nb_lane < 27) row_[turn ^ 1u][nb_lane] = nbe;
-    if (__any(stage_shell<PSDF>(mc, R, nb, code, S)) && (threadIdx.x & 63u) == 0) busy_[third][0] = 1u;
+    bool lower = false;  // a lower neighbour that is not meshed in this pass
+    if (nb_lane < 27 && nb_lane % 3 < 2 && (nb_lane / 3) % 3 < 2 && nb_lane / 9 < 2)
+      lower = nb[nb_lane] >= 0 && !row_meshed(nb[nb_lane]);
+    if (lower) busy_[third][2] = 1u;
+    if (__any(stage_shell<PSDF>(mc, R, code, S) || lower) && (tid & 63u) == 0) busy_[third][0] = 1u;
     int32_t vps[kMcVox][3];
     uint32_t word[kMcVox];
 #pragma unroll
@@ -628,7 +644,7 @@ __global__ __launch_bounds__(kMcLanes, PSDF ? 3 : 4) void mc_surfel_kernel(Src s
     // the next block's loads start
     if (threadIdx.x == 0) {
       const uint32_t before = third == 0 ? 2 : third - 1;
-      busy_[before][0] = busy_[before][1] = 0u;
+      busy_[before][0] = busy_[before][1] = busy_[before][2] = 0u;
       qn = 0;
       surfels[0] = surfels[1] = 0;
       tri_sum[0] = tri_sum[1] = 0;
@@ -661,7 +677,7 @@ __global__ __launch_bounds__(kMcLanes, PSDF ? 3 : 4) void mc_surfel_kernel(Src s
 #pragma unroll
       for (int r = 0; r < kMcVox; ++r) {
         const uint32_t prev = word[r] & 255u, nw = c[r] | (prev << 8);
-        if (nw != word[r]) V.cube[(size_t)self * kBlockVoxels + threadIdx.x + kMcLanes * r] = (uint16_t)nw;
+        if (nw != word[r]) V.cube[(size_t)self * kBlockVoxels + tid + kMcLanes * r] = (uint16_t)nw;
         lost += ntab[prev];  // c is 0 or 255: no triangle
       }
       // (rare: a block that lost its surface)
@@ -674,39 +690,57 @@ __global__ __launch_bounds__(kMcLanes, PSDF ? 3 : 4) void mc_surfel_kernel(Src s
       finish_empty(cube);
       continue;
     }
-    // every cube of the 10^3 halo, the block's own among them: validity for
-    // the writer rule, and the configuration of the block's own cubes
+    // The block's own cubes, and the crossings of the edges it owns (cross: x, y,
+    // z edges of a voxel whose ends differ in sign), from the shell's bits; the
+    // halo's cubes, of which only the validity counts, as rows of bits.
     bool crossing = false;
-#pragma unroll
-    for (int r = 0; r < kMcVox; ++r) crossing = crossing || vps[r][0] >= 0 || vps[r][1] >= 0 || vps[r][2] >= 0;
-    for (int s = (int)threadIdx.x; s < kCubeHalo * kCubeHalo * kCubeHalo; s += (int)kMcLanes) {
-      const int x = s % kCubeHalo - 1, y = (s / kCubeHalo) % kCubeHalo - 1, z = s / (kCubeHalo * kCubeHalo) - 1;
-      const int dx = x < 0 ? -1 : (x >= 8 ? 1 : 0), dy = y < 0 ? -1 : (y >= 8 ? 1 : 0),
-                dz = z < 0 ? -1 : (z >= 8 ? 1 : 0);
-      int c;
-      const bool valid = cube_index(S, x, y, z, &c);
-      const int32_t q = nb[nb27(dx, dy, dz)];
-      cv[s] = row_meshed(q) && valid;
-      if (dx <= 0 && dy <= 0 && dz <= 0) {
-        // what the block's cube word holds after this pass: computed here
-        // for a block meshed in it (its own pass computes the same bits from
-        // the same voxels), stored for one that is not
-        uint32_t hc = 0;
-        if (row_meshed(q))
-          hc = valid ? (uint32_t)c : 0u;
-        else if (q >= 0)
-          hc = V.cube[(size_t)q * kBlockVoxels + (x - 8 * dx) + 8 * (y - 8 * dy) + 64 * (z - 8 * dz)] & 255u;
-        hcfg[(x + 1) + kCfg * (y + 1) + kCfg * kCfg * (z + 1)] = (uint8_t)hc;
-        crossing = crossing || (hc != 0 && hc != 255);
-      }
-    }
-    if (__any(crossing) && (threadIdx.x & 63u) == 0) busy_[third][1] = 1u;
-    __syncthreads();
+    uint32_t cross[kMcVox];
 #pragma unroll
     for (int r = 0; r < kMcVox; ++r) {
-      const i3 o = devectorize(threadIdx.x + kMcLanes * r);
-      cube[r] = hcfg[(o.x + 1) + kCfg * (o.y + 1) + kCfg * kCfg * (o.z + 1)];
+      const i3 o = devectorize(tid + kMcLanes * r);
+      const uint32_t at = (uint32_t)sidx(o.x, o.y, o.z), up = at + kShell * kShell;
+      const uint32_t na = shell_bits(S.bits[kNeg], at), nu = shell_bits(S.bits[kNeg], up);
+      const uint32_t ca = shell_bits(S.bits[kCorner], at), cu = shell_bits(S.bits[kCorner], up);
+      cube[r] = (ca & cu & kCubeBits) == kCubeBits ? cube_of(na, nu) : 0u;
+      cross[r] = ((na ^ (na >> 1)) & 1u) | ((na ^ (na >> 11)) & 1u) << 1 | ((na ^ nu) & 1u) << 2;
+      // an edge that a valid cube uses has ends that pass the corner tests
+      cross[r] &= ca & 1u ? ((ca >> 1) & 1u) | ((ca >> 11) & 1u) << 1 | (cu & 1u) << 2 : 0u;
+      crossing = crossing || (cube[r] != 0 && cube[r] != 255) || cross[r] != 0 || vps[r][0] >= 0 || vps[r][1] >= 0 || vps[r][2] >= 0;
     }
+    // the halo's rows
+    if (tid < kCubeHalo * kCubeHalo) {
+      const uint32_t y = tid % kCubeHalo, z = tid / kCubeHalo;
+      const uint32_t at = kShell * y + kShell * kShell * z;
+      uint32_t c = shell_bits(S.bits[kCorner], at) & shell_bits(S.bits[kCorner], at + kShell * kShell);
+      c &= c >> kShell;
+      c &= c >> 1;
+      const int32_t* const q = nb + 3 * (y == 0 ? 0 : (y == 9 ? 2 : 1)) + 9 * (z == 0 ? 0 : (z == 9 ? 2 : 1));
+      cv[tid] = (uint16_t)(c & ((row_meshed(q[0]) ? 1u : 0u) | (row_meshed(q[1]) ? 0x1FEu : 0u) |
+                                        (row_meshed(q[2]) ? 0x200u : 0u)));
+    }
+    // Lower neighbours that are not meshed in this pass: the configurations that
+    // their cubes beside this block hold count.
+    const bool mixed = busy_[third][2] != 0;  // uniform
+    if (mixed) {
+      if (tid < 3 * 64) stored[tid] = 0u;
+      __syncthreads();
+      for (int s = (int)tid; s < kCfg * kCfg * kCfg; s += (int)kMcLanes) {
+        const int x = s % kCfg - 1, y = (s / kCfg) % kCfg - 1, z = s / (kCfg * kCfg) - 1;
+        const int dx = x < 0 ? -1 : 0, dy = y < 0 ? -1 : 0, dz = z < 0 ? -1 : 0;
+        const int32_t q = nb[nb27(dx, dy, dz)];
+        if (q < 0 || row_meshed(q)) continue;
+        const uint32_t hc = V.cube[(size_t)q * kBlockVoxels + (x - 8 * dx) + 8 * (y - 8 * dy) + 64 * (z - 8 * dz)] & 255u;
+        for (uint32_t m = etab[hc]; m; m &= m - 1u) {
+          const int e = __ffs(m) - 1;
+          const int ox = x + edge_owner_off(e, 0), oy = y + edge_owner_off(e, 1), oz = z + edge_owner_off(e, 2);
+          if (min(min(ox, oy), oz) < 0 || max(max(ox, oy), oz) > 7) continue;
+          atomicOr(&stored[64 * edge_axis(e) + oy + 8 * oz], 1u << ox);
+          crossing = true;
+        }
+      }
+    }
+    if (__any(crossing) && (tid & 63u) == 0) busy_[third][1] = 1u;
+    __syncthreads();
     if (!busy_[third][1]) {  // uniform: no crossed edge here or below, no slot held
       finish_empty(cube);
       continue;
@@ -714,43 +748,36 @@ __global__ __launch_bounds__(kMcLanes, PSDF ? 3 : 4) void mc_surfel_kernel(Src s
     // RecycleVerticesKernel on this block's own slots (marching_cubes.cu:
     // 303-321): a slot is referenced iff one of the four cubes around its edge
     // (this block and its lower neighbours, whose configurations are all
-    // final above) crosses the edge.  Unreferenced allocated slots are freed
+    // final above) crosses the edge: its ends differ and one of the cubes is
+    // valid, or one that is not meshed here holds it.  Unreferenced allocated slots are freed
     // (to the free list; they go on the heap after the pass, so no pop of
     // this pass can take them).  The surfel counts are the slots allocated
     // once the pass's claims are done: allocated now, or referenced (a
     // referenced free slot is claimed in this pass, here or by a lower
     // neighbour).  No other workgroup touches an unreferenced slot.
     unsigned release = 0;
-    unsigned em[kMcVox];
     {
       int inner = 0, boundary = 0;
 #pragma unroll
       for (int r = 0; r < kMcVox; ++r) {
-        const i3 o = devectorize(threadIdx.x + kMcLanes * r);
+        const i3 o = devectorize(tid + kMcLanes * r);
         const bool is_inner = o.x >= 1 && o.y >= 1 && o.z >= 1 && o.x < 7 && o.y < 7 && o.z < 7;
-        // the crossed edges of the eight cubes at o - {0, 1}^3
-        unsigned m8[8];
+        // the cubes at x - 1 (bit 0) and x of the rows y - {0, 1}, z - {0, 1}
+        const int at = crow(o.y, o.z);
+        const uint32_t m00 = cv[at] >> o.x, m10 = cv[at - 1] >> o.x, m01 = cv[at - kCubeHalo] >> o.x,
+                       m11 = cv[at - kCubeHalo - 1] >> o.x;
+        uint32_t used = cross[r] & (((m00 | m10 | m01 | m11) & 2u ? 1u : 0u) | ((m00 | m01) & 3u ? 2u : 0u) |
+                                    ((m00 | m10) & 3u ? 4u : 0u));
+        if (mixed)
 #pragma unroll
-        for (int k = 0; k < 8; ++k)
-          m8[k] = etab[hcfg[(o.x - (k & 1) + 1) + kCfg * (o.y - ((k >> 1) & 1) + 1) + kCfg * kCfg * (o.z - (k >> 2) + 1)]];
-        em[r] = m8[0];  // 0 for configurations 0 and 255
+          for (int a = 0; a < 3; ++a) used |= ((stored[64 * a + o.y + 8 * o.z] >> o.x) & 1u) << a;
+        uint32_t held = 0;
 #pragma unroll
-        for (int a = 0; a < 3; ++a) {
-          const int b1 = a == 0 ? 1 : 0, b2 = a == 2 ? 1 : 2;
-          bool used = false;
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            int d[3] = {0, 0, 0};
-            d[b1] = k & 1;
-            d[b2] = k >> 1;
-            used = used || ((m8[d[0] + 2 * d[1] + 4 * d[2]] >> edge_with(d[0], d[1], d[2], a)) & 1u) != 0;
-          }
-          if (vps[r][a] >= 0 || used) {
-            if (is_inner) ++inner;
-            else ++boundary;
-          }
-          if (vps[r][a] >= 0 && !used) release |= 1u << (3 * r + a);
-        }
+        for (int a = 0; a < 3; ++a) held |= vps[r][a] >= 0 ? 1u << a : 0u;
+        const int slots = __popc(held | used);
+        if (is_inner) inner += slots;
+        else boundary += slots;
+        release |= (held & ~used) << (3 * r);
       }
       if (inner) atomicAdd(&surfels[0], inner);
       if (boundary) atomicAdd(&surfels[1], boundary);
@@ -762,7 +789,7 @@ __global__ __launch_bounds__(kMcLanes, PSDF ? 3 : 4) void mc_surfel_kernel(Src s
 #pragma unroll
       for (int r = 0; r < kMcVox; ++r) {
         const uint32_t prev = word[r] & 255u, nw = cube[r] | (prev << 8);
-        if (nw != word[r]) V.cube[(size_t)self * kBlockVoxels + threadIdx.x + kMcLanes * r] = (uint16_t)nw;
+        if (nw != word[r]) V.cube[(size_t)self * kBlockVoxels + tid + kMcLanes * r] = (uint16_t)nw;
         // live triangles of a cube = its configuration's table row
         const int nt = ntab[cube[r]];
         delta += nt - ntab[prev];
@@ -771,25 +798,40 @@ __global__ __launch_bounds__(kMcLanes, PSDF ? 3 : 4) void mc_surfel_kernel(Src s
       if (delta) atomicAdd(&tri_sum[0], delta);
       if (assigned) atomicAdd(&tri_sum[1], assigned);
     }
-    // The crossed edges of the block's cubes become a dense item list
-    // (voxel | edge << 9), so the slot work below runs one item per lane
-    // instead of twelve edge rounds on every cube.  The same scan ranks the
-    // freed slots (bits 13 and up: the item counts sum to at most 6144).
+    // The edges that the block's own valid cubes cross become a dense item list,
+    // each once: a row of owner voxels (x 0..8 at some y, z in 0..8) has their x, y
+    // and z edges from the rows of signs and of cubes.  (An item for each crossed
+    // edge of each cube, four to a slot, took four times the claim rounds.)
+    // The same scan ranks the freed slots (bits 13 and up: there are at most
+    // 3 * 8 * 9 * 9 items).
     uint32_t free_rank, n_freed;
     {
-      static_assert(kMcVox <= 2, "at most 24 items and 6 freed slots a lane");
-      uint32_t mine = (uint32_t)__popc(release) << 13;
-#pragma unroll
-      for (int r = 0; r < kMcVox; ++r) mine += (uint32_t)__popc(em[r]);
+      constexpr uint32_t kRows = kBlockSide + 1;
+      static_assert(kRows * kRows <= 128 && kMcLanes >= 256, "the rows take the two waves that had no halo rows");
+      const uint32_t row = tid - (kMcLanes - 128), ry = row % kRows, rz = row / kRows;
+      uint32_t edges = 0;  // x edges in bits 0..7, y in 8..16, z in 17..25
+      if (row < kRows * kRows) {
+        const uint32_t at = (uint32_t)sidx(0, (int)ry, (int)rz);
+        const uint32_t na = shell_bits(S.bits[kNeg], at), nu = shell_bits(S.bits[kNeg], at + kShell * kShell);
+        // own valid cubes of the rows y - {0, 1}, z - {0, 1} (those outside the block count as none)
+        const int c = crow((int)ry, (int)rz);
+        const uint32_t y0 = ry < 8 ? 0xFFu : 0u, y1 = ry > 0 ? 0xFFu : 0u, z0 = rz < 8 ? 0xFFu : 0u, z1 = rz > 0 ? 0xFFu : 0u;
+        const uint32_t v00 = (cv[c] >> 1) & y0 & z0, v10 = (cv[c - 1] >> 1) & y1 & z0,
+                       v01 = (cv[c - kCubeHalo] >> 1) & y0 & z1, v11 = (cv[c - kCubeHalo - 1] >> 1) & y1 & z1;
+        const uint32_t ey = v00 | v01, ez = v00 | v10;
+        edges = ((na ^ (na >> 1)) & (ey | v10 | v11)) | ((na ^ (na >> kShell)) & (ey | ey << 1)) << 8 |
+                ((na ^ nu) & (ez | ez << 1)) << 17;
+      }
+      static_assert(kMcVox <= 2, "at most 6 freed slots a lane");
       uint32_t total;
-      const uint32_t at2 =
-          block_excl_scan_planes<kMcVox == 2 ? 0x1Fu | (0x7u << 13) : 0xFu | (0x3u << 13)>(mine, scan_wave, &total);
+      const uint32_t at2 = block_excl_scan_planes<0x1Fu | (0x7u << 13)>((uint32_t)__popc(release) << 13 | (uint32_t)__popc(edges),
+                                                                       scan_wave, &total);
       uint32_t at = at2 & 8191u;
       free_rank = at2 >> 13;
-#pragma unroll
-      for (int r = 0; r < kMcVox; ++r)
-        for (unsigned m = em[r]; m; m &= m - 1u)
-          items[at++] = (uint16_t)((threadIdx.x + kMcLanes * r) | ((uint32_t)(__ffs(m) - 1) << 9));
+      for (; edges; edges &= edges - 1u) {
+        const uint32_t k = (uint32_t)__ffs((int)edges) - 1u, ax = k >= 17 ? 2u : (k >= 8 ? 1u : 0u);
+        items[at++] = (uint16_t)((k - (ax == 2 ? 17u : 8u * ax)) | (ry << 4) | (rz << 8) | (ax << 12));
+      }
       if (threadIdx.x == 0) nitems = total & 8191u;
       n_freed = total >> 13;
     }
@@ -808,18 +850,17 @@ __global__ __launch_bounds__(kMcLanes, PSDF ? 3 : 4) void mc_surfel_kernel(Src s
       // Vertex slot of each item: read it; claim it if free (CAS to the
       // lock value); pop fresh vertices for all claims of the workgroup
       // with one heap operation; publish them.
-      const uint32_t jt = c0 + threadIdx.x;
+      const uint32_t jt = c0 + tid;
       const bool has = jt < n_items;
-      i3 oo{0, 0, 0};
-      int e = 0;
+      uint32_t it = 0;  // a vertex's key: owner voxel and axis
       int32_t* slot = nullptr;
       int32_t cur = kFreePtr;
       bool claimed = false;
       if (has) {
-        const uint32_t it = items[jt];
-        oo = devectorize(it & 511u);
-        e = (int)(it >> 9);
-        slot = edge_slot(V, nb, oo, e);
+        it = items[jt];
+        const uint32_t x = it & 15u, y = (it >> 4) & 15u, z = (it >> 8) & 15u;
+        const int32_t optr = row_ptr(nb[13 + (x >> 3) + 3 * (y >> 3) + 9 * (z >> 3)]);
+        slot = &V.vptr[((size_t)optr * kBlockVoxels + ((x & 7u) | (y & 7u) << 3 | (z & 7u) << 6)) * 3 + (it >> 12)];
         cur = *slot;
         if (cur == kFreePtr) {
           const int32_t old = atomicCAS(slot, kFreePtr, kLockPtr);
@@ -848,28 +889,27 @@ __global__ __launch_bounds__(kMcLanes, PSDF ? 3 : 4) void mc_surfel_kernel(Src s
         }
       }
       if (has && cur >= 0) {
-        const int ax = edge_axis(e);
-        const int offx = edge_owner_off(e, 0), offy = edge_owner_off(e, 1), offz = edge_owner_off(e, 2);
-        const int ox = oo.x + offx, oy = oo.y + offy, oz = oo.z + offz;
-        // writer rule: offsets across the edge in the two other axes (b1 < b2;
-        // selected without indexing, e being a run-time value here)
-        const int b1 = ax == 0 ? 1 : 0, b2 = ax == 2 ? 1 : 2;
-        const int own1 = b1 == 0 ? offx : offy, own2 = b2 == 1 ? offy : offz;
-        const int kself = own1 + 2 * own2;
+        // writer rule: of the four cubes around the edge, in the order (0, 0),
+        // (1, 0), (0, 1), (1, 1) of the offsets in the two other axes, the first
+        // that is valid and meshed in this pass; `first` is its bit, `own` those of
+        // the cubes of this block
+        const int x = (int)(it & 15u), y = (int)((it >> 4) & 15u), z = (int)((it >> 8) & 15u), ax = (int)(it >> 12);
+        uint32_t first = 0, own = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const int d1 = k & 1, d2 = k >> 1;
+          const int qx = x - (ax != 0 ? d1 : 0), qy = y - (ax == 0 ? d1 : (ax == 2 ? d2 : 0)), qz = z - (ax != 2 ? d2 : 0);
+          first |= (((uint32_t)cv[crow(qy, qz)] >> (qx + 1)) & 1u) << k;
+          own |= ((qx | qy | qz) & ~7) == 0 ? 1u << k : 0u;
+        }
+        first &= 0u - first;
         // A slot claimed in this pass is also written by its claimer: the
         // designated cube may have read it while still locked and skipped it.
-        bool writer = true;
-        for (int k = 0; k < kself && writer && !claimed; ++k) {
-          const int d1 = k & 1, d2 = k >> 1;
-          const int qx = ox - (b1 == 0 ? d1 : 0);
-          const int qy = oy - (b1 == 1 ? d1 : 0) - (b2 == 1 ? d2 : 0);
-          const int qz = oz - (b2 == 2 ? d2 : 0);
-          if (cv[cidx(qx, qy, qz)]) writer = false;
-        }
+        const bool writer = claimed || (first & own) != 0;
         if (writer) {  // queue the payload; all lanes of the block work the queue
           const uint32_t q = atomicAdd(&qn, 1u);
           qptr[q] = cur;
-          qkey[q] = (uint16_t)((uint32_t)ox | ((uint32_t)oy << 4) | ((uint32_t)oz << 8) | ((uint32_t)ax << 12));
+          qkey[q] = (uint16_t)it;
         }
       }
       if (threadIdx.x == 0 && c0 == 0 && n_freed) free_base = base_got;
@@ -883,7 +923,7 @@ __global__ __launch_bounds__(kMcLanes, PSDF ? 3 : 4) void mc_surfel_kernel(Src s
             const int32_t vp = vps[r][a];
             Vertex zv{};
             V.vertices[vp] = zv;
-            V.vptr[3 * ((size_t)self * kBlockVoxels + threadIdx.x + kMcLanes * r) + a] = kFreePtr;
+            V.vptr[3 * ((size_t)self * kBlockVoxels + tid + kMcLanes * r) + a] = kFreePtr;
             V.vfree[free_base + free_rank] = vp;
             ++free_rank;
           }
@@ -894,11 +934,11 @@ __global__ __launch_bounds__(kMcLanes, PSDF ? 3 : 4) void mc_surfel_kernel(Src s
       // for their normals and one for the rest (other waves each time)
       const uint32_t nq = qn;
       cnt.writes += nq;
-      const uint32_t jl = threadIdx.x >> 2, lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+      const uint32_t jl = tid >> 2, lane = tid & 63u, wave = tid >> 6;
       for (uint32_t j0 = 0; j0 < nq; j0 += kPayRound, turns += 2) {  // uniform
         const uint32_t j = j0 + jl;
         if (j < nq &&  // the same for a vertex's four lanes
-            payload_part<PSDF>(S, V.geo, mc, inv_vs, base, qkey[j], threadIdx.x & 3u, jl, pay))
+            payload_part<PSDF>(S, V.geo, mc, inv_vs, base, qkey[j], tid & 3u, jl, pay))
           flag(V, MH_STATUS_STENCIL_RANGE);
         __syncthreads();
         const uint32_t role = (wave + turns) & 3u;
