@@ -352,31 +352,57 @@ template <int CTRL>
 __device__ __forceinline__ uint32_t quad_swap(uint32_t x) {
   return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xF, 0xF, true);
 }
+// The axes of the samples that lie at a voxel's coordinate, and half a voxel to
+// either side: a vertex is off its voxel along its own axis only, so five of the
+// eight axes of a lane's samples are among a block's 81 of these.  They are
+// rounding ties, which shell_axis settles with divisions: 6850 wave instructions
+// a block of 64 rooms without the table, 5780 with it (1033 and 946 us a pass).
+struct AxisTable {
+  uint32_t c[3][9][3];  // axis, voxel 0..8, -h / 0 / +h: c0 + 64 | c1 + 64 << 8
+  float r[3][9][3];
+};
+constexpr uint32_t kAxisEntries = 81;
+__device__ __forceinline__ void axis_table_fill(AxisTable& T, uint32_t e, float vs, float inv_vs, i3 base) {
+  const uint32_t d = e % 3, o = e / 3 % 9, a = e / 27;
+  const int b = a == 0 ? base.x : (a == 1 ? base.y : base.z);
+  const float p = (float)(b + (int)o) * vs, h = 0.5f * vs;
+  const SAxis A = shell_axis(d == 0 ? p - h : (d == 1 ? p : p + h), vs, inv_vs, b);
+  auto byte = [](int c) { return (uint32_t)(min(max(c, -64), 191) + 64); };  // (out of the shell stays so)
+  (&T.c[0][0][0])[e] = byte(A.c0) | byte(A.c1) << 8;
+  (&T.r[0][0][0])[e] = A.r;
+}
+__device__ __forceinline__ SAxis axis_at(const AxisTable& T, int a, int o, int d) {
+  const uint32_t c = T.c[a][o][d];
+  return SAxis{(int)(c & 255u) - 64, (int)(c >> 8) - 64, T.r[a][o][d]};
+}
 // Lane sub's part for vertex j of the round; true if a sample lies outside the shell.
 template <bool PSDF>
 __device__ __forceinline__ bool payload_part(const Shell<PSDF>& S, const Geo& g, const McConst& mc, float inv_vs,
-                                             i3 base, uint32_t key, uint32_t sub, uint32_t j, Payload<PSDF>& P) {
+                                             const AxisTable& T, i3 base, uint32_t key, uint32_t sub, uint32_t j,
+                                             Payload<PSDF>& P) {
   const float vs = g.voxel_size;
   const int ox = (int)(key & 15u), oy = (int)((key >> 4) & 15u), oz = (int)((key >> 8) & 15u);
   const int ax = (int)(key >> 12);
   const int sA = sidx(ox, oy, oz);
   const float vA = S.sdf[sA], vB = S.sdf[sA + (ax == 0 ? 1 : (ax == 1 ? kShell : kShell * kShell))];
-  const f3 pA = voxel_to_world(g, i3{base.x + ox, base.y + oy, base.z + oz});
-  const f3 pB = mk3(pA.x + (ax == 0 ? vs : 0.0f), pA.y + (ax == 1 ? vs : 0.0f), pA.z + (ax == 2 ? vs : 0.0f));
-  f3 p;
+  // the vertex's coordinate along its axis, from its voxel's to the next one's
+  const int b = ax == 0 ? base.x : (ax == 1 ? base.y : base.z), o = (int)((key >> (4 * ax)) & 15u);
+  const float pA = (float)(b + o) * vs, pB = pA + vs;
+  float p;
   if ((double)fabsf(vA) < mc.snap) {
     p = pA;
   } else if ((double)fabsf(vB) < mc.snap) {
     p = pB;
   } else {
     const float mu = (0.0f - vA) / (vB - vA);
-    p = mk3(pA.x + mu * (pB.x - pA.x), pA.y + mu * (pB.y - pA.y), pA.z + mu * (pB.z - pA.z));
+    p = pA + mu * (pB - pA);
   }
   const float h = 0.5f * vs;
   // the first stencil's axes (lane 3: p's), and the one that the second differs in
-  SAxis X = shell_axis(sub == 0 ? p.x - h : p.x, vs, inv_vs, base.x);
-  SAxis Y = shell_axis(sub == 1 ? p.y - h : p.y, vs, inv_vs, base.y);
-  SAxis Z = shell_axis(sub == 2 ? p.z - h : p.z, vs, inv_vs, base.z);
+  const SAxis A = shell_axis((int)sub == ax ? p - h : p, vs, inv_vs, b);
+  SAxis X = ax == 0 ? A : axis_at(T, 0, ox, sub == 0 ? 0 : 1);
+  SAxis Y = ax == 1 ? A : axis_at(T, 1, oy, sub == 1 ? 0 : 1);
+  SAxis Z = ax == 2 ? A : axis_at(T, 2, oz, sub == 2 ? 0 : 1);
   bool oob = !axes_in(X, Y, Z);
   // lane 3's cell, corner coordinates + 1 in 4 bits each (inside: all in 0..10)
   const uint32_t cell = (uint32_t)(X.c0 + 1) | ((uint32_t)(X.c1 + 1) << 4) | ((uint32_t)(Y.c0 + 1) << 8) |
@@ -398,9 +424,9 @@ __device__ __forceinline__ bool payload_part(const Shell<PSDF>& S, const Geo& g,
     P.v[kPayRatio][j] = X.r;
     P.v[kPayRatio + 1][j] = Y.r;
     P.v[kPayRatio + 2][j] = Z.r;
-    P.v[kPayPos][j] = p.x;
-    P.v[kPayPos + 1][j] = p.y;
-    P.v[kPayPos + 2][j] = p.z;
+    P.v[kPayPos][j] = ax == 0 ? p : (float)(base.x + ox) * vs;
+    P.v[kPayPos + 1][j] = ax == 1 ? p : (float)(base.y + oy) * vs;
+    P.v[kPayPos + 2][j] = ax == 2 ? p : (float)(base.z + oz) * vs;
     P.v[kPayOk][j] = ok ? 1.0f : 0.0f;
     if (PSDF && ok) {
       P.v[kPayA][j] = shell_value(S.a, X, Y, Z);
@@ -411,8 +437,8 @@ __device__ __forceinline__ bool payload_part(const Shell<PSDF>& S, const Geo& g,
     for (uint32_t i = 0;; ++i) {
       P.v[kPayS + 2 * sub + i][j] = axes_in(X, Y, Z) ? shell_value(S.sdf, X, Y, Z) : NAN;
       if (i) break;
-      const SAxis A = sub == 0 ? shell_axis(p.x + h, vs, inv_vs, base.x)
-                               : (sub == 1 ? shell_axis(p.y + h, vs, inv_vs, base.y) : shell_axis(p.z + h, vs, inv_vs, base.z));
+      SAxis A = axis_at(T, (int)sub, (int)((key >> (4 * sub)) & 15u), 2);
+      if ((int)sub == ax) A = shell_axis(p + h, vs, inv_vs, b);
       if (sub == 0) X = A;
       if (sub == 1) Y = A;
       if (sub == 2) Z = A;
@@ -472,10 +498,10 @@ __device__ __forceinline__ void finish_normal(const View& V, int32_t vp, uint32_
 // shared by up to four cubes.  Its payload is written once per pass, by a
 // designated cube: the first, in the order (0,0), (1,0), (0,1), (1,1) of
 // the offsets across the edge, that is valid and belongs to a block meshed
-// in this pass.  Every cube can evaluate that rule from the staged shell (a
-// 10^3 halo of cube validities and the meshed flags of the 27 blocks), so
-// no atomics are needed; the other cubes only make sure the vertex slot is
-// allocated.  Any writer would store the same bits (canonical vertices).
+// in this pass.  Every block can evaluate that rule from the staged shell (the
+// halo's rows of valid cubes and the meshed flags of the 27 blocks), so
+// no atomics are needed; the other cubes' blocks only make sure the vertex slot
+// is allocated.  Any writer would store the same bits (canonical vertices).
 
 // Work counts of a workgroup, kept by its first lane and added to the scene's
 // counters when the scene changes.
@@ -569,6 +595,7 @@ __global__ __launch_bounds__(kMcLanes, PSDF ? 3 : 4) void mc_surfel_kernel(Src s
   uint32_t* const stored = region;  // axis, row (y + 8 z): a bit per x
   static_assert(sizeof(region) >= 3 * 64 * sizeof(uint32_t) && 3 * 64 <= kMcLanes, "region");
   __shared__ Payload<PSDF> pay;
+  __shared__ AxisTable axes;
   __shared__ uint32_t nitems;
   // per-configuration crossed edges and triangle counts, read per lane with
   // divergent indices: from LDS rather than the constant tables
@@ -707,7 +734,11 @@ __global__ __launch_bounds__(kMcLanes, PSDF ? 3 : 4) void mc_surfel_kernel(Src s
       cross[r] &= ca & 1u ? ((ca >> 1) & 1u) | ((ca >> 11) & 1u) << 1 | (cu & 1u) << 2 : 0u;
       crossing = crossing || (cube[r] != 0 && cube[r] != 255) || cross[r] != 0 || vps[r][0] >= 0 || vps[r][1] >= 0 || vps[r][2] >= 0;
     }
-    // the halo's rows
+    // the halo's rows, and by the other two waves the block's axes
+    const i3 base = i3{b.x * kBlockSide, b.y * kBlockSide, b.z * kBlockSide};
+    const float inv_vs = 1.0f / V.geo.voxel_size;
+    if (tid - (kMcLanes - 128) < kAxisEntries)
+      axis_table_fill(axes, tid - (kMcLanes - 128), V.geo.voxel_size, inv_vs, base);
     if (tid < kCubeHalo * kCubeHalo) {
       const uint32_t y = tid % kCubeHalo, z = tid / kCubeHalo;
       const uint32_t at = kShell * y + kShell * kShell * z;
@@ -782,8 +813,6 @@ __global__ __launch_bounds__(kMcLanes, PSDF ? 3 : 4) void mc_surfel_kernel(Src s
       if (inner) atomicAdd(&surfels[0], inner);
       if (boundary) atomicAdd(&surfels[1], boundary);
     }
-    const i3 base = i3{b.x * kBlockSide, b.y * kBlockSide, b.z * kBlockSide};
-    const float inv_vs = 1.0f / V.geo.voxel_size;
     {
       int delta = 0, assigned = 0;
 #pragma unroll
@@ -938,7 +967,7 @@ __global__ __launch_bounds__(kMcLanes, PSDF ? 3 : 4) void mc_surfel_kernel(Src s
       for (uint32_t j0 = 0; j0 < nq; j0 += kPayRound, turns += 2) {  // uniform
         const uint32_t j = j0 + jl;
         if (j < nq &&  // the same for a vertex's four lanes
-            payload_part<PSDF>(S, V.geo, mc, inv_vs, base, qkey[j], tid & 3u, jl, pay))
+            payload_part<PSDF>(S, V.geo, mc, inv_vs, axes, base, qkey[j], tid & 3u, jl, pay))
           flag(V, MH_STATUS_STENCIL_RANGE);
         __syncthreads();
         const uint32_t role = (wave + turns) & 3u;
