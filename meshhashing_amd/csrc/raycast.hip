@@ -936,12 +936,13 @@ void launch_slot_reduce(double* partials, uint32_t n, uint32_t slots, uint32_t* 
 // SIMD at 333 x 251, and each wave's time is the latency of its rays' samples
 // in a row; four (two) lanes a ray then take a quarter (half) of the rounds.
 // As many as fit the chip in one round of waves; past that the extra lanes only
-// add work.  Measured (5 mm desk, whole call, 1 / 2 / 4 lanes): 160 x 120
+// add work.  Four lanes go an eighth past it, the first waves being done by then
+// (5 mm desk, 333 x 251: 112 us, 131 with two; 344 x 258: 108 and 122).  Measured (5 mm desk, whole call, 1 / 2 / 4 lanes): 160 x 120
 // 155 / 128 / 92 us, 320 x 240 138 / 124 / 98, 400 x 300 147 / 130 / 137,
 // 480 x 360 149 / 155 / 152, 640 x 480 142 / 162 / 189.
 inline int ray_lanes(uint64_t pixels, int cus) {
   const uint64_t waves = (pixels + 63) / 64, room = (uint64_t)kRayWavesPerSimd * 4 * (uint64_t)cus;
-  return 4 * waves <= room ? 4 : (2 * waves <= room ? 2 : 1);
+  return 4 * waves <= room + room / 8 ? 4 : (2 * waves <= room ? 2 : 1);
 }
 
 // ------------------------------------------------------------ localisation
