@@ -160,14 +160,8 @@ __device__ __forceinline__ bool key_present(const View& V, uint64_t key, uint32_
 // losing a race re-scans the bucket with device-coherent loads (each lost
 // CAS means one more slot is taken, so this ends within bucket_size + 1
 // rounds).  A full bucket defers the key to the serial list-insert pass.
-__device__ void insert_block(const View& V, i3 p) {
-  if (!coord_ok(p)) {
-    flag(V, MH_STATUS_COORD_RANGE);
-    return;
-  }
-  const uint64_t key = pack_key(p);
-  const uint32_t first = hash_bucket(p, V.bucket_count) * V.bucket_size;
-  if (key_present(V, key, first)) return;
+// (key and first: its key and its bucket's first slot; its presence was tested)
+__device__ void insert_absent(const View& V, i3 p, uint64_t key, uint32_t first) {
   for (uint32_t round = 0; round <= V.bucket_size; ++round) {
     // every slot's key read before any is tested (no early exit between the
     // loads, so they are in flight together)
@@ -217,6 +211,15 @@ __device__ void insert_block(const View& V, i3 p) {
     V.ovf[q] = key;
   else
     flag(V, MH_STATUS_OVERFLOW_QUEUE_FULL);
+}
+__device__ __forceinline__ void insert_block(const View& V, i3 p) {
+  if (!coord_ok(p)) {
+    flag(V, MH_STATUS_COORD_RANGE);
+    return;
+  }
+  const uint64_t key = pack_key(p);
+  const uint32_t first = hash_bucket(p, V.bucket_count) * V.bucket_size;
+  if (!key_present(V, key, first)) insert_absent(V, p, key, first);
 }
 
 // AllocBlockArrayKernel, allocate.cu:8-99: per pixel, walk the blocks between
@@ -277,7 +280,19 @@ __global__ __launch_bounds__(256) void alloc_kernel(Src src_, const SceneFrame* 
   const int sx = (int)step.x, sy = (int)step.y, sz = (int)step.z;
   i3 cur = bn;
   for (int it = 0; it < kMaxDdaSteps; ++it) {
-    if (block_in_frustum(g, V.cTw, cur, V.cam)) insert_block(V, cur);
+    // A block that is there already, as nearly all are once a scene has been
+    // seen, needs no frustum test, which takes more instructions than the lookup.
+    // Bound by those: 64 rooms of 320 x 240 134 us with the test first, 122 us so; one
+    // room 11.2 and 10.4 us.
+    const bool ok = coord_ok(cur);
+    const uint64_t key = pack_key(cur);
+    const uint32_t first = ok ? hash_bucket(cur, V.bucket_count) * V.bucket_size : 0u;
+    if (!(ok && key_present(V, key, first)) && block_in_frustum(g, V.cTw, cur, V.cam)) {
+      if (ok)
+        insert_absent(V, cur, key, first);
+      else
+        flag(V, MH_STATUS_COORD_RANGE);
+    }
     if (t.x < t.y && t.x < t.z) {
       cur.x += sx;
       if (cur.x == bound.x) return;
