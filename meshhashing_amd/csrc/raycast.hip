@@ -1331,8 +1331,12 @@ constexpr int kLaneTiles = 16;
 // touched to the global table with one atomic per bound, instead of one per
 // block and tile.
 constexpr uint32_t kRangeLdsTiles = 4800;  // 640 x 480 pixels
+// Every workgroup sends its tiles once: twice as many of half the lanes took 10.2
+// us for 31 k blocks at 640 x 480 (9.2 us so, 9.5 with half as many of 1024 lanes)
+// and 31 us for 64 rooms (25 us, 26 us).
+constexpr int kRangeLdsLanes = 512;
 template <class Src, bool kLds>
-__global__ __launch_bounds__(256) void ray_range_kernel(Src src_, const SceneFrame* __restrict__ tab, RayConst R1) {
+__global__ __launch_bounds__(kLds ? kRangeLdsLanes : 256) void ray_range_kernel(Src src_, const SceneFrame* __restrict__ tab, RayConst R1) {
   const Src src = with_table(src_, tab);
   const uint32_t scene = blockIdx.y;
   const View& V = src.view(scene);
@@ -1384,7 +1388,7 @@ void launch_ray_range(Src src, const SceneFrame* tab, const RayConst& R, uint32_
                       hipStream_t s) {
   launch_ray_prepare(src, tab, R, nscenes, s);
   if (tiles <= kRangeLdsTiles) {
-    ray_range_kernel<Src, true><<<dim3(nscenes > 1 ? 64 : 256, nscenes), 256, 0, s>>>(src, tab, R);
+    ray_range_kernel<Src, true><<<dim3(nscenes > 1 ? 32 : 128, nscenes), kRangeLdsLanes, 0, s>>>(src, tab, R);
   } else {
     // the pool slots of a 118 k-block volume over the whole chip
     // (the projections are independent; 128 workgroups had left most CUs idle)
