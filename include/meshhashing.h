@@ -149,8 +149,9 @@ int mh_get_status(mh_volume* v, mh_status* out);
  * MH_DIAG_KERNEL_TIMES: each kernel the volume's stage entry points launch
  *   is bracketed by HIP events on the volume's stream; mh_kernel_times sums
  *   them per kernel name (launches, total ms) and synchronises.
- * MH_DIAG_RAY_BLOCKS: mh_raycast records which blocks its lookups find and
- *   adds their number to mh_status.ray_blocks (one more kernel per call). */
+ * MH_DIAG_RAY_BLOCKS: mh_raycast records which blocks its samples lie in and
+ *   adds their number to mh_status.ray_blocks (one more kernel per call, and
+ *   one lane a ray where a small image would otherwise take two or four). */
 #define MH_DIAG_KERNEL_TIMES 1u
 #define MH_DIAG_RAY_BLOCKS 2u
 int mh_volume_set_diagnostics(mh_volume* v, uint32_t flags);

@@ -1398,8 +1398,11 @@ void launch_ray_range(Src src, const SceneFrame* tab, const RayConst& R, uint32_
 
 template <class Src>
 void raycast_shaped(Src src, const SceneFrame* tab, const RayConst& p, uint32_t w, uint32_t h, uint32_t nscenes,
-                    bool wide, int shape, int cus, float* depth, float* vertex, float* normal, hipStream_t s) {
-  const int lanes = wide || shape != 0 ? 1 : ray_lanes((uint64_t)w * h * nscenes, cus);
+                    bool wide, bool marks, int shape, int cus, float* depth, float* vertex, float* normal,
+                    hipStream_t s) {
+  // marks: the blocks of the samples are counted; several lanes a ray also
+  // sample behind its crossing
+  const int lanes = wide || marks || shape != 0 ? 1 : ray_lanes((uint64_t)w * h * nscenes, cus);
   const int px = 64 / lanes;
   const int tw = lanes == 1 ? kRayTileWidths[shape] : (lanes == 2 ? 8 : 4), th = px / tw;
   const int log_tw = __builtin_ctz((unsigned)tw);
@@ -1418,8 +1421,8 @@ void launch_ray_range_one(const View& V, const RayConst& p, hipStream_t s) {
 
 void launch_raycast_march(const View& V, const RayConst& p, float* depth, float* vertex, float* normal,
                           hipStream_t s, int cus, int shape) {
-  raycast_shaped(One{V}, nullptr, p, p.cam.width, p.cam.height, 1, V.capacity > kNarrowCapacity, shape, cus,
-                 depth, vertex, normal, s);
+  raycast_shaped(One{V}, nullptr, p, p.cam.width, p.cam.height, 1, V.capacity > kNarrowCapacity, V.ray_mark != nullptr,
+                 shape, cus, depth, vertex, normal, s);
 }
 
 void launch_raycast(const View& V, const RayConst& p, float* depth, float* vertex, float* normal,
@@ -1427,8 +1430,8 @@ void launch_raycast(const View& V, const RayConst& p, float* depth, float* verte
   tick(kc, s, "ray_range_kernel");
   launch_ray_range(One{V}, nullptr, p, p.tiles, 1, s);
   tick(kc, s, "raycast_kernel");
-  raycast_shaped(One{V}, nullptr, p, p.cam.width, p.cam.height, 1, V.capacity > kNarrowCapacity, shape, cus,
-                 depth, vertex, normal, s);
+  raycast_shaped(One{V}, nullptr, p, p.cam.width, p.cam.height, 1, V.capacity > kNarrowCapacity, V.ray_mark != nullptr,
+                 shape, cus, depth, vertex, normal, s);
   tick(kc, s, nullptr);
 }
 
@@ -1465,8 +1468,8 @@ void launch_raycast_backward(const View& V, const RayConst& p, const float* obs,
 void launch_batch_raycast(const BatchDev& B, float* depth, float* vertex, float* normal,
                           hipStream_t s, int cus, int shape) {
   launch_ray_range(B.src(), B.frames, RayConst{}, ((B.width + 7) / 8) * ((B.height + 7) / 8), B.nscenes, s);
-  raycast_shaped(B.src(), B.frames, RayConst{}, B.width, B.height, B.nscenes, B.max_capacity > kNarrowCapacity, shape,
-                 cus, depth, vertex, normal, s);
+  raycast_shaped(B.src(), B.frames, RayConst{}, B.width, B.height, B.nscenes, B.max_capacity > kNarrowCapacity, false,
+                 shape, cus, depth, vertex, normal, s);
 }
 
 }  // namespace mh
