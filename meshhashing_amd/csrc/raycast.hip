@@ -21,17 +21,20 @@
 
 namespace mh {
 
-// Block lookups shared by the 64 rays of a workgroup (one wave): a
+// Block lookups shared by the rays of a workgroup (one wave; four in the
+// localiser's kernel of four lanes a point): a
 // direct-mapped LDS table that a lane fills after a hash probe, so a block
-// is probed about once per wave rather than once per ray.  An entry is one
-// 64-bit word, read and written by single LDS instructions, so a reader
-// always gets a block and its own index whatever order the wave's divergent
-// paths run in: bits 0-23 hold the pool index + 3 (0 marks an empty slot),
+// is probed about once per workgroup rather than once per ray.  An entry is one
+// 64-bit word, read and written whole (relaxed atomics: single LDS
+// instructions), so a reader always gets a block and its own index whatever
+// order the divergent paths and the other waves run in: bits 0-23 hold the pool
+// index + 3 (0 marks an empty slot),
 // bits 24-63 the block coordinates minus the low bits that chose the slot
 // (x, y: 3 bits, z: 2 bits), which makes (slot, entry) name one block.
-// Blocks beyond +-2^15 on an axis bypass the table.  Of the lanes that miss
+// Blocks beyond +-2^15 on an axis bypass the table.  Of a wave's lanes that miss
 // on one slot in the same instruction, only the one whose id survives in
-// `owner` writes it.
+// `owner` writes it.  That saves stores and decides nothing else: lanes of two
+// waves may both write a slot, and any of the entries is a true one.
 constexpr int kWaveTable = 256;
 struct WaveTable {
   uint64_t e[kWaveTable];
@@ -65,14 +68,16 @@ __device__ __forceinline__ int32_t table_find(const View& V, WaveTable* t, i3 b)
   const uint64_t tag = (uint64_t)((uint32_t)(b.x >> 3) & 0x1FFFu) |
                        ((uint64_t)((uint32_t)(b.y >> 3) & 0x1FFFu) << 13) |
                        ((uint64_t)((uint32_t)(b.z >> 2) & 0x3FFFu) << 26);
-  const uint64_t e = t->e[slot];
+  const uint64_t e = __hip_atomic_load(&t->e[slot], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   if (e != 0ull && (e >> 24) == tag) return (int32_t)(e & 0xFFFFFFu) - 3;
   const int32_t p = ray_probe(V, b);
   if (p >= (1 << 24) - 3) return p;  // does not fit the entry
   const uint32_t lane = threadIdx.x & 63u;
   volatile uint32_t* owner = t->owner;
   owner[slot] = lane;
-  if (owner[slot] == lane) t->e[slot] = (tag << 24) | (uint64_t)(uint32_t)(p + 3);
+  if (owner[slot] == lane)
+    __hip_atomic_store(&t->e[slot], (tag << 24) | (uint64_t)(uint32_t)(p + 3), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_WORKGROUP);
   return p;
 }
 
