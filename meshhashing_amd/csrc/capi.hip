@@ -1529,16 +1529,21 @@ int batch_chain(mh_batch* b, uint32_t flags, bool integrate) {
   if (!integrate) return MH_OK;
   launch_batch_integrate_tsdf(B, b->stream, b->cus * b->grid_per_cu, b->tiling);
   // The raycast needs only the fused TSDF and the table, the meshing pass
-  // writes neither: when the raycast's waves (one per 64 pixels) fit on the
-  // chip in one round, it runs on the side stream beside meshing, so each
-  // fills the other's tail (the slowest tiles end ~3x after the median).
-  // With more waves than that there is no idle tail to fill, and sharing
-  // the chip only slowed both (64 scenes of 320 x 240: 14 %).  Captured, the
-  // fork and join become graph edges.
+  // writes neither: when the raycast's waves at one lane a ray (one per 64
+  // pixels) fit on the chip in one round, it runs on the side stream beside
+  // meshing, so each fills the other's tail (the slowest tiles end ~3x after the
+  // median).  With more than that there is no idle tail to fill, and sharing
+  // the chip only slowed both (64 scenes of 320 x 240: 14 %).  A small image's
+  // march takes up to four lanes a ray and so up to an eighth more waves than
+  // fit; beside meshing it is the faster choice all the same (replayed frames
+  // of a 2 cm room, in turn and beside: 160 x 120 163 and 130 us, 333 x 251 188 and
+  // 165, 350 x 262 189 and 166, 400 x 300 204 and 183; two rooms of 320 x 240 240 and
+  // 208, sixteen of 96 x 72 546 and 528).  Captured, the fork and join become graph
+  // edges.
   if (batch_overlaps(b, flags)) {
     HIP_TRY(hipEventRecord(b->fork, b->stream));
     HIP_TRY(hipStreamWaitEvent(b->side, b->fork, 0));
-    launch_batch_raycast(B, b->out_depth, b->out_vertex, b->out_normal, b->side, b->cus, b->ray_shape);
+    launch_batch_raycast(B, b->out_depth, b->out_vertex, b->out_normal, b->side, b->cus, b->ray_shape, true);
     launch_batch_marching_cubes(B, b->d_nbt, b->stream, b->cus, kMcShapes[b->mc_shape], true);
     HIP_TRY(hipEventRecord(b->join, b->side));
     HIP_TRY(hipStreamWaitEvent(b->stream, b->join, 0));

@@ -241,8 +241,9 @@ void launch_ray_range_one(const View& V, const RayConst& p, hipStream_t s);
 // diagnostics: add the distinct blocks the last raycast sampled (V.ray_mark
 // == V.ray_stamp) to the work counters
 void launch_ray_mark_count(const View& V, hipStream_t s, int grid);
+// beside: a meshing pass runs at the same time
 void launch_batch_raycast(const BatchDev& B, float* depth, float* vertex, float* normal,
-                          hipStream_t s, int cus, int shape = 0);
+                          hipStream_t s, int cus, int shape = 0, bool beside = false);
 // adjoint: 31 FP64 sums (loss, dL/dxi[6], J^T J upper triangle[21], pixels,
 // gated-out pixels, observed pixels)
 constexpr int kGradSlots = 31;

@@ -940,14 +940,26 @@ void launch_slot_reduce(double* partials, uint32_t n, uint32_t slots, uint32_t* 
 // Lanes a ray: an image of few pixels leaves the chip nearly empty, a wave a
 // SIMD at 333 x 251, and each wave's time is the latency of its rays' samples
 // in a row; four (two) lanes a ray then take a quarter (half) of the rounds.
-// As many as fit the chip in one round of waves; past that the extra lanes only
-// add work.  Four lanes go an eighth past it, the first waves being done by then
-// (5 mm desk, 333 x 251: 112 us, 131 with two; 344 x 258: 108 and 122).  Measured (5 mm desk, whole call, 1 / 2 / 4 lanes): 160 x 120
-// 155 / 128 / 92 us, 320 x 240 138 / 124 / 98, 400 x 300 147 / 130 / 137,
-// 480 x 360 149 / 155 / 152, 640 x 480 142 / 162 / 189.
-inline int ray_lanes(uint64_t pixels, int cus) {
+// Two as long as their waves fit the chip in one round; past that the extra lanes
+// only add work.  Four an eighth past it, the first waves being done by then.
+// Measured, whole call, us with 1 / 2 / 4 lanes (5 mm desk; 5 mm room; 2 cm room):
+//   320 x 240    148 / 119 / 101    107 /  99 /  91    72 / 66 / 58
+//   350 x 262    147 / 132 / 107    106 / 104 / 111    71 / 68 / 65  (just inside the four's line)
+//   358 x 268    150 / 129 / 116    103 / 101 / 112    75 / 73 / 70  (just past it)
+//   400 x 300    137 / 131 / 120    103 / 106 / 121    75 / 75 / 77
+//   462 x 346    141 / 141 / 136    109 / 115 / 135    77 / 82 / 85  (just inside the two's)
+//   480 x 360    140 / 144 / 138    113 / 136 / 149    76 / 88 / 92
+// so that either line lies where the scenes' sums are about even.  beside: a
+// meshing pass runs on the chip at the same time.  Two lanes then bring nothing
+// (replayed frames: 2 cm room 400 x 300 183 us with one, 187 with two, 1 cm 249
+// and 267; two 4 cm rooms of 320 x 240 134 and 144; 5 mm desk 400 x 300 293 and
+// 312), and four still do where the march is the longer branch (2 cm room 160 x
+// 120 178 and 130, 320 x 240 175 and 162, two of 237 x 177 208 and 180, four of
+// 175 x 131 245 and 224) but cost time where the meshing pass is (5 mm desk
+// 320 x 240 273 and 311; 1 cm room even, 241 and 237).
+inline int ray_lanes(uint64_t pixels, int cus, bool beside) {
   const uint64_t waves = (pixels + 63) / 64, room = (uint64_t)kRayWavesPerSimd * 4 * (uint64_t)cus;
-  return 4 * waves <= room + room / 8 ? 4 : (2 * waves <= room ? 2 : 1);
+  return 4 * waves <= room + room / 8 ? 4 : (!beside && 2 * waves <= room ? 2 : 1);
 }
 
 // ------------------------------------------------------------ localisation
@@ -1135,7 +1147,11 @@ void launch_point_to_psdf(const View& V, const M4& wTc, int corrected, double* p
                           const LocalizeStep& step, hipStream_t s, int cus) {
   const dim3 grid((V.cam.width / 2 + 7) / 8, (V.cam.height / 2 + 7) / 8);
   const bool wide = V.capacity > kNarrowCapacity;
-  const int lanes = !wide && ray_lanes((uint64_t)grid.x * grid.y * 64, cus) == 4 ? 4 : 1;
+  // The march's line holds here too (20 steps in us, one / four lanes: 2 cm room
+  // 320 x 240 543 / 396, 672 x 504 just inside it 630 / 596, 720 x 540 just past it
+  // 645 / 623, 800 x 600 679 / 679, 1200 x 900 992 / 997; 5 mm desk 584 / 415, 698 /
+  // 639, 741 / 690, 766 / 741, 1048 / 1148).
+  const int lanes = !wide && ray_lanes((uint64_t)grid.x * grid.y * 64, cus, false) == 4 ? 4 : 1;
   const auto k = wide ? point_to_psdf_kernel<true, 1> : (lanes == 4 ? point_to_psdf_kernel<false, 4> : point_to_psdf_kernel<false, 1>);
   k<<<grid, 64 * lanes, 0, s>>>(V, wTc, 1.0f / V.geo.voxel_size, corrected, partials, step);
   const uint32_t n = grid.x * grid.y;
@@ -1403,11 +1419,11 @@ void launch_ray_range(Src src, const SceneFrame* tab, const RayConst& R, uint32_
 
 template <class Src>
 void raycast_shaped(Src src, const SceneFrame* tab, const RayConst& p, uint32_t w, uint32_t h, uint32_t nscenes,
-                    bool wide, bool marks, int shape, int cus, float* depth, float* vertex, float* normal,
-                    hipStream_t s) {
+                    bool wide, bool marks, bool beside, int shape, int cus, float* depth, float* vertex,
+                    float* normal, hipStream_t s) {
   // marks: the blocks of the samples are counted; several lanes a ray also
   // sample behind its crossing
-  const int lanes = wide || marks || shape != 0 ? 1 : ray_lanes((uint64_t)w * h * nscenes, cus);
+  const int lanes = wide || marks || shape != 0 ? 1 : ray_lanes((uint64_t)w * h * nscenes, cus, beside);
   const int px = 64 / lanes;
   const int tw = lanes == 1 ? kRayTileWidths[shape] : (lanes == 2 ? 8 : 4), th = px / tw;
   const int log_tw = __builtin_ctz((unsigned)tw);
@@ -1427,7 +1443,7 @@ void launch_ray_range_one(const View& V, const RayConst& p, hipStream_t s) {
 void launch_raycast_march(const View& V, const RayConst& p, float* depth, float* vertex, float* normal,
                           hipStream_t s, int cus, int shape) {
   raycast_shaped(One{V}, nullptr, p, p.cam.width, p.cam.height, 1, V.capacity > kNarrowCapacity, V.ray_mark != nullptr,
-                 shape, cus, depth, vertex, normal, s);
+                 false, shape, cus, depth, vertex, normal, s);
 }
 
 void launch_raycast(const View& V, const RayConst& p, float* depth, float* vertex, float* normal,
@@ -1436,7 +1452,7 @@ void launch_raycast(const View& V, const RayConst& p, float* depth, float* verte
   launch_ray_range(One{V}, nullptr, p, p.tiles, 1, s);
   tick(kc, s, "raycast_kernel");
   raycast_shaped(One{V}, nullptr, p, p.cam.width, p.cam.height, 1, V.capacity > kNarrowCapacity, V.ray_mark != nullptr,
-                 shape, cus, depth, vertex, normal, s);
+                 false, shape, cus, depth, vertex, normal, s);
   tick(kc, s, nullptr);
 }
 
@@ -1471,10 +1487,10 @@ void launch_raycast_backward(const View& V, const RayConst& p, const float* obs,
 }
 
 void launch_batch_raycast(const BatchDev& B, float* depth, float* vertex, float* normal,
-                          hipStream_t s, int cus, int shape) {
+                          hipStream_t s, int cus, int shape, bool beside) {
   launch_ray_range(B.src(), B.frames, RayConst{}, ((B.width + 7) / 8) * ((B.height + 7) / 8), B.nscenes, s);
   raycast_shaped(B.src(), B.frames, RayConst{}, B.width, B.height, B.nscenes, B.max_capacity > kNarrowCapacity, false,
-                 shape, cus, depth, vertex, normal, s);
+                 beside, shape, cus, depth, vertex, normal, s);
 }
 
 }  // namespace mh
