@@ -1974,11 +1974,14 @@ int mh_batch_run(mh_batch* b, const mh_mc_params* mc, uint32_t flags, mh_tune_re
       const int rc = build_ray(v, &b->rp[s], v->V.cTw.m, &f.ray);
       if (rc) return rc;
       f.ray.range = b->d_range + (size_t)s * ray_range_words(b->W, b->H);
-      // Beside the meshing pass the march is the longer branch once the
-      // surfel pass leaves room on the chip (fewer than all resident
-      // workgroups): its waves then issue first on a shared SIMD.  Beside an
-      // all-resident surfel pass the boost cost time instead.
-      f.ray.boost = batch_overlaps(b, flags) && kMcShapes[b->mc_shape].grid_per_cu > 0;
+      // Beside a meshing pass of two workgroups a CU (half of what is resident)
+      // the march is mostly the longer branch: its waves then issue first on a
+      // shared SIMD (replayed 1 cm room, 400 x 300 265 us without and 256 with,
+      // 640 x 480 322 and 309; 2 cm 160 and 161; 5 mm desk 333 and 342).  Beside an
+      // all-resident one it changes nothing (238 and 239, 333 and 333), and beside
+      // one workgroup a CU, where meshing is the longer branch, it costs time
+      // (1 cm room 319 and 330, 334 and 360; 5 mm desk 478 and 495).
+      f.ray.boost = batch_overlaps(b, flags) && kMcShapes[b->mc_shape].grid_per_cu >= 2;
     }
     f.V = v->V;
     f.V.raw = b->raw + (size_t)s * b->W * b->H;
