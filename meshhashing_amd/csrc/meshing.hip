@@ -450,11 +450,29 @@ __device__ __forceinline__ bool payload_part(const Shell<PSDF>& S, const Geo& g,
   return oob;
 }
 
-// Position, radius and colour of vertex j of the round.
+// Position, radius and colour of vertex j of the round.  An end that is no number
+// (a NaN passes the corner tests) makes none of all three coordinates, the other
+// axes' being pA + NaN * 0, and of its sample, in the cell of the voxel 0 that a
+// NaN rounds to.
 template <bool PSDF>
-__device__ __forceinline__ void finish_sample(const View& V, int32_t vp, uint32_t j, const Payload<PSDF>& P) {
+__device__ __forceinline__ void finish_sample(const Shell<PSDF>& S, const View& V, i3 base, int32_t vp, uint32_t j,
+                                              const Payload<PSDF>& P) {
+  float px = P.v[kPayPos][j], py = P.v[kPayPos + 1][j], pz = P.v[kPayPos + 2][j];
+  bool ok = P.v[kPayOk][j] != 0.0f;
+  const float sum = px + py + pz;
+  const bool none = !(sum == sum);
+  if (none) {
+    px = py = pz = sum;
+    ok = (uint32_t)-base.x <= 8u && (uint32_t)-base.y <= 8u && (uint32_t)-base.z <= 8u;
+    if (ok) {
+      const uint32_t s = (uint32_t)sidx(-base.x, -base.y, -base.z);
+      ok = (S.bits[kThere][s >> 5] >> (s & 31u)) & 1u;
+    } else {
+      flag(V, MH_STATUS_STENCIL_RANGE);
+    }
+  }
   float radius = 0.0f, cr = 0.0f, cg = 0.0f, cb = 0.0f;  // the reference reads an uninitialised query here
-  if (P.v[kPayOk][j] != 0.0f) {
+  if (ok) {
     const float rx = P.v[kPayRatio][j], ry = P.v[kPayRatio + 1][j], rz = P.v[kPayRatio + 2][j];
     float rad = 0.0f;
 #pragma unroll
@@ -464,16 +482,17 @@ __device__ __forceinline__ void finish_sample(const View& V, int32_t vp, uint32_
     }
     const float inv_sigma2 = 1.0f / (rad * rad);
     radius = sqrtf(1.0f / inv_sigma2);
-    const float a = PSDF ? P.v[PSDF ? kPayA : 0][j] : 0.0f, b = PSDF ? P.v[PSDF ? kPayB : 0][j] : 0.0f;
+    float a = PSDF ? P.v[PSDF ? kPayA : 0][j] : 0.0f, b = PSDF ? P.v[PSDF ? kPayB : 0][j] : 0.0f;
+    if (PSDF && none) a = sum;
     const f3 c = val_to_rgb(a / (a + b), 0.4f, 1.0f);
     cr = c.x;
     cg = c.y;
     cb = c.z;
   }
   Vertex* dst = &V.vertices[vp];
-  dst->px = P.v[kPayPos][j];
-  dst->py = P.v[kPayPos + 1][j];
-  dst->pz = P.v[kPayPos + 2][j];
+  dst->px = px;
+  dst->py = py;
+  dst->pz = pz;
   dst->radius = radius;
   dst->cr = cr;
   dst->cg = cg;
@@ -975,7 +994,7 @@ __global__ __launch_bounds__(kMcLanes, PSDF ? 3 : 4) void mc_surfel_kernel(Src s
         const uint32_t role = (wave + turns) & 3u;
         if (j0 + lane < nq) {
           if (role == 0) finish_normal<PSDF>(V, qptr[j0 + lane], lane, pay);
-          if (role == 1) finish_sample<PSDF>(V, qptr[j0 + lane], lane, pay);
+          if (role == 1) finish_sample<PSDF>(S, V, base, qptr[j0 + lane], lane, pay);
         }
         __syncthreads();
       }
