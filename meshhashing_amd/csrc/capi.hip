@@ -2144,7 +2144,8 @@ constexpr size_t kNoAllocPartialBytes = round_up((size_t)kNoAllocTiles * kGradSl
 constexpr size_t kNoAllocResultOff = kNoAllocPartialOff + kNoAllocPartialBytes;
 constexpr size_t kNoAllocResultBytes = round_up(kGradSlots * sizeof(double));
 constexpr size_t kNoAllocRangeOff = kNoAllocResultOff + kNoAllocResultBytes;
-constexpr size_t kNoAllocRangeBytes = round_up((2 * (size_t)kNoAllocTiles + 1) * sizeof(uint32_t));
+constexpr size_t kNoAllocRangeBytes =
+    round_up(ray_range_words(kNoAllocMaxWidth, kNoAllocMaxHeight) * sizeof(uint32_t));
 constexpr size_t kNoAllocScratchBytes = kNoAllocRangeOff + kNoAllocRangeBytes;  // ~5.2 MB
 
 }  // namespace
