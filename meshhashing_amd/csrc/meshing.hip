@@ -461,7 +461,7 @@ __device__ __forceinline__ void finish_sample(const Shell<PSDF>& S, const View& 
   bool ok = P.v[kPayOk][j] != 0.0f;
   const float sum = px + py + pz;
   const bool none = !(sum == sum);
-  if (none) {
+  if (__builtin_expect(none, 0)) {
     px = py = pz = sum;
     ok = (uint32_t)-base.x <= 8u && (uint32_t)-base.y <= 8u && (uint32_t)-base.z <= 8u;
     if (ok) {
