@@ -83,11 +83,13 @@ __device__ __forceinline__ const McConst& mc_of(const Many& m, uint32_t s, const
 }
 // Surfel pass: 256 lanes a workgroup (two voxels a lane).  The next block's
 // shell, cube words and vertex slots are loaded into registers while the
-// current block is worked on, which takes up to 128 registers: four workgroups
+// current block is worked on, which takes 128 registers and spills seven a lane
+// (three over a batch; none of a probabilistic volume's 168): four workgroups
 // a CU, each a block at work and one on its way.  Bound by the instructions it
-// issues where there are many blocks (64 rooms, 71 k blocks: 946 us, 667 of them
-// VALU), by the chain of a block's phases where there are few (1444 blocks: 47 us,
-// two rounds of workgroups).  With eight lanes a vertex's payload and an item an
+// issues where there are many blocks (64 rooms, 71 k blocks: 958 us, 673 of them
+// VALU), by memory as well where most of them hold a fine surface (11 k blocks of a
+// 5 mm frame: 155 us, 455 MB at 60 % of a device copy's rate), by the chain of a
+// block's phases where there are few (1444 blocks: 50 us, two rounds of workgroups).  With eight lanes a vertex's payload and an item an
 // edge of each cube, the replayed 640 x 480, 5 mm frame and a batch of 64 rooms took 358
 // us and 2.87 ms so, 412 us and 3.35 ms with 512 lanes and two workgroups a CU, 466 us
 // and 3.57 ms with 512 lanes, three workgroups and 80 registers (spills).
