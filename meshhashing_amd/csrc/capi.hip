@@ -316,6 +316,16 @@ int build_ray(const mh_volume* v, const mh_raycaster_params* p, const float cTw[
   std::memcpy(R->cTw.m, cTw, sizeof(float) * 16);
   invert4<float>(cTw, R->wTc.m);
   R->range = nullptr;
+  // A sample at t lies at camera z t dir_c.z times the length that the pose gives
+  // a unit direction; the tile ranges are widened by 1e-3 for all but that.  (A
+  // pose that is no number counts as rigid: its rays have no samples either way.)
+  float dev = 0.0f;
+  for (int i = 0; i < 3; ++i)
+    for (int j = i; j < 3; ++j) {
+      const float d = cTw[4 * i] * cTw[4 * j] + cTw[4 * i + 1] * cTw[4 * j + 1] + cTw[4 * i + 2] * cTw[4 * j + 2];
+      dev = std::max(dev, std::fabs(d - (i == j ? 1.0f : 0.0f)));
+    }
+  R->whole = dev > 3e-4f;
   R->tiles_x = (p->width + 7) / 8;
   R->tiles = R->tiles_x * ((p->height + 7) / 8);
   return MH_OK;

@@ -29,6 +29,9 @@ struct RayConst {
   // (launch_ray_rows).
   uint32_t* range;
   uint32_t tiles_x, tiles;
+  // every tile's range is whole: the pose is not rigid, so that t dir_c.z is not
+  // the camera z of a ray's sample
+  int whole;
   // the march's waves raise their issue priority (a batch's raycast beside a
   // meshing pass of two workgroups a CU)
   int boost;

@@ -1225,7 +1225,7 @@ __global__ __launch_bounds__(64, kRayWavesPerSimd) void raycast_kernel(Src src_,
 // sample outside its tile's [zmin, zmax].  A box that reaches through the plane
 // z = min_depth / 2 is clipped there: a camera inside a room nearly always has
 // such blocks beside it (a wall's, at the camera's own depth), and switching the
-// ranges off for them made every ray walk up to its surface from min_depth (5 mm
+// ranges off for them (a pose that is not rigid has none: RayConst::whole) made every ray walk up to its surface from min_depth (5 mm
 // room at 1237 x 931: the march 854 us, 499 us with the ranges).
 //
 // Before it, one launch clears the tile ranges (its first kClearGroups
@@ -1241,7 +1241,7 @@ __global__ __launch_bounds__(256) void ray_prepare_kernel(Src src_, const SceneF
     const RayConst& R = ray_of(src, blockIdx.y, R1);
     if (!R.range) return;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < 2 * R.tiles; i += kClearGroups * blockDim.x)
-      R.range[i] = (i & 1u) ? 0u : 0x7f800000u;  // zmin +inf, zmax 0
+      R.range[i] = ((i & 1u) != 0u) == (R.whole != 0) ? 0x7f800000u : 0u;  // zmin +inf, zmax 0; whole: 0, +inf
     return;
   }
   const View V = src.view(blockIdx.y);
@@ -1362,6 +1362,7 @@ __global__ __launch_bounds__(kLds ? kRangeLdsLanes : 256) void ray_range_kernel(
   const uint32_t scene = blockIdx.y;
   const View& V = src.view(scene);
   const RayConst& R = ray_of(src, scene, R1);
+  if (R.whole) return;
   const uint32_t n = V.ctr->block_hwm;
   const float vs = V.geo.voxel_size;
   __shared__ uint32_t lds_range[kLds ? 2 * kRangeLdsTiles : 1];
